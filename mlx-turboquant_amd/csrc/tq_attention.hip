@@ -1566,6 +1566,98 @@ static bool fill_split(UniformArgs& u, const tq_codec* kc, const tq_codec* vc, c
   return true;
 }
 
+// Width kind of one side for the kernels of tq_decode_mfma.h: the bits of an
+// integer width (2 to 4), bits_hi + bits_lo of a fractional one split at d / 2
+// (7 = 3.5 bits, 5 = 2.5), or 0.
+static int mfma_kind(const tq_codec* c) {
+  if (!c->centroids_hi) return 0;
+  if (c->split == c->d) return c->bits_hi >= 2 && c->bits_hi <= 4 ? c->bits_hi : 0;
+  if (2 * c->split == c->d && c->centroids_lo && (c->bits_hi == 4 || c->bits_hi == 3) && c->bits_lo == c->bits_hi - 1)
+    return c->bits_hi + c->bits_lo;
+  return 0;
+}
+
+// The kernels of tq_decode_mfma.h: one query token, no sketch, head_dim 64 /
+// 96 / 128 / 256, widths 2-4 and 2.5 / 3.5 on either side (keys at head_dim 96:
+// integer, the 12 dims of a lane's half are not whole 8-dim k-steps), fp16 or
+// bf16 uncompressed tokens, any query-head ratio, uniform or ragged. Code
+// rows are read at byte granularity; q, sink and ring rows in 16-byte pieces.
+static bool mfma_eligible(const tq_codec* kc, const tq_codec* vc, const tq_attn_desc* d) {
+  if (d->n_q > 1 || (d->qjl && d->max_comp > 0)) return false;
+  if (!(kc->d == 64 || kc->d == 96 || kc->d == 128 || kc->d == 256) || vc->d != kc->d) return false;
+  const int kk = mfma_kind(kc), vk = mfma_kind(vc);
+  if (!kk || !vk || (kc->d == 96 && kk > 4)) return false;
+  if (!(kc->rotation_parts && vc->rotation)) return false;
+  if (d->kv_dtype != TQ_F16 && d->kv_dtype != TQ_BF16) return false;
+  auto al4 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 3) == 0; };
+  if (!aligned16(d->q) || !aligned16(kc->rotation_parts) || !aligned16(vc->rotation)) return false;
+  if (d->max_comp > 0 && !(al4(d->kstore.norms) && al4(d->vstore.norms) && (kk <= 4 || d->kstore.codes_lo) &&
+                           (vk <= 4 || d->vstore.codes_lo)))
+    return false;
+  // (32-bit byte offsets within a row's codes)
+  if ((int64_t)d->max_comp * (kc->d / 2) > 0x7fffffffLL) return false;
+  if (d->max_sink > 0 && !(aligned16(d->sink_k) && aligned16(d->sink_v) && d->sink_head_stride % 8 == 0)) return false;
+  if (d->max_res > 0 && !(aligned16(d->res_k) && aligned16(d->res_v) && d->res_head_stride % 8 == 0)) return false;
+  return d->max_comp > 0 || d->max_sink > 0 || d->max_res > 0;
+}
+
+// Workgroups per (sequence, head group): one wave per 32-token block of the
+// uncompressed tokens, and for the compressed ones what is left of one
+// workgroup per CU (a CU of their own each where the uncompressed tokens
+// alone fill half the chip), at least one block per wave.
+static void mfma_geometry(const tq_attn_desc* d, int& gsub, int& g, int& ncw, int& nfw) {
+  const int G = d->hq / d->hkv;
+  g = group_heads(G);
+  gsub = G / g;
+  const int64_t rows = (int64_t)d->batch * d->hkv * gsub;
+  const int per = MFMA_WAVES * 32;
+  nfw = (int)(((int64_t)d->max_sink + d->max_res + per - 1) / per);
+  const int most = (d->max_comp + per - 1) / per;
+  const int cus = device_cus();
+  int64_t avail = cus - rows * nfw;
+  if (avail < cus / 2) avail = cus;
+  const int64_t share = avail / rows > 1 ? avail / rows : 1;
+  ncw = share < most ? (int)share : most;
+}
+
+static size_t mfma_part_bytes(const tq_codec* kc, const tq_attn_desc* d) {
+  int gsub, g, ncw, nfw;
+  mfma_geometry(d, gsub, g, ncw, nfw);
+  return (size_t)d->batch * d->hq * (ncw + nfw) * (kc->d + 4) * 4;
+}
+
+static int mfma_run(const tq_codec* kc, const tq_codec* vc, const tq_attn_desc* d, void* workspace, hipStream_t s) {
+  MfmaArgs a{};
+  mfma_geometry(d, a.gsub, a.g, a.ncw, a.nfw);
+  const int kk = mfma_kind(kc), vk = mfma_kind(vc);
+  a.kc = d->kstore.codes_hi; a.k_hs = d->kstore.hi_head_stride;
+  a.kcl = d->kstore.codes_lo; a.kl_hs = d->kstore.lo_head_stride;
+  a.kn = d->kstore.norms; a.kn_hs = d->kstore.norm_head_stride;
+  a.vc = d->vstore.codes_hi; a.v_hs = d->vstore.hi_head_stride;
+  a.vcl = d->vstore.codes_lo; a.vl_hs = d->vstore.lo_head_stride;
+  a.vn = d->vstore.norms; a.vn_hs = d->vstore.norm_head_stride;
+  a.sink_k = d->sink_k; a.sink_v = d->sink_v; a.sink_hs = d->sink_head_stride;
+  a.res_k = d->res_k; a.res_v = d->res_v; a.res_hs = d->res_head_stride;
+  a.res_cap = d->res_cap; a.res_start0 = d->res_start0;
+  a.comp_len_b = d->comp_len; a.sink_len_b = d->sink_len; a.res_len_b = d->res_len; a.res_start_b = d->res_start;
+  a.max_comp = d->max_comp; a.max_sink = d->max_sink; a.max_res = d->max_res;
+  a.q = d->q; a.q_dtype = d->q_dtype; a.out = d->out;
+  a.batch = d->batch; a.hq = d->hq; a.hkv = d->hkv;
+  a.qscale = d->scale * 1.4426950408889634f;
+  a.rot16 = kc->rotation_parts; a.vrot = vc->rotation;
+  a.kcen_hi = kc->centroids_hi; a.kcen_lo = kk > 4 ? kc->centroids_lo : kc->centroids_hi;
+  a.vcen_hi = vc->centroids_hi; a.vcen_lo = vk > 4 ? vc->centroids_lo : vc->centroids_hi;
+  a.vbh = vc->bits_hi; a.vbl = vk > 4 ? vc->bits_lo : vc->bits_hi; a.vfrac = vk > 4;
+  a.part = static_cast<float*>(workspace);
+  const bool bf = d->kv_dtype == TQ_BF16;
+  switch (kc->d) {
+    case 64: return launch_mfma_d64(a, kk, bf, s);
+    case 96: return launch_mfma_d96(a, kk, bf, s);
+    case 128: return launch_mfma_d128(a, kk, bf, s);
+    default: return launch_mfma_d256(a, kk, bf, s);
+  }
+}
+
 // The QJL route: S q, key-term bias, K4/V2 partials with the bias
 // (scores stored) + merge (max and sum exported), value term, final S^T add.
 static int qjl_fast_run(const tq_codec* kc, const tq_codec* vc, const tq_attn_desc* d, void* workspace,
@@ -1815,6 +1907,10 @@ size_t tq_decode_workspace_bytes(const tq_codec* kcodec, const tq_attn_desc* d) 
   size_t general = heads * D * 4 * 2 + heads * (size_t)m * 4 + heads * nch * part_stride(D, m) * 4;
   const size_t fast = d->hkv > 0 && d->hq % d->hkv == 0 ? fast_part_bytes(d) : 0;
   size_t bytes = general > fast ? general : fast;
+  if (d->batch > 0 && d->hkv > 0 && d->hq > 0 && d->hq % d->hkv == 0 && d->n_q <= 1) {
+    const size_t mf = mfma_part_bytes(kcodec, d);
+    if (mf > bytes) bytes = mf;
+  }
   if (d->qjl && kcodec->d == 128 && kcodec->qjl_m > 0 && kcodec->qjl_m <= 256 && d->max_comp > 0 && d->hkv > 0 &&
       d->hq % d->hkv == 0) {
     const size_t qf = qjl_layout(kcodec, d).total;
@@ -1876,6 +1972,10 @@ int tq_decode_attention(const tq_codec* kc, const tq_codec* vc, const tq_attn_de
         TQ_LAUNCH_CHECK("tq_decode_attention (fractional widths)");
       return TQ_OK;
     }
+  }
+  if (mfma_eligible(kc, vc, d) && !(d->flags & TQ_ATTN_GENERAL)) {
+    if (mfma_run(kc, vc, d, workspace, s) != 0) TQ_LAUNCH_CHECK("tq_decode_attention (mfma)");
+    return TQ_OK;
   }
 
   AttnArgs a;
@@ -1963,7 +2063,8 @@ int tq_measure_decode_partials(const tq_codec* kc, const tq_codec* vc, const tq_
 // valid call, without launching anything: 0 the general kernel, 1 the dense
 // kernel, 2 the K4/V2 kernels, 3 the K4/V2 kernels with the QJL terms, 4 the
 // uniform-batch kernels of the other integer widths, 5 those of the
-// fractional widths, 6 the query-tiled prefill kernels.
+// fractional widths, 6 the query-tiled prefill kernels, 7 the kernels of
+// tq_decode_mfma.h.
 int tq_debug_decode_route(const tq_codec* kc, const tq_codec* vc, const tq_attn_desc* d) {
   if (!kc || !vc || !d || d->hkv <= 0 || d->hq % d->hkv) return -1;
   if (d->flags & TQ_ATTN_GENERAL) return 0;
@@ -1974,6 +2075,7 @@ int tq_debug_decode_route(const tq_codec* kc, const tq_codec* vc, const tq_attn_
   int nwg, bpw, fpw;
   if (widths_eligible(kc, vc, d) && uniform_route(vc, d, nwg, bpw, fpw, true)) return 4;
   if (split_eligible(kc, vc, d) && uniform_route(vc, d, nwg, bpw, fpw)) return 5;
+  if (mfma_eligible(kc, vc, d)) return 7;
   return 0;
 }
 

@@ -163,6 +163,44 @@ int launch_uniform_widths(const UniformArgs& a, int G, int kb, int vb, int merge
 // of a fractional codec (7 or 5) or the bits of an integer one (2 to 4).
 int launch_uniform_split(const UniformArgs& a, int G, int kkind, int vkind, int merge, hipStream_t s);
 
+// Arguments of the decode kernels of tq_decode_mfma.h: rows of (sequence,
+// head group), ncw workgroups per row over the compressed blocks and nfw over
+// the uncompressed tokens, one partial of D + 4 floats per workgroup and head.
+constexpr int MFMA_WAVES = 8;  // waves per workgroup
+
+struct MfmaArgs {
+  const uint8_t* kc;  int64_t k_hs;    // key codes: integer width, or dims [0, D / 2) of a fractional one
+  const uint8_t* kcl; int64_t kl_hs;   // key codes of dims [D / 2, D) (fractional)
+  const float* kn;    int64_t kn_hs;
+  const uint8_t* vc;  int64_t v_hs;    // values likewise
+  const uint8_t* vcl; int64_t vl_hs;
+  const float* vn;    int64_t vn_hs;
+  const void* sink_k; const void* sink_v; int64_t sink_hs;   // elements
+  const void* res_k;  const void* res_v;  int64_t res_hs;    // ring
+  int res_cap, res_start0;
+  const int32_t* comp_len_b; const int32_t* sink_len_b; const int32_t* res_len_b; const int32_t* res_start_b;
+  int max_comp, max_sink, max_res;
+  const void* q; int q_dtype;
+  float* out;
+  int batch, hq, hkv;
+  int gsub, g;           // head groups per kv head, query heads per group (at most 8)
+  float qscale;          // scale * log2(e)
+  const uint16_t* rot16; // (2, D, D) fp16 high part / remainder of R (key codec)
+  const float* vrot;     // (D, D) R float32, row-major (value codec)
+  const float* kcen_hi; const float* kcen_lo;  // codebooks in device memory
+  const float* vcen_hi; const float* vcen_lo;
+  int vbh, vbl, vfrac;   // value widths; vfrac: fractional (split at D / 2)
+  float* part;           // (batch, hkv gsub, ncw + nfw, g, D + 4)
+  int ncw, nfw;
+  int tail;              // LDS offset past the tables / combine buffers (set by the launch)
+};
+// Partials and merge for head_dim 64 / 96 / 128 / 256; kk: the key width kind
+// (2-4, 5 = 2.5 bits, 7 = 3.5 bits), bf: bf16 sink / ring tokens.
+int launch_mfma_d64(const MfmaArgs& a, int kk, bool bf, hipStream_t s);
+int launch_mfma_d96(const MfmaArgs& a, int kk, bool bf, hipStream_t s);
+int launch_mfma_d128(const MfmaArgs& a, int kk, bool bf, hipStream_t s);
+int launch_mfma_d256(const MfmaArgs& a, int kk, bool bf, hipStream_t s);
+
 // Arguments of the dense (fp16 / bf16 K/V) decode-attention kernel: the
 // fp16 segments of tq_attn_desc, head_dim 128.
 struct DenseArgs {

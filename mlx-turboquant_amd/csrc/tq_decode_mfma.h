@@ -1,0 +1,783 @@
+// Decode attention on MFMA for what the K4/V2 / widths / split kernels do not
+// take: head_dim 64, 96, 128 and 256, integer widths 2-4 and fractional
+// widths on either side, any number of query heads per kv head (groups of at
+// most 8), fp16 or bf16 sink / ring tokens, uniform and ragged batches. A
+// partials kernel over a fixed grid and a merge kernel.
+//
+// Grid (ncw + nfw, hkv * gsub, batch), 8 waves. Workgroup c < ncw of a row
+// (sequence, head group) takes compressed 32-token blocks (an equal share of
+// the sequence's own blocks, wave w blocks w + 8k of it); workgroup ncw + f
+// takes 32-token blocks of the uncompressed [sink | ring] list. Each writes one
+// partial per query head, [M, L, 0, 0, out[D] / L], in rotated space (c < ncw)
+// or original space; the merge weighs them, applies the value codec's R once
+// to the rotated sum and adds the other.
+//
+// Scores are S^T = K q^T on MFMA 16x16x32 f16 (A = 16 tokens x 32 dims). The
+// assignment of dims to k-slots is free as long as both operands agree, so
+// lane (token r, q4) owns D / 4 contiguous dims of its token: 32 lanes read
+// whole code rows, 8 dims per k-step. A pair of codes (2B bits) is looked up
+// in an LDS table whose 8-byte entry is (c_hi pair, c_lo pair) in fp16, c_lo =
+// c - fp16(c): four lookups fill the high-part and the remainder operand of a
+// k-step. The query's fp16 high part and remainder are two columns of B, so
+// two MFMAs per step give the product to 2^-22. For GC = 4 the 16 columns are
+// two groups of 8, group t serving 16-token tile t of the block (column c8
+// the high part of head c8, c8 < 4, or the remainder of head 7 - c8); for
+// GC = 8 column r is part r >> 3 of head r & 7. Columns past the group's
+// heads repeat head 0 and are not written.
+//
+// Output, transposed too: O^T += V^T P^T, A row r = dims (D / 16) r + nb of
+// MFMA nb (the value codes of a token's row are one dword, two at D = 256, per
+// lane; the two 8-row halves take the two widths of a fractional codec), high
+// part and remainder in two MFMAs; P^T = p * n_v as fp16 high part / remainder
+// columns, scaled by a power of two per column, and stays in the lane that
+// computed the scores.
+//
+// Tables have 16 replicas per entry (128-byte rows): both sides of every width
+// pair fit 80 KB, against 2-way bank conflicts on some lookups.
+//
+// Bound: latency (set-up, the block loads' round trips, combine), as in the
+// uniform-batch kernels; one layer's codes are 2-9 MB, under 2 us of HBM time.
+// Measured per layer in a graph of 16 layers, partials + merge against the
+// general kernel's three launches (float32 VALU dot products): bf16 K4/V4, 28
+// heads on 4, T 16,001: 20.4 us (kernels 12.8 + 6.7) from 101 us; head_dim 64,
+// bf16 K4/V2, 2 sequences, 32 heads on 8, T 8,229: 14.5 us from 56 us;
+// head_dim 256, bf16 K4/V3, 8 heads on 2, T 12,000: 35 us from 112 us.
+#pragma once
+
+#include <math.h>
+
+#include "tq_common.h"
+#include "tq_decode_fast.h"
+#include "tq_decode_uniform.h"
+
+namespace tq {
+namespace mk {
+
+using uk::as_h8;
+using uk::f4;
+using uk::fexp2;
+using uk::half8;
+using uk::hx2;
+using uk::mfma;
+using uk::pk_rtz;
+using uk::row_ror;
+using uk::rows_max;
+using uk::rows_sum;
+using uk::u2;
+using uk::u4;
+using uk::wave_max_u32;
+
+constexpr int MW = MFMA_WAVES;
+constexpr int MTH = MW * 64;   // threads
+constexpr float M_INIT = uk::M_INIT;
+constexpr int TROW = 128;      // bytes per table entry: 16 replicas
+
+// N bytes at any address into dwords (the compiler picks the load widths)
+template <int N>
+__device__ inline void load_bytes(uint32_t (&w)[(N + 3) / 4], const uint8_t* p) {
+  w[(N + 3) / 4 - 1] = 0u;
+  __builtin_memcpy(&w[0], p, N);
+}
+
+// The pair table of one codebook (word i of `cw` lane 16 bk + i: fp16 high
+// part | remainder << 16 of centroid i): entry e = (code of dim 2f) | (code
+// of dim 2f + 1) << bits.
+__device__ inline void build_table(uint8_t* tab, int bk, int bits, uint32_t cw, int tid) {
+  const int n16 = (1 << (2 * bits)) * (TROW / 16);  // whole waves (2 bits: 128)
+  const uint32_t mask = (1u << bits) - 1u;
+  for (int s = tid; s < n16; s += MTH) {
+    const uint32_t e = s / (TROW / 16);
+    const uint32_t ca = __builtin_amdgcn_ds_bpermute((16 * bk + (e & mask)) * 4, cw);
+    const uint32_t cb = __builtin_amdgcn_ds_bpermute((16 * bk + (e >> bits)) * 4, cw);
+    const uint32_t hi = __builtin_amdgcn_perm(cb, ca, 0x05040100u), lo = __builtin_amdgcn_perm(cb, ca, 0x07060302u);
+    *reinterpret_cast<u4*>(tab + 16 * s) = u4{hi, lo, hi, lo};
+  }
+}
+
+// Key width kind KK: 2-4 bits, 7 = 3.5 bits (4 / 3), 5 = 2.5 bits (3 / 2),
+// the halves split at D / 2.
+template <int D, int KK>
+struct KGeo {
+  static constexpr bool FR = KK > 4;
+  static constexpr int NSEG = FR ? 2 : 1;
+  static constexpr int SD = D / NSEG;    // dims per segment
+  static constexpr int SST = SD / 32;    // k-steps per segment
+  static constexpr int KS = D / 32;      // k-steps
+  static constexpr int bits(int seg) { return FR ? (seg ? KK / 2 : (KK + 1) / 2) : KK; }
+  static constexpr int segb(int seg) { return SD * bits(seg) / 32; }  // bytes per lane and segment
+  static constexpr int ndw(int seg) { return (segb(seg) + 3) / 4; }
+  static constexpr int NDW = FR ? ndw(0) + ndw(1) : ndw(0);
+  static constexpr int tab(int seg) { return seg ? (1 << (2 * bits(0))) * TROW : 0; }  // table offset
+  static constexpr int TABS = tab(0) + (1 << (2 * bits(0))) * TROW + (FR ? (1 << (2 * bits(1))) * TROW : 0);
+};
+
+// LDS: [key tables | value tables], reused by the combine buffers, then (from
+// MfmaArgs::tail) the query operands, the combine headers and the norm staging.
+template <int D, int GC>
+struct Lds {
+  static constexpr int QS = 2 * D + 16;               // bytes per (head, part) of the query operands
+  static constexpr int CMS = D + 4;                   // floats per (wave, head) of the combine buffers
+  static constexpr int cmb = MW * GC * CMS * 4;
+  static constexpr int qop = 0;                       // offsets past tail
+  static constexpr int cml = qop + GC * 2 * QS;
+  static constexpr int nst = cml + MW * GC * 8;
+  static constexpr int end = nst + MW * 256;
+};
+
+template <int D, int KK>
+struct Blk {
+  uint32_t k[2][KGeo<D, KK>::NDW];
+  uint32_t v[8][D == 256 ? 2 : 1];
+  float nk, nv;  // of token t0 + (lane & 31)
+};
+
+template <int D, int GC, int KK, bool BF>
+__global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
+  using G_ = KGeo<D, KK>;
+  using L_ = Lds<D, GC>;
+  constexpr int U = D / 16;           // dims per MFMA row of the output
+  constexpr int NF = U / 2;           // pair fields per row
+  constexpr int VW = D == 256 ? 2 : 1;
+  constexpr int TS = GC == 4 ? 2 : 1; // tiles sharing the columns
+  constexpr int NS = 8 / TS;          // scores per lane per block
+  constexpr int PSD = D + 4;
+  extern __shared__ __align__(16) uint8_t smem[];
+  uint8_t* tail = smem + a.tail;
+
+  const int c = blockIdx.x, gy = blockIdx.y, b = blockIdx.z;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, q4 = lane >> 4;
+  const int kvh = gy / a.gsub, row = b * a.hkv + kvh;
+  const int head0 = gy * a.g;  // query head of the group's first column: kvh (hq / hkv) + (gy % gsub) g
+  const int c8 = r & 7;
+  const int tile = TS == 2 ? r >> 3 : 0;
+  const bool lo_part = TS == 2 ? c8 >= 4 : r >= 8;
+  const int hc = TS == 2 ? (c8 < 4 ? c8 : 7 - c8) : c8;
+  const int hd = hc < a.g ? hc : 0;
+  const bool writer = !lo_part && c8 < a.g && tile == 0;
+  const float partf = lo_part ? 1.f : 0.f;
+  const bool packed = c < a.ncw;
+
+  auto clampi = [](int v, int mx) { return min(max(v, 0), mx); };
+  const int comp = a.comp_len_b ? clampi(a.comp_len_b[b], a.max_comp) : a.max_comp;
+  const int sink = a.sink_len_b ? clampi(a.sink_len_b[b], a.max_sink) : a.max_sink;
+  const int res = a.res_len_b ? clampi(a.res_len_b[b], a.max_res) : a.max_res;
+  const int nfp = sink + res;
+  // blocks [blk0, blk1) of 32 tokens
+  const int nblk = ((packed ? comp : nfp) + 31) >> 5;
+  const int share = packed ? (nblk + a.ncw - 1) / a.ncw : (nblk + a.nfw - 1) / a.nfw;
+  const int blk0 = (packed ? c : c - a.ncw) * share, blk1 = min(blk0 + share, nblk);
+  float* part = a.part + ((int64_t)(b * gridDim.y + gy) * gridDim.x + c) * a.g * PSD;
+  if (blk0 >= blk1) {  // nothing of this sequence (uniform over the workgroup): empty partials
+    if (tid < a.g) *reinterpret_cast<float4*>(part + tid * PSD) = make_float4(M_INIT, 0.f, 0.f, 0.f);
+    return;
+  }
+
+  // ---- loads of the compressed blocks: tokens past the sequence read its
+  // last token (masked); all addresses stay inside the sequence's rows
+  const uint8_t* kb0 = a.kc + (int64_t)row * a.k_hs;
+  const uint8_t* kb1 = G_::FR ? a.kcl + (int64_t)row * a.kl_hs : nullptr;
+  const float* knorm = a.kn + (int64_t)row * a.kn_hs;
+  const float* vnorm = a.vn + (int64_t)row * a.vn_hs;
+  // the value codes of MFMA row r: dims U r .. of the hi row (r < 8 or an
+  // integer width) or of the lo row, read as dwords kept inside the row
+  const bool vlo = a.vfrac && r >= 8;
+  const int vb = vlo ? a.vbl : a.vbh;                        // width of this lane's dims
+  const int vrow = (a.vfrac ? D / 2 : D) * vb / 8;           // bytes per token
+  const uint8_t* vp = vlo ? a.vcl + (int64_t)row * a.vl_hs : a.vc + (int64_t)row * a.v_hs;
+  int voff[VW], vsh[VW];
+#pragma unroll
+  for (int i = 0; i < VW; ++i) {
+    const int bit = vb * (U * (vlo ? r - 8 : r) + 8 * i);
+    voff[i] = min(bit >> 3, vrow - 4);
+    vsh[i] = bit - 8 * voff[i];
+  }
+  auto load_blk = [&](Blk<D, KK>& B, int blk) {
+    const int t0 = blk << 5, last = comp - 1;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const uint32_t tt = min(t0 + 16 * t + r, last);
+      uint32_t w0[G_::ndw(0)];
+      load_bytes<G_::segb(0)>(w0, kb0 + (tt * (uint32_t)(4 * G_::segb(0)) + q4 * G_::segb(0)));
+#pragma unroll
+      for (int i = 0; i < G_::ndw(0); ++i) B.k[t][i] = w0[i];
+      if constexpr (G_::FR) {
+        uint32_t w1[G_::ndw(1)];
+        load_bytes<G_::segb(1)>(w1, kb1 + (tt * (uint32_t)(4 * G_::segb(1)) + q4 * G_::segb(1)));
+#pragma unroll
+        for (int i = 0; i < G_::ndw(1); ++i) B.k[t][G_::ndw(0) + i] = w1[i];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint32_t tt = min(t0 + (i < 4 ? 4 * q4 + i : 12 + 4 * q4 + i), last);
+#pragma unroll
+      for (int j = 0; j < VW; ++j) __builtin_memcpy(&B.v[i][j], vp + (tt * (uint32_t)vrow + voff[j]), 4);
+    }
+    const int tn = min(t0 + (lane & 31), last);
+    B.nk = knorm[tn];
+    B.nv = vnorm[tn];
+  };
+
+  // ---- set-up: codebooks (one centroid per lane: key hi / lo, value hi / lo
+  // in the four 16-lane rows), the query rows, the first block
+  uint32_t cw = 0;
+  Blk<D, KK> B0, B1;
+  if (packed) {
+    const float* bp = q4 == 0 ? a.kcen_hi : q4 == 1 ? a.kcen_lo : q4 == 2 ? a.vcen_hi : a.vcen_lo;
+    const int nb = 1 << (q4 == 0 ? G_::bits(0) : q4 == 1 ? G_::bits(G_::NSEG - 1) : q4 == 2 ? a.vbh : a.vbl);
+    const float x = bp[min(r, nb - 1)];
+    const _Float16 h = (_Float16)x, l = (_Float16)(x - (float)h);
+    cw = (uint32_t)__builtin_bit_cast(uint16_t, h) | (uint32_t)__builtin_bit_cast(uint16_t, l) << 16;
+  }
+  // q rows as MFMA A operands (row r = head min(r, g - 1), k-slots = dims 32 kb
+  // + 8 q4 ..): fp16 high part and remainder of q 2^-qe (query_exponent)
+  half8 qo_hi[G_::KS], qo_lo[G_::KS];
+  float qe_scale;
+  {
+    const int esz = a.q_dtype == TQ_F32 ? 4 : 2;
+    const uint8_t* qr = static_cast<const uint8_t*>(a.q) + ((int64_t)b * a.hq + head0 + min(r, a.g - 1)) * D * esz;
+    float x[G_::KS][8];
+#pragma unroll
+    for (int kb = 0; kb < G_::KS; ++kb) {
+      const int d = 32 * kb + 8 * q4;
+      if (a.q_dtype == TQ_F32) {
+        const float4 u0 = *reinterpret_cast<const float4*>(qr + 4 * d);
+        const float4 u1 = *reinterpret_cast<const float4*>(qr + 4 * d + 16);
+        x[kb][0] = u0.x; x[kb][1] = u0.y; x[kb][2] = u0.z; x[kb][3] = u0.w;
+        x[kb][4] = u1.x; x[kb][5] = u1.y; x[kb][6] = u1.z; x[kb][7] = u1.w;
+      } else {
+        const u4 u = *reinterpret_cast<const u4*>(qr + 2 * d);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const uint32_t hb = (u[i >> 1] >> (16 * (i & 1))) & 0xFFFFu;
+          x[kb][i] = a.q_dtype == TQ_BF16 ? __uint_as_float(hb << 16) : (float)__builtin_bit_cast(_Float16, (uint16_t)hb);
+        }
+      }
+    }
+    if (packed) load_blk(B0, min(blk0 + w, blk1 - 1));
+    float ss = 0.f;
+#pragma unroll
+    for (int kb = 0; kb < G_::KS; ++kb)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) ss = fmaf(x[kb][i], x[kb][i], ss);
+    ss = rows_sum(ss);  // the 4 lanes of row r hold the dims of its head
+    const int qe = query_exponent(sqrtf(ss), a.qscale, uk::Q_LIMIT, uk::Q_LOW);
+    const float qdown = __builtin_amdgcn_ldexpf(1.f, -qe);
+#pragma unroll
+    for (int kb = 0; kb < G_::KS; ++kb)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float xs = x[kb][i] * qdown;
+        qo_hi[kb][i] = (_Float16)xs;
+        qo_lo[kb][i] = (_Float16)(xs - (float)qo_hi[kb][i]);
+      }
+    qe_scale = __builtin_amdgcn_ldexpf(1.f, __builtin_amdgcn_ds_bpermute(4 * hd, qe));  // lane h: head h
+  }
+  uint8_t* qop = tail + L_::qop;
+  if (packed) {
+    // rotated query, D[h][n] = sum_i q[h][i] R[j0 + n][i], written (times
+    // qscale) as fp16 high part / remainder rows [head][part][D]
+    for (int jt = w; jt < U; jt += MW) {
+      const uint16_t* rh = a.rot16 + (16 * jt + r) * D + 8 * q4;
+      u4 rqh[G_::KS], rql[G_::KS];
+#pragma unroll
+      for (int kb = 0; kb < G_::KS; ++kb) {
+        rqh[kb] = *reinterpret_cast<const u4*>(rh + 32 * kb);
+        rql[kb] = *reinterpret_cast<const u4*>(rh + D * D + 32 * kb);
+      }
+      f4 dq = {0.f, 0.f, 0.f, 0.f}, dl = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kb = 0; kb < G_::KS; ++kb) {
+        dq = mfma(qo_hi[kb], as_h8(rqh[kb]), dq);
+        dl = mfma(qo_hi[kb], as_h8(rql[kb]), dl);
+        dl = mfma(qo_lo[kb], as_h8(rqh[kb]), dl);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int h = 4 * q4 + i;
+        if (h < a.g && h < GC) {
+          const float v = (dq[i] + dl[i]) * a.qscale;
+          const _Float16 hi = (_Float16)v, lo = (_Float16)(v - (float)hi);
+          uint8_t* d = qop + (h * 2) * L_::QS + 2 * (16 * jt + r);
+          *reinterpret_cast<_Float16*>(d) = hi;
+          *reinterpret_cast<_Float16*>(d + L_::QS) = lo;
+        }
+      }
+    }
+    build_table(smem, 0, G_::bits(0), cw, tid);
+    if constexpr (G_::FR) build_table(smem + G_::tab(1), 1, G_::bits(1), cw, tid);
+    build_table(smem + G_::TABS, 2, a.vbh, cw, tid);
+    if (a.vfrac) build_table(smem + G_::TABS + (1 << (2 * a.vbh)) * TROW, 3, a.vbl, cw, tid);
+  } else if (w == 0 && r < a.g && r < GC) {
+    // uncompressed tokens: the query in original space
+#pragma unroll
+    for (int kb = 0; kb < G_::KS; ++kb) {
+      uint8_t* d = qop + (r * 2) * L_::QS + 2 * (32 * kb + 8 * q4);
+      *reinterpret_cast<half8*>(d) = qo_hi[kb];
+      *reinterpret_cast<half8*>(d + L_::QS) = qo_lo[kb];
+    }
+  }
+  __syncthreads();
+
+  // B operands of the scores: step (seg, s) k-slot (q4, e) is dim seg SD +
+  // q4 SD / 4 + 8 s + e (original space: one segment)
+  half8 qb[G_::KS];
+  {
+    const uint8_t* src = qop + (hd * 2 + (lo_part ? 1 : 0)) * L_::QS;
+#pragma unroll
+    for (int s = 0; s < G_::KS; ++s) {
+      const int seg = packed ? s / G_::SST : 0;
+      const int d = packed ? seg * G_::SD + q4 * (G_::SD / 4) + 8 * (s % G_::SST) : q4 * (D / 4) + 8 * s;
+      qb[s] = *reinterpret_cast<const half8*>(src + 2 * d);
+    }
+  }
+
+  // ---- online softmax in base 2, per lane, of column r
+  float m_run = M_INIT, l_run = 0.f;
+  int vx = 0;         // exponent of the column: acc holds the sums times 2^-vx
+  bool vset = false;  // vx set by the wave's first block with a nonzero weight (wave-uniform)
+  f4 acc[U];
+#pragma unroll
+  for (int nb = 0; nb < U; ++nb) acc[nb] = f4{0.f, 0.f, 0.f, 0.f};
+
+  auto softmax_pv = [&](float (&s)[NS], const float (&nv)[NS]) {
+    float bm = s[0];
+#pragma unroll
+    for (int i = 1; i < NS; ++i) bm = fmaxf(bm, s[i]);
+    bm = rows_max(bm);
+    if (__builtin_amdgcn_ballot_w64(bm > m_run) != 0) {
+      const float mnew = bm > m_run ? bm + uk::RESCALE_MARGIN : m_run;
+      const float corr = fexp2(m_run - mnew);
+      l_run *= corr;
+#pragma unroll
+      for (int nb = 0; nb < U; ++nb) acc[nb] *= corr;
+      m_run = mnew;
+    }
+    float pv[NS];
+    float pm = 0.f;
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      const float p = fexp2(s[i] - m_run);
+      l_run += p;
+      pv[i] = p * nv[i];
+      pm = fmaxf(pm, fabsf(pv[i]));
+    }
+    const float pmx = pm * __builtin_amdgcn_ldexpf(1.f, -vx);
+    if (__builtin_amdgcn_ballot_w64(pmx > uk::PV_LIMIT || (!vset && pmx > 0.f)) != 0) {
+      const float cm = rows_max(pmx);  // max of the column
+      int dx;
+      if (!vset) {
+        dx = cm > 0.f ? max((int)ceilf(log2f(cm / uk::PV_SET)), -110) : 0;
+        vset = true;
+      } else {
+        dx = cm > uk::PV_LIMIT ? (int)ceilf(log2f(cm / uk::PV_LIMIT)) : 0;
+      }
+      const float f = __builtin_amdgcn_ldexpf(1.f, -dx);
+#pragma unroll
+      for (int nb = 0; nb < U; ++nb) acc[nb] *= f;
+      vx += dx;
+    }
+    const float down = __builtin_amdgcn_ldexpf(1.f, -vx);
+    uint32_t d[NS / 2];
+#pragma unroll
+    for (int j = 0; j < NS / 2; ++j) {
+      const float p0 = pv[2 * j] * down, p1 = pv[2 * j + 1] * down;
+      const hx2 h = __builtin_amdgcn_cvt_pkrtz(p0, p1);
+      d[j] = pk_rtz(fmaf(-partf, (float)h[0], p0), fmaf(-partf, (float)h[1], p1));
+    }
+    u4 pb;
+    if constexpr (TS == 2) {
+      pb[0] = tile ? 0u : d[0];
+      pb[1] = tile ? 0u : d[1];
+      pb[2] = tile ? d[0] : 0u;
+      pb[3] = tile ? d[1] : 0u;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) pb[j] = d[j];
+    }
+    return as_h8(pb);
+  };
+  // the scores of this lane from the two tiles' MFMA results, times `f` per
+  // token; masked past `end` tokens
+  auto lane_scores = [&](float (&sc)[NS], f4 sA, f4 sB, const float (&f)[NS], int t0, int end) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (TS == 2) {
+        const float sv = tile ? sB[i] : sA[i];
+        sc[i] = (sv + uk::partner<4>(sv)) * f[i];
+      } else {
+        sc[i] = (sA[i] + uk::partner<8>(sA[i])) * f[i];
+        sc[4 + i] = (sB[i] + uk::partner<8>(sB[i])) * f[4 + i];
+      }
+    }
+    if (t0 + 32 > end) {
+#pragma unroll
+      for (int i = 0; i < NS; ++i)
+        if (t0 + 16 * (tile + (i >> 2)) + 4 * q4 + (i & 3) >= end) sc[i] = -INFINITY;
+    }
+  };
+
+  if (packed) {
+    const uint32_t cp = (uint32_t)r * 8;  // replica of this lane
+    const uint32_t cpv = cp + G_::TABS + (vlo ? (1u << (2 * a.vbh)) * TROW : 0u);
+    const uint32_t vbw = 2 * vb;  // bits per field
+    float* nst = reinterpret_cast<float*>(tail + L_::nst) + w * 64;  // [key norms 32][value norms 32]
+    auto lut = [&](uint32_t addr) { return *reinterpret_cast<const u2*>(smem + addr); };
+    auto compute = [&](const Blk<D, KK>& B, int blk) {
+      const int t0 = blk << 5;
+      nst[lane] = lane < 32 ? B.nk : B.nv;
+      float nk[NS], nv[NS];
+#pragma unroll
+      for (int t = 0; t < 2 / TS; ++t) {
+        const float4 k4 = *reinterpret_cast<const float4*>(nst + 16 * (t + tile) + 4 * q4);
+        const float4 v4 = *reinterpret_cast<const float4*>(nst + 32 + 16 * (t + tile) + 4 * q4);
+        nk[4 * t] = k4.x * qe_scale; nk[4 * t + 1] = k4.y * qe_scale;
+        nk[4 * t + 2] = k4.z * qe_scale; nk[4 * t + 3] = k4.w * qe_scale;
+        nv[4 * t] = v4.x; nv[4 * t + 1] = v4.y; nv[4 * t + 2] = v4.z; nv[4 * t + 3] = v4.w;
+      }
+      f4 sc2[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+      for (int s = 0; s < G_::KS; ++s) {
+        const int seg = s / G_::SST, bits = G_::bits(seg), o = seg ? G_::ndw(0) : 0;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          u4 hi, lo;
+#pragma unroll
+          for (int f = 0; f < 4; ++f) {
+            const int bit = bits * (8 * (s % G_::SST) + 2 * f), wd = o + (bit >> 5), sh = bit & 31;
+            const uint32_t x = sh + 2 * bits <= 32
+                                   ? B.k[t][wd] >> sh
+                                   : __builtin_amdgcn_alignbit(B.k[t][wd + 1 < G_::NDW ? wd + 1 : wd], B.k[t][wd], sh);
+            const u2 e = lut((((x & ((1u << (2 * bits)) - 1u)) * TROW) | cp) + G_::tab(seg));
+            hi[f] = e[0];
+            lo[f] = e[1];
+          }
+          sc2[t] = mfma(as_h8(hi), qb[s], sc2[t]);
+          sc2[t] = mfma(as_h8(lo), qb[s], sc2[t]);
+        }
+      }
+      float sc[NS];
+      lane_scores(sc, sc2[0], sc2[1], nk, t0, comp);
+      const half8 pb = softmax_pv(sc, nv);
+#pragma unroll
+      for (int f = 0; f < NF; ++f) {
+        // dims U r + 2 f, + 1 of the block's 4 token pairs
+        u4 va0, va1, vl0, vl1;
+        const uint32_t off = (uint32_t)vsh[f >> 2] + vbw * (f & 3);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const u2 x = lut(__builtin_amdgcn_ubfe(B.v[2 * j][f >> 2], off, vbw) * TROW + cpv);
+          const u2 y = lut(__builtin_amdgcn_ubfe(B.v[2 * j + 1][f >> 2], off, vbw) * TROW + cpv);
+          va0[j] = __builtin_amdgcn_perm(y[0], x[0], 0x05040100u);
+          va1[j] = __builtin_amdgcn_perm(y[0], x[0], 0x07060302u);
+          vl0[j] = __builtin_amdgcn_perm(y[1], x[1], 0x05040100u);
+          vl1[j] = __builtin_amdgcn_perm(y[1], x[1], 0x07060302u);
+        }
+        acc[2 * f] = mfma(as_h8(va0), pb, acc[2 * f]);
+        acc[2 * f + 1] = mfma(as_h8(va1), pb, acc[2 * f + 1]);
+        acc[2 * f] = mfma(as_h8(vl0), pb, acc[2 * f]);
+        acc[2 * f + 1] = mfma(as_h8(vl1), pb, acc[2 * f + 1]);
+      }
+    };
+    // two blocks in flight; blocks past the wave's share re-read its last one
+    int blk = blk0 + w;
+    if (blk < blk1) {
+      for (;;) {
+        load_blk(B1, min(blk + MW, blk1 - 1));
+        compute(B0, blk);
+        blk += MW;
+        if (blk >= blk1) break;
+        load_blk(B0, min(blk + MW, blk1 - 1));
+        compute(B1, blk);
+        blk += MW;
+        if (blk >= blk1) break;
+      }
+    }
+  } else {
+    // uncompressed tokens: keys / values straight from memory
+    const int rstart = clampi(a.res_start_b ? a.res_start_b[b] : a.res_start0, max(a.res_cap - 1, 0));
+    const uint16_t* sk = static_cast<const uint16_t*>(a.sink_k) + (int64_t)row * a.sink_hs;
+    const uint16_t* sv = static_cast<const uint16_t*>(a.sink_v) + (int64_t)row * a.sink_hs;
+    const uint16_t* rk = static_cast<const uint16_t*>(a.res_k) + (int64_t)row * a.res_hs;
+    const uint16_t* rv = static_cast<const uint16_t*>(a.res_v) + (int64_t)row * a.res_hs;
+    auto token = [&](int u, const uint16_t* s0, const uint16_t* r0) {
+      u = min(u, nfp - 1);
+      int sl = rstart + (u - sink);
+      sl = sl >= a.res_cap ? sl - a.res_cap : sl;
+      return u < sink ? s0 + (int64_t)u * D : r0 + (int64_t)sl * D;
+    };
+    for (int blk = blk0 + w; blk < blk1; blk += MW) {
+      const int t0 = blk << 5;
+      u4 kr[2][G_::KS];
+      uint32_t vr[8][U / 2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const uint16_t* p = token(t0 + 16 * t + r, sk, rk) + q4 * (D / 4);
+#pragma unroll
+        for (int s = 0; s < G_::KS; ++s) kr[t][s] = *reinterpret_cast<const u4*>(p + 8 * s);
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const uint16_t* p = token(t0 + (i < 4 ? 4 * q4 + i : 12 + 4 * q4 + i), sv, rv) + U * r;
+        __builtin_memcpy(&vr[i][0], __builtin_assume_aligned(p, 4), 2 * U);
+      }
+      // bf16: keys and values of the block scaled by powers of two that bring
+      // the largest |x| of each into [2^14, 2^15): exact in fp16 down to 2^-38
+      // of it; the scores and the weights are scaled back
+      float kback = 1.f, vback = 1.f;
+      if constexpr (BF) {
+        uint32_t mk = 0, mv = 0;
+        auto up = [](uint32_t& m, uint32_t x) {
+          x &= 0x7FFF7FFFu;
+          m = max(m, max(x & 0xFFFFu, x >> 16));
+        };
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int s = 0; s < G_::KS; ++s)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) up(mk, kr[t][s][i]);
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+          for (int j = 0; j < U / 2; ++j) up(mv, vr[i][j]);
+        mk = wave_max_u32(mk);
+        mv = wave_max_u32(mv);
+        const int ek = mk == 0u ? 0 : max(-100, (int)(mk >> 7) - 127 - 14);
+        const int ev = mv == 0u ? 0 : max(-100, (int)(mv >> 7) - 127 - 14);
+        const float ks = __builtin_amdgcn_ldexpf(1.f, -ek), vs = __builtin_amdgcn_ldexpf(1.f, -ev);
+        kback = __builtin_amdgcn_ldexpf(1.f, ek);
+        vback = __builtin_amdgcn_ldexpf(1.f, ev);
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int s = 0; s < G_::KS; ++s) kr[t][s] = uk::bf16_to_f16(kr[t][s], ks);
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+          for (int j = 0; j < U / 2; ++j)
+            vr[i][j] = pk_rtz(__uint_as_float(vr[i][j] << 16) * vs, __uint_as_float(vr[i][j] & 0xFFFF0000u) * vs);
+      }
+      f4 sc2[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+      for (int s = 0; s < G_::KS; ++s)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) sc2[t] = mfma(as_h8(kr[t][s]), qb[s], sc2[t]);
+      float sc[NS], kf[NS], nv[NS];
+#pragma unroll
+      for (int i = 0; i < NS; ++i) kf[i] = a.qscale * qe_scale * kback, nv[i] = vback;
+      lane_scores(sc, sc2[0], sc2[1], kf, t0, nfp);
+      const half8 pb = softmax_pv(sc, nv);
+#pragma unroll
+      for (int nb = 0; nb < U; ++nb) {
+        const uint32_t sel = (nb & 1) ? 0x07060302u : 0x05040100u;
+        u4 va;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) va[j] = __builtin_amdgcn_perm(vr[2 * j + 1][nb >> 1], vr[2 * j][nb >> 1], sel);
+        acc[nb] = mfma(as_h8(va), pb, acc[nb]);
+      }
+    }
+  }
+
+  // ---- combine the waves through LDS (the table region); the two fp16 parts
+  // of a head meet through `partner`, for GC = 4 the two tiles at their common max
+  l_run = rows_sum(l_run);
+  float tsc = __builtin_amdgcn_ldexpf(1.f, vx);
+  if constexpr (TS == 2) {
+    const float m2 = fmaxf(m_run, row_ror<8>(m_run));
+    const float t = fexp2(m_run - m2);
+    tsc *= t;
+    l_run *= t;
+    l_run += row_ror<8>(l_run);
+    m_run = m2;
+  }
+  __syncthreads();
+  float* cm = reinterpret_cast<float*>(smem) + (w * GC) * L_::CMS;
+  float* cl = reinterpret_cast<float*>(tail + L_::cml);  // [wave][head][M, L]
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float vr[U];
+#pragma unroll
+    for (int nb = 0; nb < U; ++nb) {
+      float x = (acc[nb][i] + uk::partner<GC>(acc[nb][i])) * tsc;
+      if constexpr (TS == 2) x += row_ror<8>(x);
+      vr[nb] = x;
+    }
+    if (writer) {
+      float* d = cm + hd * L_::CMS + U * (4 * q4 + i);
+#pragma unroll
+      for (int nb = 0; nb < U; nb += 2) *reinterpret_cast<float2*>(d + nb) = make_float2(vr[nb], vr[nb + 1]);
+    }
+  }
+  if (q4 == 0 && writer) *reinterpret_cast<float2*>(cl + (w * GC + hd) * 2) = make_float2(m_run, l_run);
+  __syncthreads();
+  const float* cms = reinterpret_cast<const float*>(smem);
+  for (int e = tid; e < a.g * D; e += MTH) {
+    const int h = e / D, j = e % D;
+    float M = M_INIT;
+#pragma unroll
+    for (int ww = 0; ww < MW; ++ww) M = fmaxf(M, cl[(ww * GC + h) * 2]);
+    float sr = 0.f, Ls = 0.f;
+#pragma unroll
+    for (int ww = 0; ww < MW; ++ww) {
+      const float2 st = *reinterpret_cast<const float2*>(cl + (ww * GC + h) * 2);
+      const float sc = fexp2(st.x - M);
+      sr = fmaf(sc, cms[(ww * GC + h) * L_::CMS + j], sr);
+      Ls = fmaf(sc, st.y, Ls);
+    }
+    part[h * PSD + 4 + j] = Ls > 0.f ? sr / Ls : 0.f;
+    if (j == 0) *reinterpret_cast<float4*>(part + h * PSD) = make_float4(M, Ls, 0.f, 0.f);
+  }
+}
+
+// Merge of the np = ncw + nfw partials of a query head: with w_p = 2^(M_p - M)
+// L_p / L, out = (sum_{p < ncw} w_p y_p) R + sum_{p >= ncw} w_p x_p (x = R^T y,
+// R the value codec's float32 rotation). Grid (hq, batch), NT threads: PG
+// groups of D threads sum the partials p = group + PG k; for the rotation
+// thread (4 columns, row block) takes D / RB rows of R, requested before the
+// partials are waited for.
+template <int D>
+struct MergeGeo {
+  static constexpr int NT = D == 256 ? 1024 : 256;
+  static constexpr int PG = NT / D;             // partial groups (4 / 2 / 2 / 4)
+  static constexpr int CT = D / 4;              // column threads of a row block
+  static constexpr int RB = D == 96 ? 8 : NT / CT;  // row blocks
+  static constexpr int RR = D / RB;             // rows per block
+};
+
+template <int D>
+__global__ __launch_bounds__(MergeGeo<D>::NT) void mfma_merge_kernel(MfmaArgs a, int np) {
+  using M_ = MergeGeo<D>;
+  constexpr int PSD = D + 4, MB = 8;
+  extern __shared__ __align__(16) uint8_t smem[];
+  float* wsh = reinterpret_cast<float*>(smem);  // [np rounded to 64] weights, then
+  __shared__ float ys[M_::PG][D], xs[M_::PG][D];
+  __shared__ __align__(16) float red[M_::RB][D];
+  const int hq = blockIdx.x, b = blockIdx.y;
+  const int gq = a.hq / a.hkv / a.gsub;  // == a.g
+  const int gy = hq / gq, h = hq % gq;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int64_t pst = (int64_t)a.g * PSD;
+  const float* pp = a.part + (int64_t)(b * a.hkv * a.gsub + gy) * np * pst + h * PSD;
+  const int d = tid % D, grp = tid / D;
+  const bool act = grp < M_::PG;
+  float x[MB];
+  auto load = [&](int p0) {
+#pragma unroll
+    for (int i = 0; i < MB; ++i) x[i] = pp[min(p0 + M_::PG * i + grp, np - 1) * pst + 4 + d];
+  };
+  // every wave reads all headers for the max and the sum; wave 0 keeps the weights
+  float M = M_INIT;
+  for (int p = lane; p < np; p += 64) {
+    const float2 hd = *reinterpret_cast<const float2*>(pp + p * pst);
+    M = hd.y > 0.f ? fmaxf(M, hd.x) : M;
+  }
+  load(0);
+  const int j4 = 4 * (tid % M_::CT), ib = tid / M_::CT;
+  float4 rr[M_::RR];
+  if (ib < M_::RB) {
+#pragma unroll
+    for (int k = 0; k < M_::RR; ++k) rr[k] = *reinterpret_cast<const float4*>(a.vrot + (M_::RR * ib + k) * D + j4);
+  }
+  M = uk::wave_max(M);
+  float ls = 0.f;
+  for (int p = lane; p < np; p += 64) {
+    const float2 hd = *reinterpret_cast<const float2*>(pp + p * pst);
+    const float wp = hd.y > 0.f ? fexp2(hd.x - M) * hd.y : 0.f;
+    if (tid < 64) wsh[p] = wp;
+    ls += wp;
+  }
+  const float Ls = uk::wave_sum(ls);
+  const float inv = Ls > 0.f ? 1.f / Ls : 0.f;
+  __syncthreads();
+  float acc = 0.f, acco = 0.f;
+  for (int p0 = 0;;) {
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+      const int p = p0 + M_::PG * i + grp;
+      const float wp = act && p < np ? wsh[p] : 0.f;
+      const float v = wp != 0.f ? x[i] : 0.f;  // (empty partials may hold anything)
+      acc = fmaf(p < a.ncw ? wp : 0.f, v, acc);
+      acco = fmaf(p < a.ncw ? 0.f : wp, v, acco);
+    }
+    p0 += M_::PG * MB;
+    if (p0 >= np) break;
+    load(p0);
+  }
+  if (act) {
+    ys[grp][d] = acc;
+    xs[grp][d] = acco;
+  }
+  __syncthreads();
+  if (ib < M_::RB) {
+    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int k = 0; k < M_::RR; ++k) {
+      float y = 0.f;
+#pragma unroll
+      for (int q = 0; q < M_::PG; ++q) y += ys[q][M_::RR * ib + k];
+      o.x = fmaf(y, rr[k].x, o.x);
+      o.y = fmaf(y, rr[k].y, o.y);
+      o.z = fmaf(y, rr[k].z, o.z);
+      o.w = fmaf(y, rr[k].w, o.w);
+    }
+    *reinterpret_cast<float4*>(&red[ib][j4]) = o;
+  }
+  __syncthreads();
+  if (tid < D) {
+    float s = 0.f;
+#pragma unroll
+    for (int k = 0; k < M_::RB; ++k) s += red[k][tid];
+#pragma unroll
+    for (int q = 0; q < M_::PG; ++q) s += xs[q][tid];
+    a.out[((int64_t)b * a.hq + hq) * D + tid] = s * inv;
+  }
+}
+
+template <int D, int GC, int KK>
+static void launch_k(const MfmaArgs& a, bool bf, hipStream_t s) {
+  using G_ = KGeo<D, KK>;
+  MfmaArgs x = a;
+  const int vt = (1 << (2 * a.vbh)) * TROW + (a.vfrac ? (1 << (2 * a.vbl)) * TROW : 0);
+  x.tail = G_::TABS + vt > Lds<D, GC>::cmb ? G_::TABS + vt : Lds<D, GC>::cmb;
+  const int lds = x.tail + Lds<D, GC>::end;
+  const dim3 grid(a.ncw + a.nfw, a.hkv * a.gsub, a.batch);
+  if (bf)
+    hipLaunchKernelGGL((mfma_decode_kernel<D, GC, KK, true>), grid, dim3(MTH), lds, s, x);
+  else
+    hipLaunchKernelGGL((mfma_decode_kernel<D, GC, KK, false>), grid, dim3(MTH), lds, s, x);
+}
+
+template <int D, int KK>
+static void launch_g(const MfmaArgs& a, bool bf, hipStream_t s) {
+  if (a.g <= 4)
+    launch_k<D, 4, KK>(a, bf, s);
+  else
+    launch_k<D, 8, KK>(a, bf, s);
+}
+
+// kk: key width kind (KGeo)
+template <int D>
+int launch_mfma(const MfmaArgs& a, int kk, bool bf, hipStream_t s) {
+  switch (kk) {
+    case 2: launch_g<D, 2>(a, bf, s); break;
+    case 3: launch_g<D, 3>(a, bf, s); break;
+    case 4: launch_g<D, 4>(a, bf, s); break;
+    case 5:
+      if constexpr (D != 96) launch_g<D, 5>(a, bf, s);
+      break;
+    case 7:
+      if constexpr (D != 96) launch_g<D, 7>(a, bf, s);
+      break;
+    default: return -1;
+  }
+  const int np = a.ncw + a.nfw;
+  hipLaunchKernelGGL((mfma_merge_kernel<D>), dim3(a.hq, a.batch), dim3(MergeGeo<D>::NT), ((np + 63) & ~63) * 4, s, a,
+                     np);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+}  // namespace mk
+}  // namespace tq

@@ -1,0 +1,9 @@
+// head_dim 128 instantiations of the decode kernels of tq_decode_mfma.h.
+
+#include "tq_decode_mfma.h"
+
+namespace tq {
+
+int launch_mfma_d128(const MfmaArgs& a, int kk, bool bf, hipStream_t s) { return mk::launch_mfma<128>(a, kk, bf, s); }
+
+}  // namespace tq

@@ -1,0 +1,9 @@
+// head_dim 256 instantiations of the decode kernels of tq_decode_mfma.h.
+
+#include "tq_decode_mfma.h"
+
+namespace tq {
+
+int launch_mfma_d256(const MfmaArgs& a, int kk, bool bf, hipStream_t s) { return mk::launch_mfma<256>(a, kk, bf, s); }
+
+}  // namespace tq

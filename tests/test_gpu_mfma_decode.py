@@ -1,0 +1,153 @@
+"""GPU parity of the decode kernels of tq_decode_mfma.h: head_dim 64 / 96 /
+128 / 256, integer and fractional widths on either side, any number of query
+heads per kv head, fp16 and bf16 uncompressed tokens, uniform and ragged
+batches. The route is asserted through the library's test hook (7), the
+output held to float64 attention over the stored codes at 5e-6 (scores and
+weights carry about 2^-22 relative, as in the K4/V2 kernels' bound) and to the
+general kernel at 1e-4.
+"""
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from gpu_helpers import min_cos, rel_err, to_dev
+from test_gpu_attention import decode_route, dense_from_gpu_codes
+
+pytestmark = pytest.mark.gpu
+
+REL_TOL = 5e-6
+COS_TOL = 0.9999
+
+
+def _kv(B, H, T, D, seed, kmul=1.0, vmul=1.0):
+    rng = np.random.RandomState(seed)
+    s = np.exp(rng.randn(D) * 0.5)
+    return (rng.randn(B, H, T, D) * s * kmul).astype(np.float32), (rng.randn(B, H, T, D) * vmul).astype(np.float32)
+
+
+def _caches(kw, k, v, dt):
+    from turboquant_amd import TurboQuantKVCache
+    kt, vt = torch.from_numpy(k).to(dt), torch.from_numpy(v).to(dt)
+    c = TurboQuantKVCache(**kw)
+    c.update(kt.cuda(), vt.cuda())
+    o = O.CacheOracle(**kw)
+    o.update(kt.float().numpy(), vt.float().numpy())
+    return c, o
+
+
+def _check(c, o, q, label, route=7):
+    qd = to_dev(q)
+    assert decode_route(c, qd) == route
+    fast = c.attend(qd).cpu().numpy()
+    gen = c.attend(qd, general_kernel=True).cpu().numpy()
+    kk, vv = dense_from_gpu_codes(c, o)
+    ref = O.attention(q, kk, vv)
+    print(f"{label}: rel {rel_err(fast, ref):.3e} vs general {rel_err(fast, gen):.3e}")
+    assert np.isfinite(fast).all()
+    assert rel_err(fast, ref) < REL_TOL and min_cos(fast, ref) >= COS_TOL
+    assert rel_err(fast, gen) < 1e-4
+
+
+PAIRS = [(4, 2), (2, 4), (3, 3), (4, 4), (3.5, 2.5), (2.5, 3.5), (3, 2.5)]
+
+
+@pytest.mark.parametrize("D,kb,vb", [(d, k, v) for d in (64, 96, 256) for k, v in PAIRS if d != 96 or k == int(k)] + [
+    (128, 4, 4), (128, 3.5, 2)], ids=str)
+@pytest.mark.parametrize("G,T,sink,window,dt", [
+    (4, 1500, 16, 64, torch.bfloat16),  # a partial last block, one workgroup's uncompressed tokens
+    (7, 700, 0, 32, torch.float16),     # eight columns with an idle one
+    (1, 9000, 300, 300, torch.bfloat16),  # several blocks per wave, three workgroups of uncompressed tokens
+])
+def test_mfma_matches_oracle(D, kb, vb, G, T, sink, window, dt):
+    if D == 128 and dt == torch.float16 and G != 7:
+        pytest.skip("another route")
+    k, v = _kv(1, 2, T, D, seed=int(T + 10 * kb + vb + G))
+    c, o = _caches(dict(head_dim=D, num_kv_heads=2, key_bits=kb, value_bits=vb, residual_window=window,
+                        fp16_sink_size=sink), k, v, dt)
+    q = np.random.RandomState(int(kb * 8 + vb + G)).randn(1, 2 * G, 1, D).astype(np.float16)
+    _check(c, o, q, f"d{D} K{kb}/V{vb} G={G} T={T} {dt}")
+
+
+@pytest.mark.parametrize("D,G,batch", [(128, 3, 2), (64, 16, 1), (256, 10, 1), (96, 12, 3), (128, 5, 1)])
+def test_mfma_query_groups(D, G, batch):
+    """Head groups of at most 8 per launch row: 3, 8 + 8, 5 + 5, 6 + 6, 5."""
+    k, v = _kv(batch, 2, 1000, D, seed=D + G)
+    c, o = _caches(dict(head_dim=D, num_kv_heads=2, residual_window=64, fp16_sink_size=4), k, v, torch.float16)
+    q = np.random.RandomState(G).randn(batch, 2 * G, 1, D).astype(np.float16)
+    _check(c, o, q, f"d{D} G={G} B={batch}")
+
+
+@pytest.mark.parametrize("D,T", [(64, 1), (64, 33), (96, 200), (256, 256)])
+def test_mfma_uncompressed_only(D, T):
+    k, v = _kv(2, 2, T, D, seed=T)
+    c, o = _caches(dict(head_dim=D, num_kv_heads=2, residual_window=128, fp16_sink_size=16), k, v, torch.bfloat16)
+    assert c._compressed_len == 0
+    _check(c, o, np.random.RandomState(T).randn(2, 8, 1, D).astype(np.float16), f"d{D} T={T}")
+
+
+# (a score of magnitude S is exact to about S 2^-22, so its weight to that
+# relative error: 5e-6 holds for |S| up to about 20, logits of std 1.5 here)
+@pytest.mark.parametrize("kmul,vmul,qmul", [(300.0, 3e4, 1.0), (1e-3, 1e-7, 1.0), (1.0, 1.0, 1e-5)])
+@pytest.mark.parametrize("D", [64, 256])
+def test_mfma_magnitudes(D, kmul, vmul, qmul):
+    """bf16 tokens past / below the fp16 range, queries whose fp16 operands
+    need a power of two, value norms that move the weights' exponent."""
+    k, v = _kv(1, 2, 900, D, seed=3, kmul=kmul, vmul=vmul)
+    c, o = _caches(dict(head_dim=D, num_kv_heads=2, residual_window=64, fp16_sink_size=16), k, v, torch.bfloat16)
+    q = (np.random.RandomState(1).randn(1, 8, 1, D) * qmul / kmul).astype(np.float32)
+    _check(c, o, q, f"d{D} k x{kmul} v x{vmul} q x{qmul}")
+
+
+def test_mfma_ragged_equals_single_sequences():
+    """A ragged batch (per-sequence lengths, a sequence with nothing
+    compressed, wrapped rings) on these kernels: each sequence equals its own
+    call over the same stores, whose partials are cut elsewhere."""
+    from turboquant_amd import _lib
+    from turboquant_amd.ragged import RaggedKVBatch
+    H, G, D = 2, 3, 128
+    lens = [40, 300, 1777, 5000]
+    rb = RaggedKVBatch(4, H, head_dim=D, key_bits=3.5, value_bits=3, residual_window=64, fp16_sink_size=16)
+    rng = np.random.RandomState(9)
+    for b, t in enumerate(lens):
+        rb.load(b, *(to_dev(rng.randn(H, t, D).astype(np.float16)) for _ in range(2)))
+    for _ in range(5):
+        rb.step(*(to_dev(rng.randn(4, H, D).astype(np.float16)) for _ in range(2)))
+    q = to_dev(rng.randn(4, H * G, D).astype(np.float16))
+    out = torch.empty(q.shape, dtype=torch.float32, device=q.device)
+    d, keep = rb.descriptor(q, out, D ** -0.5)
+    fn = _lib.load().tq_debug_decode_route
+    fn.restype, fn.argtypes = ctypes.c_int32, [ctypes.c_void_p] * 3
+    assert fn(ctypes.addressof(rb.kc.struct), ctypes.addressof(rb.vc.struct), ctypes.addressof(d)) == 7
+    got = rb.attend(q).cpu().numpy()
+    gen = rb.attend(q, general=True).cpu().numpy()
+    assert np.isfinite(got).all()
+    for b in range(4):
+        assert rel_err(got[b], gen[b]) < REL_TOL, b
+
+
+def test_mfma_graph_replays():
+    """Captured and replayed several times with eager work between: the same
+    output as the eager call."""
+    k, v = _kv(1, 2, 2000, 64, seed=8)
+    c, _ = _caches(dict(head_dim=64, num_kv_heads=2, residual_window=64), k, v, torch.bfloat16)
+    q = to_dev(np.random.RandomState(2).randn(1, 8, 1, 64).astype(np.float16))
+    ref = c.attend(q).clone()
+    out = torch.empty_like(ref)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        c.attend(q, out=out)
+    torch.cuda.current_stream().wait_stream(s)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        c.attend(q, out=out)
+    for _ in range(4):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref)
+        assert torch.equal(c.attend(q), ref)
