@@ -23,6 +23,20 @@ struct CompressArgs {
   int row_hi, row_lo, row_sign;
 };
 
+struct DequantArgs {
+  tq_store src;
+  tq_span span;
+  float* out;
+  int64_t out_hs;
+  const float* rot;
+  const float* cen_hi;
+  const float* cen_lo;
+  const float* proj;
+  int d;  // head_dim
+  int bits_hi, bits_lo, split, qjl_m, apply_qjl;
+  int row_hi, row_lo, row_sign;
+};
+
 // float64 sum of squares of row[0, D) in the library's norm order: 32-dim
 // blocks, each summed sequentially from 0, block sums combined pairwise level
 // by level ((B0+B1)+(B2+B3) for D = 128). Squares of fp16 / fp32 values are
@@ -59,5 +73,9 @@ __device__ inline void store_codes(uint8_t* dst, const uint32_t (&code)[32]) {
 // MFMA compress for fp16 inputs with head_dim 128 and no QJL sketch; returns
 // 1 when it launched, 0 when the arguments need the general kernel.
 int launch_compress_fast(const CompressArgs& a, hipStream_t s);
+
+// MFMA dequantize for head_dim 64 / 96 / 128 / 256 and sketches of at most 128
+// projections; returns 1 when it launched, 0 when the general kernel is needed.
+int launch_dequant_mfma(const DequantArgs& a, hipStream_t s);
 
 }  // namespace tq

@@ -563,20 +563,6 @@ __device__ __forceinline__ void drain_vector(const CompressArgs& a, DrainLds& L,
   }
 }
 
-struct DequantArgs {
-  tq_store src;
-  tq_span span;
-  float* out;
-  int64_t out_hs;
-  const float* rot;
-  const float* cen_hi;
-  const float* cen_lo;
-  const float* proj;
-  int d;  // head_dim
-  int bits_hi, bits_lo, split, qjl_m, apply_qjl;
-  int row_hi, row_lo, row_sign;
-};
-
 template <int DP>
 __global__ __launch_bounds__(256) void dequant_kernel(DequantArgs a) {
   using G = Geo<DP>;
@@ -1130,6 +1116,10 @@ int tq_dequantize(const tq_codec* codec, const tq_store* src, const tq_span* spa
   a.row_lo = row_bytes(codec->d - codec->split, a.bits_lo);
   a.row_sign = a.qjl_m / 8;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (launch_dequant_mfma(a, s)) {
+    TQ_LAUNCH_CHECK("tq_dequantize");
+    return TQ_OK;
+  }
   launch_padded(codec->d, [&](auto dp) {
     constexpr int DP = decltype(dp)::value;
     dim3 g((span->n_tok + Geo<DP>::VPW - 1) / Geo<DP>::VPW, span->rows);
