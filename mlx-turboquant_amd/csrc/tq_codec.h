@@ -74,6 +74,11 @@ __device__ inline void store_codes(uint8_t* dst, const uint32_t (&code)[32]) {
 // 1 when it launched, 0 when the arguments need the general kernel.
 int launch_compress_fast(const CompressArgs& a, hipStream_t s);
 
+// MFMA compress for head_dim 64 / 96 / 128 / 256, any input type, and sketches
+// of at most 128 projections up to head_dim 128; returns 1 when it launched,
+// 0 when the arguments need the general kernel.
+int launch_compress_mfma(const CompressArgs& a, hipStream_t s);
+
 // MFMA dequantize for head_dim 64 / 96 / 128 / 256 and sketches of at most 128
 // projections; returns 1 when it launched, 0 when the general kernel is needed.
 int launch_dequant_mfma(const DequantArgs& a, hipStream_t s);

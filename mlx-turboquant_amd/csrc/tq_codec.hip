@@ -1074,6 +1074,11 @@ int tq_compress(const tq_codec* codec, const void* x, int32_t x_dtype, int64_t x
     TQ_LAUNCH_CHECK("tq_compress");
     return TQ_OK;
   }
+  // other input types and head_dims, sketches (tq_compress_mfma.hip)
+  if (!(codec->flags & TQ_CODEC_GENERAL_COMPRESS) && launch_compress_mfma(a, s)) {
+    TQ_LAUNCH_CHECK("tq_compress");
+    return TQ_OK;
+  }
   launch_padded(codec->d, [&](auto dp) {
     constexpr int DP = decltype(dp)::value;
     dim3 g((span->n_tok + Geo<DP>::VPW - 1) / Geo<DP>::VPW, span->rows);

@@ -1,6 +1,8 @@
 """The MFMA codec kernels outside fp16 / head_dim 128 / no sketch: dequantize
 (tq_dequant_mfma.hip) at the edges of its 32-token tiles, every width kind,
-sketches and per-sequence spans, against float64 over the same codes."""
+sketches and per-sequence spans, against float64 over the same codes; compress
+(tq_compress_mfma.hip) against the oracle (codes outside the float32 boundary
+band, bit-exact norms) and the general kernel."""
 
 import ctypes
 
@@ -9,7 +11,7 @@ import pytest
 import torch
 
 import oracle as O
-from gpu_helpers import rel_err, to_dev
+from gpu_helpers import code_parity, gpu_compress, rel_err, to_dev, unpack_codes
 
 pytestmark = pytest.mark.gpu
 
@@ -67,3 +69,69 @@ def test_dequant_mfma(d, bits, m, n_b, src, dst):
             assert rel_err(x, ref[b, :, src[b]:src[b] + n_b[b]]) < 5e-7
         rest = np.delete(got[b], np.s_[dst[b]:dst[b] + n_b[b]], axis=1)
         assert (rest == 7.0).all()
+
+
+def _compress(x, bits, m=0, general=False):
+    """numpy (codes_hi, codes_lo, norms, signs, gamma) of a (B, H, T, D) tensor."""
+    from turboquant_amd import _codec
+    B, H, T, D = x.shape
+    codec = _codec.get_codec(D, bits, 42, m, x.device)
+    st = _codec.PackedStore(codec, B, H, qjl=m > 0)
+    st.reserve(T, 0)
+    _codec.compress_into(codec, x, 0, T, st, 0, general=general)
+    return tuple(None if t is None else t[:, :, :T].cpu().numpy()
+                 for t in (st.codes_hi, st.codes_lo, st.norms, st.signs, st.gamma))
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("d,bits", [(64, 1), (64, 3.5), (64, 4), (96, 3), (96, 2), (128, 4), (128, 2.5), (128, 1),
+                                    (256, 4), (256, 3.5), (256, 2)])
+@pytest.mark.parametrize("T", [1, 63, 65, 700])
+def test_compress_mfma_codes(d, bits, dt, T):
+    rng = np.random.RandomState(int(d + 10 * bits + T))
+    x = torch.from_numpy(rng.randn(2, 3, T, d).astype(np.float32) * np.exp(rng.randn(2, 3, T, 1)).astype(np.float32)).to(dt)
+    xf = x.float().numpy()
+    _, _, _, _, norms_equal, _ = code_parity(xf, bits, gpu=_compress(x.cuda(), bits))
+    assert norms_equal
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("d,bits,m", [(64, 2, 64), (96, 3, 32), (128, 4, 128), (128, 3.5, 40), (128, 1, 96)])
+def test_compress_mfma_sketch(d, bits, m, dt):
+    """Signs of projections away from zero (|r . S| > 1e-4 ||x||; the residual
+    and its projection carry about 1e-6 ||x||) and residual norms, float64 over
+    the kernel's own codes."""
+    rng = np.random.RandomState(d + m)
+    x = torch.from_numpy(rng.randn(1, 2, 150, d).astype(np.float32)).to(dt)
+    hi, lo, n, signs, gamma = _compress(x.cuda(), bits, m)
+    xf = x.double().numpy()
+    code_parity(x.float().numpy(), bits, gpu=(hi, lo, n, None, None))
+    res = xf - O.dequantize(hi, lo, n, O.rotation_matrix(d), bits, d)
+    from turboquant_amd.qjl import generate_projection_matrix
+    proj = res @ generate_projection_matrix(d, m).astype(np.float64).T
+    got = np.unpackbits(signs, axis=-1, bitorder="little").astype(bool)
+    clear = np.abs(proj) > 1e-4 * np.linalg.norm(xf, axis=-1, keepdims=True)
+    assert clear.mean() > 0.9 and (got[..., :m] == (proj >= 0))[clear].all()
+    assert got[..., m:].all()  # the zero rows past m project to 0: bit set
+    assert rel_err(gamma, np.linalg.norm(res, axis=-1)) < 2e-6
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("d", [64, 96, 128, 256])
+def test_compress_mfma_special_vectors(d, dt):
+    """Zero, tiny, subnormal, huge, overflowing-norm, infinite and NaN vectors:
+    the codes and norms of the general kernel."""
+    rng = np.random.RandomState(d)
+    base = torch.from_numpy(rng.randn(16, d).astype(np.float32))
+    mul = {torch.float16: [1, 0, 6e-8, 1e-6, 1e4], torch.bfloat16: [1, 0, 1e-40, 1e-36, 1e-20, 1e30, 3e37],
+           torch.float32: [1, 0, 1e-42, 1e-37, 1e-20, 1e30, 3e37, 1e38]}[dt]
+    rows = [base * f for f in mul]
+    rows += [base.index_fill(1, torch.tensor([3]), v) for v in (float("inf"), float("-inf"), float("nan"))]
+    x = torch.cat(rows).clamp(-3.3e38, 3.3e38) if dt == torch.float32 else torch.cat(rows)
+    x = torch.cat([x, *(base.index_fill(1, torch.tensor([3]), float("inf")),)]).to(dt)[None, None].cuda().contiguous()
+    for bits in (4, 1):
+        a, b = _compress(x, bits), _compress(x, bits, general=True)
+        assert np.array_equal(a[2], b[2], equal_nan=True)
+        ca, cb = unpack_codes(a[0], a[1], bits, d), unpack_codes(b[0], b[1], bits, d)
+        bad = (ca != cb).any(-1)[0, 0]
+        assert not bad.any(), (np.nonzero(bad)[0] // 16, bits)
