@@ -1601,19 +1601,28 @@ static bool mfma_eligible(const tq_codec* kc, const tq_codec* vc, const tq_attn_
   return d->max_comp > 0 || d->max_sink > 0 || d->max_res > 0;
 }
 
-// Workgroups per (sequence, head group): one wave per 32-token block of the
-// uncompressed tokens, and for the compressed ones what is left of one
-// workgroup per CU (a CU of their own each where the uncompressed tokens
-// alone fill half the chip), at least one block per wave.
+// Workgroups per (sequence, head group) of the mfma kernels. A wave's block is
+// about 1,000 VALU instructions, four cycles each on its SIMD, and a workgroup
+// puts two waves on every SIMD: while CUs are free a workgroup takes MFMA_WAVES
+// / 2 blocks, one wave per SIMD (head_dim 128, 28 heads on 4, T 600: 13.8 ->
+// 13.3 us per layer; head_dim 256, T 600: 25.1 -> 23.9), else an equal share of
+// one workgroup per CU. More than about 60 partials cost the merge a second
+// round of loads (head_dim 256, T 12,000, 96 partials instead of 48: partials
+// 20.2 -> 18.7 us, merge 6.3 -> 8.4 us), so past that the workgroups are filled
+// first. Uncompressed tokens: likewise, 8 blocks per workgroup where 4 would
+// take a quarter of the CUs.
 static void mfma_geometry(const tq_attn_desc* d, int& gsub, int& g, int& ncw, int& nfw) {
   const int G = d->hq / d->hkv;
   g = group_heads(G);
   gsub = G / g;
   const int64_t rows = (int64_t)d->batch * d->hkv * gsub;
-  const int per = MFMA_WAVES * 32;
-  nfw = (int)(((int64_t)d->max_sink + d->max_res + per - 1) / per);
-  const int most = (d->max_comp + per - 1) / per;
+  const int half = MFMA_WAVES / 2 * 32;
   const int cus = device_cus();
+  nfw = (int)(((int64_t)d->max_sink + d->max_res + half - 1) / half);
+  if (rows * nfw > cus / 4) nfw = (nfw + 1) / 2;
+  constexpr int ONE_ROUND = 60;
+  int most = (d->max_comp + half - 1) / half;
+  if (most > ONE_ROUND) most = most / 2 > ONE_ROUND ? (most + 1) / 2 : ONE_ROUND;
   int64_t avail = cus - rows * nfw;
   if (avail < cus / 2) avail = cus;
   const int64_t share = avail / rows > 1 ? avail / rows : 1;
@@ -1649,12 +1658,12 @@ static int mfma_run(const tq_codec* kc, const tq_codec* vc, const tq_attn_desc* 
   a.vcen_hi = vc->centroids_hi; a.vcen_lo = vk > 4 ? vc->centroids_lo : vc->centroids_hi;
   a.vbh = vc->bits_hi; a.vbl = vk > 4 ? vc->bits_lo : vc->bits_hi; a.vfrac = vk > 4;
   a.part = static_cast<float*>(workspace);
-  const bool bf = d->kv_dtype == TQ_BF16;
+  a.bf = d->kv_dtype == TQ_BF16;
   switch (kc->d) {
-    case 64: return launch_mfma_d64(a, kk, bf, s);
-    case 96: return launch_mfma_d96(a, kk, bf, s);
-    case 128: return launch_mfma_d128(a, kk, bf, s);
-    default: return launch_mfma_d256(a, kk, bf, s);
+    case 64: return launch_mfma_d64(a, kk, s);
+    case 96: return launch_mfma_d96(a, kk, s);
+    case 128: return launch_mfma_d128(a, kk, s);
+    default: return launch_mfma_d256(a, kk, s);
   }
 }
 

@@ -190,16 +190,17 @@ struct MfmaArgs {
   const float* kcen_hi; const float* kcen_lo;  // codebooks in device memory
   const float* vcen_hi; const float* vcen_lo;
   int vbh, vbl, vfrac;   // value widths; vfrac: fractional (split at D / 2)
+  int bf;                // bf16 sink / ring tokens (else fp16)
   float* part;           // (batch, hkv gsub, ncw + nfw, g, D + 4)
   int ncw, nfw;
   int tail;              // LDS offset past the tables / combine buffers (set by the launch)
 };
 // Partials and merge for head_dim 64 / 96 / 128 / 256; kk: the key width kind
-// (2-4, 5 = 2.5 bits, 7 = 3.5 bits), bf: bf16 sink / ring tokens.
-int launch_mfma_d64(const MfmaArgs& a, int kk, bool bf, hipStream_t s);
-int launch_mfma_d96(const MfmaArgs& a, int kk, bool bf, hipStream_t s);
-int launch_mfma_d128(const MfmaArgs& a, int kk, bool bf, hipStream_t s);
-int launch_mfma_d256(const MfmaArgs& a, int kk, bool bf, hipStream_t s);
+// (2-4, 5 = 2.5 bits, 7 = 3.5 bits).
+int launch_mfma_d64(const MfmaArgs& a, int kk, hipStream_t s);
+int launch_mfma_d96(const MfmaArgs& a, int kk, hipStream_t s);
+int launch_mfma_d128(const MfmaArgs& a, int kk, hipStream_t s);
+int launch_mfma_d256(const MfmaArgs& a, int kk, hipStream_t s);
 
 // Arguments of the dense (fp16 / bf16 K/V) decode-attention kernel: the
 // fp16 segments of tq_attn_desc, head_dim 128.

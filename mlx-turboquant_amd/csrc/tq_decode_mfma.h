@@ -35,13 +35,22 @@
 // Tables have 16 replicas per entry (128-byte rows): both sides of every width
 // pair fit 80 KB, against 2-way bank conflicts on some lookups.
 //
-// Bound: latency (set-up, the block loads' round trips, combine), as in the
-// uniform-batch kernels; one layer's codes are 2-9 MB, under 2 us of HBM time.
+// Bound: latency and VALU issue, not memory (one layer's codes are 2-9 MB,
+// under 2 us of HBM time): launch, the set-up's two barriers, the first block's
+// round trip, about 1,000 VALU instructions per block and wave at four cycles
+// each (two waves per SIMD), the combine. So the set-up shares its work: a
+// thread converts 8 query elements for all waves, one branch per type around
+// each loop (a per-element branch on the query's type alone cost 1,000-2,400
+// instructions per wave: 2.6 us per layer at head_dim 128), bf16 tokens go to
+// bf16 MFMAs as they are against three bf16 parts of the query and the weights
+// (scaling them into fp16 took 500 instructions per block), and the
+// accumulators are not rescaled before the first block.
 // Measured per layer in a graph of 16 layers, partials + merge against the
 // general kernel's three launches (float32 VALU dot products): bf16 K4/V4, 28
-// heads on 4, T 16,001: 20.4 us (kernels 12.8 + 6.7) from 101 us; head_dim 64,
-// bf16 K4/V2, 2 sequences, 32 heads on 8, T 8,229: 14.5 us from 56 us;
-// head_dim 256, bf16 K4/V3, 8 heads on 2, T 12,000: 35 us from 112 us.
+// heads on 4, T 16,001: 15.6 us (kernels 11.2 + 4.6) from 101 us; head_dim 64,
+// bf16 K4/V2, 2 sequences, 32 heads on 8, T 8,229: 13.1 us (10.2 + 4.0) from 56
+// us; head_dim 256, bf16 K4/V3, 8 heads on 2, T 12,000: 26.4 us (20.2 + 6.3)
+// from 112 us (its rotation reads 256 KB of R per workgroup).
 #pragma once
 
 #include <math.h>
@@ -65,12 +74,37 @@ using uk::rows_max;
 using uk::rows_sum;
 using uk::u2;
 using uk::u4;
-using uk::wave_max_u32;
 
 constexpr int MW = MFMA_WAVES;
 constexpr int MTH = MW * 64;   // threads
 constexpr float M_INIT = uk::M_INIT;
 constexpr int TROW = 128;      // bytes per table entry: 16 replicas
+// The tables hold CSC times the centroids, and queries are scaled up to QLOW <=
+// scale ||q||: the fp16 remainders of both stay normal (unscaled, a remainder of
+// 0.1 is a multiple of 6e-8).
+constexpr float CSC = 256.f;
+constexpr float QLOW = 4096.f;
+
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+__device__ inline f4 mfma_b(u4 a, u4 b, f4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, a), __builtin_bit_cast(bf8, b), c, 0, 0, 0);
+}
+
+// v = p[0] + p[1] + p[2], three bf16 parts of 8 values each (truncated: exact)
+__device__ inline void split_b(const float (&v)[8], u4 (&p)[3]) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    uint32_t a = __float_as_uint(v[2 * j]), b = __float_as_uint(v[2 * j + 1]);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      p[k][j] = __builtin_amdgcn_perm(b, a, 0x07060302u);  // the high halves
+      if (k < 2) {
+        a = __float_as_uint(__uint_as_float(a) - __uint_as_float(a & 0xFFFF0000u));
+        b = __float_as_uint(__uint_as_float(b) - __uint_as_float(b & 0xFFFF0000u));
+      }
+    }
+  }
+}
 
 // N bytes at any address into dwords (the compiler picks the load widths)
 template <int N>
@@ -118,8 +152,10 @@ struct Lds {
   static constexpr int QS = 2 * D + 16;               // bytes per (head, part) of the query operands
   static constexpr int CMS = D + 4;                   // floats per (wave, head) of the combine buffers
   static constexpr int cmb = MW * GC * CMS * 4;
-  static constexpr int qop = 0;                       // offsets past tail
-  static constexpr int cml = qop + GC * 2 * QS;
+  static constexpr int qsrc = 0;                      // offsets past tail: the query, 2 or 3 parts per head
+  static constexpr int qop = qsrc + GC * 3 * QS;      // the rotated query
+  static constexpr int qex = qop + GC * 2 * QS;       // 2^qe per head
+  static constexpr int cml = qex + GC * 4;
   static constexpr int nst = cml + MW * GC * 8;
   static constexpr int end = nst + MW * 256;
 };
@@ -131,7 +167,8 @@ struct Blk {
   float nk, nv;  // of token t0 + (lane & 31)
 };
 
-template <int D, int GC, int KK, bool BF>
+// VF: the values' width is fractional (two tables, rows of two widths)
+template <int D, int GC, int KK, bool VF>
 __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
   using G_ = KGeo<D, KK>;
   using L_ = Lds<D, GC>;
@@ -141,6 +178,10 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
   constexpr int TS = GC == 4 ? 2 : 1; // tiles sharing the columns
   constexpr int NS = 8 / TS;          // scores per lane per block
   constexpr int PSD = D + 4;
+  // the first uncompressed block's keys and values are requested before the
+  // query is converted; at D = 256 the registers do not hold both: each is
+  // requested where it is used
+  constexpr bool EARLY = D < 256;
   extern __shared__ __align__(16) uint8_t smem[];
   uint8_t* tail = smem + a.tail;
 
@@ -182,10 +223,11 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
   const float* vnorm = a.vn + (int64_t)row * a.vn_hs;
   // the value codes of MFMA row r: dims U r .. of the hi row (r < 8 or an
   // integer width) or of the lo row, read as dwords kept inside the row
-  const bool vlo = a.vfrac && r >= 8;
-  const int vb = vlo ? a.vbl : a.vbh;                        // width of this lane's dims
-  const int vrow = (a.vfrac ? D / 2 : D) * vb / 8;           // bytes per token
-  const uint8_t* vp = vlo ? a.vcl + (int64_t)row * a.vl_hs : a.vc + (int64_t)row * a.v_hs;
+  const bool vlo = VF && r >= 8;
+  const int vb = VF && vlo ? a.vbl : a.vbh;                  // width of this lane's dims
+  const int vrow = (VF ? D / 2 : D) * vb / 8;           // bytes per token
+  const uint8_t* vp = a.vc + (int64_t)row * a.v_hs;
+  if constexpr (VF) vp = vlo ? a.vcl + (int64_t)row * a.vl_hs : vp;
   int voff[VW], vsh[VW];
 #pragma unroll
   for (int i = 0; i < VW; ++i) {
@@ -220,79 +262,141 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
     B.nv = vnorm[tn];
   };
 
-  // ---- set-up: codebooks (one centroid per lane: key hi / lo, value hi / lo
-  // in the four 16-lane rows), the query rows, the first block
+  // ---- set-up: the query (8 elements per thread, LPH lanes per head) and the
+  // codebooks (one centroid per lane: key hi / lo, value hi / lo in the four
+  // 16-lane rows), then the first block
+  constexpr int LPH = D == 96 ? 16 : D / 8;
+  const int qh = tid / LPH, qi = tid % LPH;
+  const bool qact = qh < a.g && qi < D / 8;
+  u4 qw0 = {0u, 0u, 0u, 0u}, qw1 = {0u, 0u, 0u, 0u};
+  if (qact) {
+    const int64_t e = ((int64_t)b * a.hq + head0 + qh) * D + 8 * qi;
+    if (a.q_dtype == TQ_F32) {
+      qw0 = *reinterpret_cast<const u4*>(static_cast<const float*>(a.q) + e);
+      qw1 = *reinterpret_cast<const u4*>(static_cast<const float*>(a.q) + e + 4);
+    } else {
+      qw0 = *reinterpret_cast<const u4*>(static_cast<const uint16_t*>(a.q) + e);
+    }
+  }
   uint32_t cw = 0;
   Blk<D, KK> B0, B1;
+  // rows 16 jt + r of R (fp16 high part, remainder) as B operands of the query rotation
+  u4 rqh[G_::KS], rql[G_::KS];
+  auto load_rot = [&](int jt) {
+    const uint16_t* rh = a.rot16 + (16 * jt + r) * D + 8 * q4;
+#pragma unroll
+    for (int kb = 0; kb < G_::KS; ++kb) {
+      rqh[kb] = *reinterpret_cast<const u4*>(rh + 32 * kb);
+      rql[kb] = *reinterpret_cast<const u4*>(rh + D * D + 32 * kb);
+    }
+  };
   if (packed) {
     const float* bp = q4 == 0 ? a.kcen_hi : q4 == 1 ? a.kcen_lo : q4 == 2 ? a.vcen_hi : a.vcen_lo;
     const int nb = 1 << (q4 == 0 ? G_::bits(0) : q4 == 1 ? G_::bits(G_::NSEG - 1) : q4 == 2 ? a.vbh : a.vbl);
     const float x = bp[min(r, nb - 1)];
-    const _Float16 h = (_Float16)x, l = (_Float16)(x - (float)h);
+    if (w < U) load_rot(w);
+    load_blk(B0, min(blk0 + w, blk1 - 1));
+    const _Float16 h = (_Float16)(CSC * x), l = (_Float16)(CSC * x - (float)h);
     cw = (uint32_t)__builtin_bit_cast(uint16_t, h) | (uint32_t)__builtin_bit_cast(uint16_t, l) << 16;
   }
-  // q rows as MFMA A operands (row r = head min(r, g - 1), k-slots = dims 32 kb
-  // + 8 q4 ..): fp16 high part and remainder of q 2^-qe (query_exponent)
-  half8 qo_hi[G_::KS], qo_lo[G_::KS];
-  float qe_scale;
-  {
-    const int esz = a.q_dtype == TQ_F32 ? 4 : 2;
-    const uint8_t* qr = static_cast<const uint8_t*>(a.q) + ((int64_t)b * a.hq + head0 + min(r, a.g - 1)) * D * esz;
-    float x[G_::KS][8];
+  // uncompressed tokens: keys / values straight from memory
+  u4 kr[2][G_::KS];
+  uint32_t vr[8][U / 2];
+  const int rstart = clampi(a.res_start_b ? a.res_start_b[b] : a.res_start0, max(a.res_cap - 1, 0));
+  auto token = [&](int u, const void* sink_p, const void* res_p) {
+    u = min(u, nfp - 1);
+    int sl = rstart + (u - sink);
+    sl = sl >= a.res_cap ? sl - a.res_cap : sl;
+    return u < sink ? static_cast<const uint16_t*>(sink_p) + (int64_t)row * a.sink_hs + (int64_t)u * D
+                    : static_cast<const uint16_t*>(res_p) + (int64_t)row * a.res_hs + (int64_t)sl * D;
+  };
+  auto load_k = [&](int t0) {
 #pragma unroll
-    for (int kb = 0; kb < G_::KS; ++kb) {
-      const int d = 32 * kb + 8 * q4;
-      if (a.q_dtype == TQ_F32) {
-        const float4 u0 = *reinterpret_cast<const float4*>(qr + 4 * d);
-        const float4 u1 = *reinterpret_cast<const float4*>(qr + 4 * d + 16);
-        x[kb][0] = u0.x; x[kb][1] = u0.y; x[kb][2] = u0.z; x[kb][3] = u0.w;
-        x[kb][4] = u1.x; x[kb][5] = u1.y; x[kb][6] = u1.z; x[kb][7] = u1.w;
-      } else {
-        const u4 u = *reinterpret_cast<const u4*>(qr + 2 * d);
+    for (int t = 0; t < 2; ++t) {
+      const uint16_t* p = token(t0 + 16 * t + r, a.sink_k, a.res_k) + 8 * q4;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const uint32_t hb = (u[i >> 1] >> (16 * (i & 1))) & 0xFFFFu;
-          x[kb][i] = a.q_dtype == TQ_BF16 ? __uint_as_float(hb << 16) : (float)__builtin_bit_cast(_Float16, (uint16_t)hb);
-        }
-      }
+      for (int s = 0; s < G_::KS; ++s) kr[t][s] = *reinterpret_cast<const u4*>(p + 32 * s);
     }
-    if (packed) load_blk(B0, min(blk0 + w, blk1 - 1));
+  };
+  auto load_v = [&](int t0) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint16_t* p = token(t0 + (i < 4 ? 4 * q4 + i : 12 + 4 * q4 + i), a.sink_v, a.res_v) + U * r;
+      __builtin_memcpy(&vr[i][0], __builtin_assume_aligned(p, 4), 2 * U);
+    }
+  };
+  if constexpr (EARLY)
+    if (!packed) {
+      load_k((blk0 + w) << 5);
+      load_v((blk0 + w) << 5);
+    }
+
+  // q 2^-qe (query_exponent) in parts: fp16 high part and remainder, or for
+  // bf16 uncompressed tokens three bf16 parts
+  const bool bfp = !packed && a.bf;
+  if (w * 64 < a.g * LPH) {
+    float x[8];
+    if (a.q_dtype == TQ_F16) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = (float)as_h8(qw0)[i];
+    } else if (a.q_dtype == TQ_BF16) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = __uint_as_float(i & 1 ? qw0[i >> 1] & 0xFFFF0000u : qw0[i >> 1] << 16);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = __uint_as_float(i < 4 ? qw0[i] : qw1[i - 4]);
+    }
     float ss = 0.f;
 #pragma unroll
-    for (int kb = 0; kb < G_::KS; ++kb)
+    for (int i = 0; i < 8; ++i) ss = fmaf(x[i], x[i], ss);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) ss = fmaf(x[kb][i], x[kb][i], ss);
-    ss = rows_sum(ss);  // the 4 lanes of row r hold the dims of its head
-    const int qe = query_exponent(sqrtf(ss), a.qscale, uk::Q_LIMIT, uk::Q_LOW);
+    for (int k = 1; k < LPH; k *= 2) ss += __shfl_xor(ss, k);
+    const int qe = query_exponent(sqrtf(ss), a.qscale, uk::Q_LIMIT, QLOW);
     const float qdown = __builtin_amdgcn_ldexpf(1.f, -qe);
+    if (qact) {
+      uint8_t* d = tail + L_::qsrc + qh * 3 * L_::QS + 16 * qi;
 #pragma unroll
-    for (int kb = 0; kb < G_::KS; ++kb)
+      for (int i = 0; i < 8; ++i) x[i] *= qdown;
+      if (bfp) {
+        u4 p[3];
+        split_b(x, p);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float xs = x[kb][i] * qdown;
-        qo_hi[kb][i] = (_Float16)xs;
-        qo_lo[kb][i] = (_Float16)(xs - (float)qo_hi[kb][i]);
+        for (int k = 0; k < 3; ++k) *reinterpret_cast<u4*>(d + k * L_::QS) = p[k];
+      } else {
+        half8 hi, lo;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          hi[i] = (_Float16)x[i];
+          lo[i] = (_Float16)(x[i] - (float)hi[i]);
+        }
+        *reinterpret_cast<half8*>(d) = hi;
+        *reinterpret_cast<half8*>(d + L_::QS) = lo;
       }
-    qe_scale = __builtin_amdgcn_ldexpf(1.f, __builtin_amdgcn_ds_bpermute(4 * hd, qe));  // lane h: head h
+      if (qi == 0) *reinterpret_cast<float*>(tail + L_::qex + 4 * qh) = __builtin_amdgcn_ldexpf(1.f, qe);
+    }
   }
+  if (packed) {
+    build_table(smem, 0, G_::bits(0), cw, tid);
+    if constexpr (G_::FR) build_table(smem + G_::tab(1), 1, G_::bits(1), cw, tid);
+    build_table(smem + G_::TABS, 2, a.vbh, cw, tid);
+    if constexpr (VF) build_table(smem + G_::TABS + (1 << (2 * a.vbh)) * TROW, 3, a.vbl, cw, tid);
+  }
+  __syncthreads();
+  const float qe_scale = *reinterpret_cast<const float*>(tail + L_::qex + 4 * hd);
   uint8_t* qop = tail + L_::qop;
   if (packed) {
     // rotated query, D[h][n] = sum_i q[h][i] R[j0 + n][i], written (times
     // qscale) as fp16 high part / remainder rows [head][part][D]
+    const uint8_t* qs = tail + L_::qsrc + min(r, a.g - 1) * 3 * L_::QS + 16 * q4;
     for (int jt = w; jt < U; jt += MW) {
-      const uint16_t* rh = a.rot16 + (16 * jt + r) * D + 8 * q4;
-      u4 rqh[G_::KS], rql[G_::KS];
-#pragma unroll
-      for (int kb = 0; kb < G_::KS; ++kb) {
-        rqh[kb] = *reinterpret_cast<const u4*>(rh + 32 * kb);
-        rql[kb] = *reinterpret_cast<const u4*>(rh + D * D + 32 * kb);
-      }
+      if (jt != w) load_rot(jt);
       f4 dq = {0.f, 0.f, 0.f, 0.f}, dl = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int kb = 0; kb < G_::KS; ++kb) {
-        dq = mfma(qo_hi[kb], as_h8(rqh[kb]), dq);
-        dl = mfma(qo_hi[kb], as_h8(rql[kb]), dl);
-        dl = mfma(qo_lo[kb], as_h8(rqh[kb]), dl);
+        const half8 qhi = *reinterpret_cast<const half8*>(qs + 64 * kb);
+        dq = mfma(qhi, as_h8(rqh[kb]), dq);
+        dl = mfma(qhi, as_h8(rql[kb]), dl);
+        dl = mfma(*reinterpret_cast<const half8*>(qs + L_::QS + 64 * kb), as_h8(rqh[kb]), dl);
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -306,30 +410,20 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
         }
       }
     }
-    build_table(smem, 0, G_::bits(0), cw, tid);
-    if constexpr (G_::FR) build_table(smem + G_::tab(1), 1, G_::bits(1), cw, tid);
-    build_table(smem + G_::TABS, 2, a.vbh, cw, tid);
-    if (a.vfrac) build_table(smem + G_::TABS + (1 << (2 * a.vbh)) * TROW, 3, a.vbl, cw, tid);
-  } else if (w == 0 && r < a.g && r < GC) {
-    // uncompressed tokens: the query in original space
-#pragma unroll
-    for (int kb = 0; kb < G_::KS; ++kb) {
-      uint8_t* d = qop + (r * 2) * L_::QS + 2 * (32 * kb + 8 * q4);
-      *reinterpret_cast<half8*>(d) = qo_hi[kb];
-      *reinterpret_cast<half8*>(d + L_::QS) = qo_lo[kb];
-    }
+    __syncthreads();
   }
-  __syncthreads();
 
   // B operands of the scores: step (seg, s) k-slot (q4, e) is dim seg SD +
-  // q4 SD / 4 + 8 s + e (original space: one segment)
+  // q4 SD / 4 + 8 s + e (uncompressed tokens: 32 s + 8 q4 + e, so that one load
+  // covers 64 contiguous bytes of each of 16 rows; the order above would fetch
+  // every 128-byte line once per step)
   half8 qb[G_::KS];
   {
-    const uint8_t* src = qop + (hd * 2 + (lo_part ? 1 : 0)) * L_::QS;
+    const uint8_t* src = packed ? qop + (hd * 2 + (lo_part ? 1 : 0)) * L_::QS
+                                : tail + L_::qsrc + (hd * 3 + (lo_part ? 1 : 0)) * L_::QS;
 #pragma unroll
     for (int s = 0; s < G_::KS; ++s) {
-      const int seg = packed ? s / G_::SST : 0;
-      const int d = packed ? seg * G_::SD + q4 * (G_::SD / 4) + 8 * (s % G_::SST) : q4 * (D / 4) + 8 * s;
+      const int d = packed ? s / G_::SST * G_::SD + q4 * (G_::SD / 4) + 8 * (s % G_::SST) : 32 * s + 8 * q4;
       qb[s] = *reinterpret_cast<const half8*>(src + 2 * d);
     }
   }
@@ -342,51 +436,34 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
 #pragma unroll
   for (int nb = 0; nb < U; ++nb) acc[nb] = f4{0.f, 0.f, 0.f, 0.f};
 
-  auto softmax_pv = [&](float (&s)[NS], const float (&nv)[NS]) {
+  bool any = false;   // the wave has accumulated a block
+  // running max and sum over the block's scores s, weights times nv to pv; the
+  // accumulators follow a raised max (nothing to follow in the first block)
+  auto softmax = [&](const float (&s)[NS], const float (&nv)[NS], float (&pv)[NS]) {
     float bm = s[0];
 #pragma unroll
     for (int i = 1; i < NS; ++i) bm = fmaxf(bm, s[i]);
     bm = rows_max(bm);
     if (__builtin_amdgcn_ballot_w64(bm > m_run) != 0) {
       const float mnew = bm > m_run ? bm + uk::RESCALE_MARGIN : m_run;
-      const float corr = fexp2(m_run - mnew);
-      l_run *= corr;
+      if (any) {
+        const float corr = fexp2(m_run - mnew);
+        l_run *= corr;
 #pragma unroll
-      for (int nb = 0; nb < U; ++nb) acc[nb] *= corr;
+        for (int nb = 0; nb < U; ++nb) acc[nb] *= corr;
+      }
       m_run = mnew;
     }
-    float pv[NS];
-    float pm = 0.f;
+    any = true;
 #pragma unroll
     for (int i = 0; i < NS; ++i) {
       const float p = fexp2(s[i] - m_run);
       l_run += p;
       pv[i] = p * nv[i];
-      pm = fmaxf(pm, fabsf(pv[i]));
     }
-    const float pmx = pm * __builtin_amdgcn_ldexpf(1.f, -vx);
-    if (__builtin_amdgcn_ballot_w64(pmx > uk::PV_LIMIT || (!vset && pmx > 0.f)) != 0) {
-      const float cm = rows_max(pmx);  // max of the column
-      int dx;
-      if (!vset) {
-        dx = cm > 0.f ? max((int)ceilf(log2f(cm / uk::PV_SET)), -110) : 0;
-        vset = true;
-      } else {
-        dx = cm > uk::PV_LIMIT ? (int)ceilf(log2f(cm / uk::PV_LIMIT)) : 0;
-      }
-      const float f = __builtin_amdgcn_ldexpf(1.f, -dx);
-#pragma unroll
-      for (int nb = 0; nb < U; ++nb) acc[nb] *= f;
-      vx += dx;
-    }
-    const float down = __builtin_amdgcn_ldexpf(1.f, -vx);
-    uint32_t d[NS / 2];
-#pragma unroll
-    for (int j = 0; j < NS / 2; ++j) {
-      const float p0 = pv[2 * j] * down, p1 = pv[2 * j + 1] * down;
-      const hx2 h = __builtin_amdgcn_cvt_pkrtz(p0, p1);
-      d[j] = pk_rtz(fmaf(-partf, (float)h[0], p0), fmaf(-partf, (float)h[1], p1));
-    }
+  };
+  // the two tiles' k-slots of the P^T operand from the lane's packed pairs
+  auto slots = [&](const uint32_t (&d)[NS / 2]) {
     u4 pb;
     if constexpr (TS == 2) {
       pb[0] = tile ? 0u : d[0];
@@ -397,7 +474,37 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) pb[j] = d[j];
     }
-    return as_h8(pb);
+    return pb;
+  };
+  // P^T in fp16: high part or remainder by column, times 2^-vx; vx is set by
+  // the wave's first nonzero weight (the accumulators are zero until then)
+  auto weights_h = [&](const float (&pv)[NS]) {
+    float pm = 0.f;
+#pragma unroll
+    for (int i = 0; i < NS; ++i) pm = fmaxf(pm, fabsf(pv[i]));
+    const float pmx = pm * __builtin_amdgcn_ldexpf(1.f, -vx);
+    if (__builtin_amdgcn_ballot_w64(pmx > uk::PV_LIMIT || (!vset && pmx > 0.f)) != 0) {
+      const float cm = rows_max(pmx);  // max of the column
+      if (!vset) {
+        vx = cm > 0.f ? max((int)ceilf(log2f(cm / uk::PV_SET)), -110) : 0;
+        vset = true;
+      } else {
+        const int dx = cm > uk::PV_LIMIT ? (int)ceilf(log2f(cm / uk::PV_LIMIT)) : 0;
+        const float f = __builtin_amdgcn_ldexpf(1.f, -dx);
+#pragma unroll
+        for (int nb = 0; nb < U; ++nb) acc[nb] *= f;
+        vx += dx;
+      }
+    }
+    const float down = __builtin_amdgcn_ldexpf(1.f, -vx);
+    uint32_t d[NS / 2];
+#pragma unroll
+    for (int j = 0; j < NS / 2; ++j) {
+      const float p0 = pv[2 * j] * down, p1 = pv[2 * j + 1] * down;
+      const hx2 h = __builtin_amdgcn_cvt_pkrtz(p0, p1);
+      d[j] = pk_rtz(fmaf(-partf, (float)h[0], p0), fmaf(-partf, (float)h[1], p1));
+    }
+    return slots(d);
   };
   // the scores of this lane from the two tiles' MFMA results, times `f` per
   // token; masked past `end` tokens
@@ -423,6 +530,7 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
     const uint32_t cp = (uint32_t)r * 8;  // replica of this lane
     const uint32_t cpv = cp + G_::TABS + (vlo ? (1u << (2 * a.vbh)) * TROW : 0u);
     const uint32_t vbw = 2 * vb;  // bits per field
+    const float ks = qe_scale * (1.f / CSC);
     float* nst = reinterpret_cast<float*>(tail + L_::nst) + w * 64;  // [key norms 32][value norms 32]
     auto lut = [&](uint32_t addr) { return *reinterpret_cast<const u2*>(smem + addr); };
     auto compute = [&](const Blk<D, KK>& B, int blk) {
@@ -433,8 +541,7 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
       for (int t = 0; t < 2 / TS; ++t) {
         const float4 k4 = *reinterpret_cast<const float4*>(nst + 16 * (t + tile) + 4 * q4);
         const float4 v4 = *reinterpret_cast<const float4*>(nst + 32 + 16 * (t + tile) + 4 * q4);
-        nk[4 * t] = k4.x * qe_scale; nk[4 * t + 1] = k4.y * qe_scale;
-        nk[4 * t + 2] = k4.z * qe_scale; nk[4 * t + 3] = k4.w * qe_scale;
+        nk[4 * t] = k4.x * ks; nk[4 * t + 1] = k4.y * ks; nk[4 * t + 2] = k4.z * ks; nk[4 * t + 3] = k4.w * ks;
         nv[4 * t] = v4.x; nv[4 * t + 1] = v4.y; nv[4 * t + 2] = v4.z; nv[4 * t + 3] = v4.w;
       }
       f4 sc2[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
@@ -460,7 +567,9 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
       }
       float sc[NS];
       lane_scores(sc, sc2[0], sc2[1], nk, t0, comp);
-      const half8 pb = softmax_pv(sc, nv);
+      float pv[NS];
+      softmax(sc, nv, pv);
+      const half8 pb = as_h8(weights_h(pv));
 #pragma unroll
       for (int f = 0; f < NF; ++f) {
         // dims U r + 2 f, + 1 of the block's 4 token pairs
@@ -496,87 +605,72 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
       }
     }
   } else {
-    // uncompressed tokens: keys / values straight from memory
-    const int rstart = clampi(a.res_start_b ? a.res_start_b[b] : a.res_start0, max(a.res_cap - 1, 0));
-    const uint16_t* sk = static_cast<const uint16_t*>(a.sink_k) + (int64_t)row * a.sink_hs;
-    const uint16_t* sv = static_cast<const uint16_t*>(a.sink_v) + (int64_t)row * a.sink_hs;
-    const uint16_t* rk = static_cast<const uint16_t*>(a.res_k) + (int64_t)row * a.res_hs;
-    const uint16_t* rv = static_cast<const uint16_t*>(a.res_v) + (int64_t)row * a.res_hs;
-    auto token = [&](int u, const uint16_t* s0, const uint16_t* r0) {
-      u = min(u, nfp - 1);
-      int sl = rstart + (u - sink);
-      sl = sl >= a.res_cap ? sl - a.res_cap : sl;
-      return u < sink ? s0 + (int64_t)u * D : r0 + (int64_t)sl * D;
-    };
     for (int blk = blk0 + w; blk < blk1; blk += MW) {
       const int t0 = blk << 5;
-      u4 kr[2][G_::KS];
-      uint32_t vr[8][U / 2];
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const uint16_t* p = token(t0 + 16 * t + r, sk, rk) + q4 * (D / 4);
-#pragma unroll
-        for (int s = 0; s < G_::KS; ++s) kr[t][s] = *reinterpret_cast<const u4*>(p + 8 * s);
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const uint16_t* p = token(t0 + (i < 4 ? 4 * q4 + i : 12 + 4 * q4 + i), sv, rv) + U * r;
-        __builtin_memcpy(&vr[i][0], __builtin_assume_aligned(p, 4), 2 * U);
-      }
-      // bf16: keys and values of the block scaled by powers of two that bring
-      // the largest |x| of each into [2^14, 2^15): exact in fp16 down to 2^-38
-      // of it; the scores and the weights are scaled back
-      float kback = 1.f, vback = 1.f;
-      if constexpr (BF) {
-        uint32_t mk = 0, mv = 0;
-        auto up = [](uint32_t& m, uint32_t x) {
-          x &= 0x7FFF7FFFu;
-          m = max(m, max(x & 0xFFFFu, x >> 16));
-        };
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-          for (int s = 0; s < G_::KS; ++s)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) up(mk, kr[t][s][i]);
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-#pragma unroll
-          for (int j = 0; j < U / 2; ++j) up(mv, vr[i][j]);
-        mk = wave_max_u32(mk);
-        mv = wave_max_u32(mv);
-        const int ek = mk == 0u ? 0 : max(-100, (int)(mk >> 7) - 127 - 14);
-        const int ev = mv == 0u ? 0 : max(-100, (int)(mv >> 7) - 127 - 14);
-        const float ks = __builtin_amdgcn_ldexpf(1.f, -ek), vs = __builtin_amdgcn_ldexpf(1.f, -ev);
-        kback = __builtin_amdgcn_ldexpf(1.f, ek);
-        vback = __builtin_amdgcn_ldexpf(1.f, ev);
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-          for (int s = 0; s < G_::KS; ++s) kr[t][s] = uk::bf16_to_f16(kr[t][s], ks);
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-#pragma unroll
-          for (int j = 0; j < U / 2; ++j)
-            vr[i][j] = pk_rtz(__uint_as_float(vr[i][j] << 16) * vs, __uint_as_float(vr[i][j] & 0xFFFF0000u) * vs);
+      if (!EARLY || blk != blk0 + w) {
+        load_k(t0);
+        if constexpr (EARLY) load_v(t0);
       }
       f4 sc2[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+      float sc[NS], kf[NS], nv[NS], pv[NS];
 #pragma unroll
-      for (int s = 0; s < G_::KS; ++s)
+      for (int i = 0; i < NS; ++i) kf[i] = a.qscale * qe_scale, nv[i] = 1.f;
+      if (a.bf) {
+        // bf16 tokens on bf16 MFMAs: the third part of the query (and of the
+        // weights) in an operand of its own, in the first part's columns
+        const uint8_t* src = tail + L_::qsrc + (hd * 3 + 2) * L_::QS + 16 * q4;
 #pragma unroll
-        for (int t = 0; t < 2; ++t) sc2[t] = mfma(as_h8(kr[t][s]), qb[s], sc2[t]);
-      float sc[NS], kf[NS], nv[NS];
+        for (int s = 0; s < G_::KS; ++s) {
+          const u4 x = *reinterpret_cast<const u4*>(src + 64 * s);
+          const u4 q3 = u4{lo_part ? 0u : x[0], lo_part ? 0u : x[1], lo_part ? 0u : x[2], lo_part ? 0u : x[3]};
 #pragma unroll
-      for (int i = 0; i < NS; ++i) kf[i] = a.qscale * qe_scale * kback, nv[i] = vback;
+          for (int t = 0; t < 2; ++t) {
+            sc2[t] = mfma_b(kr[t][s], __builtin_bit_cast(u4, qb[s]), sc2[t]);
+            sc2[t] = mfma_b(kr[t][s], q3, sc2[t]);
+          }
+        }
+      } else {
+#pragma unroll
+        for (int s = 0; s < G_::KS; ++s)
+#pragma unroll
+          for (int t = 0; t < 2; ++t) sc2[t] = mfma(as_h8(kr[t][s]), qb[s], sc2[t]);
+      }
+      if constexpr (!EARLY) load_v(t0);
       lane_scores(sc, sc2[0], sc2[1], kf, t0, nfp);
-      const half8 pb = softmax_pv(sc, nv);
+      softmax(sc, nv, pv);
+      u4 pb, p3 = {0u, 0u, 0u, 0u};
+      if (a.bf) {
+        uint32_t d[NS / 2], d3[NS / 2];
+#pragma unroll
+        for (int j = 0; j < NS / 2; ++j) {
+          uint32_t x[2], y[2];
+#pragma unroll
+          for (int k = 0; k < 2; ++k) {
+            const uint32_t p = __float_as_uint(pv[2 * j + k]);
+            const uint32_t p2 = __float_as_uint(__uint_as_float(p) - __uint_as_float(p & 0xFFFF0000u));
+            x[k] = lo_part ? p2 : p;
+            y[k] = lo_part ? 0u : __float_as_uint(__uint_as_float(p2) - __uint_as_float(p2 & 0xFFFF0000u));
+          }
+          d[j] = __builtin_amdgcn_perm(x[1], x[0], 0x07060302u);
+          d3[j] = __builtin_amdgcn_perm(y[1], y[0], 0x07060302u);
+        }
+        pb = slots(d);
+        p3 = slots(d3);
+      } else {
+        pb = weights_h(pv);
+      }
 #pragma unroll
       for (int nb = 0; nb < U; ++nb) {
         const uint32_t sel = (nb & 1) ? 0x07060302u : 0x05040100u;
         u4 va;
 #pragma unroll
         for (int j = 0; j < 4; ++j) va[j] = __builtin_amdgcn_perm(vr[2 * j + 1][nb >> 1], vr[2 * j][nb >> 1], sel);
-        acc[nb] = mfma(as_h8(va), pb, acc[nb]);
+        if (a.bf) {
+          acc[nb] = mfma_b(va, pb, acc[nb]);
+          acc[nb] = mfma_b(va, p3, acc[nb]);
+        } else {
+          acc[nb] = mfma(as_h8(va), as_h8(pb), acc[nb]);
+        }
       }
     }
   }
@@ -584,7 +678,7 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
   // ---- combine the waves through LDS (the table region); the two fp16 parts
   // of a head meet through `partner`, for GC = 4 the two tiles at their common max
   l_run = rows_sum(l_run);
-  float tsc = __builtin_amdgcn_ldexpf(1.f, vx);
+  float tsc = __builtin_amdgcn_ldexpf(packed ? 1.f / CSC : 1.f, vx);
   if constexpr (TS == 2) {
     const float m2 = fmaxf(m_run, row_ror<8>(m_run));
     const float t = fexp2(m_run - m2);
@@ -634,58 +728,62 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
 
 // Merge of the np = ncw + nfw partials of a query head: with w_p = 2^(M_p - M)
 // L_p / L, out = (sum_{p < ncw} w_p y_p) R + sum_{p >= ncw} w_p x_p (x = R^T y,
-// R the value codec's float32 rotation). Grid (hq, batch), NT threads: PG
-// groups of D threads sum the partials p = group + PG k; for the rotation
-// thread (4 columns, row block) takes D / RB rows of R, requested before the
-// partials are waited for.
+// R the value codec's float32 rotation). Grid (hq, batch): a chain of dependent
+// round trips, so everything is requested at once: PG groups of D threads hold
+// MB partials each (64 of them in one round at D <= 128), every wave reads all
+// headers, and thread (4 columns, row block) its D / RB rows of R.
 template <int D>
 struct MergeGeo {
-  static constexpr int NT = D == 256 ? 1024 : 256;
-  static constexpr int PG = NT / D;             // partial groups (4 / 2 / 2 / 4)
+  static constexpr int PG = D == 256 ? 4 : 8;   // partial groups
+  static constexpr int NT = PG * D;             // threads
+  static constexpr int MB = D == 256 ? 16 : 8;  // partials per group and round
   static constexpr int CT = D / 4;              // column threads of a row block
-  static constexpr int RB = D == 96 ? 8 : NT / CT;  // row blocks
+  static constexpr int RB = NT / CT;            // row blocks (32; 16 at D = 256)
   static constexpr int RR = D / RB;             // rows per block
 };
 
 template <int D>
 __global__ __launch_bounds__(MergeGeo<D>::NT) void mfma_merge_kernel(MfmaArgs a, int np) {
   using M_ = MergeGeo<D>;
-  constexpr int PSD = D + 4, MB = 8;
+  constexpr int PSD = D + 4, MB = M_::MB, PG = M_::PG;
   extern __shared__ __align__(16) uint8_t smem[];
-  float* wsh = reinterpret_cast<float*>(smem);  // [np rounded to 64] weights, then
-  __shared__ float ys[M_::PG][D], xs[M_::PG][D];
+  float* wsh = reinterpret_cast<float*>(smem);  // [np rounded up to whole rounds] weights
+  __shared__ float ys[PG][D], xs[PG][D], yt[D];
   __shared__ __align__(16) float red[M_::RB][D];
   const int hq = blockIdx.x, b = blockIdx.y;
-  const int gq = a.hq / a.hkv / a.gsub;  // == a.g
-  const int gy = hq / gq, h = hq % gq;
+  const int gy = hq / a.g, h = hq % a.g;
   const int tid = threadIdx.x, lane = tid & 63;
   const int64_t pst = (int64_t)a.g * PSD;
   const float* pp = a.part + (int64_t)(b * a.hkv * a.gsub + gy) * np * pst + h * PSD;
   const int d = tid % D, grp = tid / D;
-  const bool act = grp < M_::PG;
+  float2 hd[4];  // headers lane + 64 k (past 256: the loops below)
+#pragma unroll
+  for (int k = 0; k < 4; ++k) hd[k] = *reinterpret_cast<const float2*>(pp + min(lane + 64 * k, np - 1) * pst);
   float x[MB];
   auto load = [&](int p0) {
 #pragma unroll
-    for (int i = 0; i < MB; ++i) x[i] = pp[min(p0 + M_::PG * i + grp, np - 1) * pst + 4 + d];
+    for (int i = 0; i < MB; ++i) x[i] = pp[min(p0 + PG * i + grp, np - 1) * pst + 4 + d];
   };
-  // every wave reads all headers for the max and the sum; wave 0 keeps the weights
-  float M = M_INIT;
-  for (int p = lane; p < np; p += 64) {
-    const float2 hd = *reinterpret_cast<const float2*>(pp + p * pst);
-    M = hd.y > 0.f ? fmaxf(M, hd.x) : M;
-  }
   load(0);
   const int j4 = 4 * (tid % M_::CT), ib = tid / M_::CT;
   float4 rr[M_::RR];
-  if (ib < M_::RB) {
 #pragma unroll
-    for (int k = 0; k < M_::RR; ++k) rr[k] = *reinterpret_cast<const float4*>(a.vrot + (M_::RR * ib + k) * D + j4);
+  for (int k = 0; k < M_::RR; ++k) rr[k] = *reinterpret_cast<const float4*>(a.vrot + (M_::RR * ib + k) * D + j4);
+
+  float M = M_INIT;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) M = hd[k].y > 0.f ? fmaxf(M, hd[k].x) : M;  // (repeats of the last header change nothing)
+  for (int p = 256 + lane; p < np; p += 64) {
+    const float2 e = *reinterpret_cast<const float2*>(pp + p * pst);
+    M = e.y > 0.f ? fmaxf(M, e.x) : M;
   }
   M = uk::wave_max(M);
   float ls = 0.f;
-  for (int p = lane; p < np; p += 64) {
-    const float2 hd = *reinterpret_cast<const float2*>(pp + p * pst);
-    const float wp = hd.y > 0.f ? fexp2(hd.x - M) * hd.y : 0.f;
+  const int npr = (np + PG * MB - 1) / (PG * MB) * (PG * MB);
+  for (int p = lane, k = 0; p < npr; p += 64, ++k) {
+    float2 e = k == 0 ? hd[0] : k == 1 ? hd[1] : k == 2 ? hd[2] : hd[3];
+    if (k >= 4 && p < np) e = *reinterpret_cast<const float2*>(pp + p * pst);
+    const float wp = p < np && e.y > 0.f ? fexp2(e.x - M) * e.y : 0.f;
     if (tid < 64) wsh[p] = wp;
     ls += wp;
   }
@@ -696,28 +794,31 @@ __global__ __launch_bounds__(MergeGeo<D>::NT) void mfma_merge_kernel(MfmaArgs a,
   for (int p0 = 0;;) {
 #pragma unroll
     for (int i = 0; i < MB; ++i) {
-      const int p = p0 + M_::PG * i + grp;
-      const float wp = act && p < np ? wsh[p] : 0.f;
+      const int p = p0 + PG * i + grp;
+      const float wp = wsh[p];
       const float v = wp != 0.f ? x[i] : 0.f;  // (empty partials may hold anything)
       acc = fmaf(p < a.ncw ? wp : 0.f, v, acc);
       acco = fmaf(p < a.ncw ? 0.f : wp, v, acco);
     }
-    p0 += M_::PG * MB;
+    p0 += PG * MB;
     if (p0 >= np) break;
     load(p0);
   }
-  if (act) {
-    ys[grp][d] = acc;
-    xs[grp][d] = acco;
+  ys[grp][d] = acc;
+  xs[grp][d] = acco;
+  __syncthreads();
+  if (tid < D) {
+    float y = 0.f;
+#pragma unroll
+    for (int q = 0; q < PG; ++q) y += ys[q][tid];
+    yt[tid] = y;
   }
   __syncthreads();
-  if (ib < M_::RB) {
+  {
     float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
     for (int k = 0; k < M_::RR; ++k) {
-      float y = 0.f;
-#pragma unroll
-      for (int q = 0; q < M_::PG; ++q) y += ys[q][M_::RR * ib + k];
+      const float y = yt[M_::RR * ib + k];
       o.x = fmaf(y, rr[k].x, o.x);
       o.y = fmaf(y, rr[k].y, o.y);
       o.z = fmaf(y, rr[k].z, o.z);
@@ -731,51 +832,52 @@ __global__ __launch_bounds__(MergeGeo<D>::NT) void mfma_merge_kernel(MfmaArgs a,
 #pragma unroll
     for (int k = 0; k < M_::RB; ++k) s += red[k][tid];
 #pragma unroll
-    for (int q = 0; q < M_::PG; ++q) s += xs[q][tid];
+    for (int q = 0; q < PG; ++q) s += xs[q][tid];
     a.out[((int64_t)b * a.hq + hq) * D + tid] = s * inv;
   }
 }
 
 template <int D, int GC, int KK>
-static void launch_k(const MfmaArgs& a, bool bf, hipStream_t s) {
+static void launch_k(const MfmaArgs& a, hipStream_t s) {
   using G_ = KGeo<D, KK>;
   MfmaArgs x = a;
   const int vt = (1 << (2 * a.vbh)) * TROW + (a.vfrac ? (1 << (2 * a.vbl)) * TROW : 0);
   x.tail = G_::TABS + vt > Lds<D, GC>::cmb ? G_::TABS + vt : Lds<D, GC>::cmb;
   const int lds = x.tail + Lds<D, GC>::end;
   const dim3 grid(a.ncw + a.nfw, a.hkv * a.gsub, a.batch);
-  if (bf)
+  if (a.vfrac)
     hipLaunchKernelGGL((mfma_decode_kernel<D, GC, KK, true>), grid, dim3(MTH), lds, s, x);
   else
     hipLaunchKernelGGL((mfma_decode_kernel<D, GC, KK, false>), grid, dim3(MTH), lds, s, x);
 }
 
 template <int D, int KK>
-static void launch_g(const MfmaArgs& a, bool bf, hipStream_t s) {
+static void launch_g(const MfmaArgs& a, hipStream_t s) {
   if (a.g <= 4)
-    launch_k<D, 4, KK>(a, bf, s);
+    launch_k<D, 4, KK>(a, s);
   else
-    launch_k<D, 8, KK>(a, bf, s);
+    launch_k<D, 8, KK>(a, s);
 }
 
 // kk: key width kind (KGeo)
 template <int D>
-int launch_mfma(const MfmaArgs& a, int kk, bool bf, hipStream_t s) {
+int launch_mfma(const MfmaArgs& a, int kk, hipStream_t s) {
   switch (kk) {
-    case 2: launch_g<D, 2>(a, bf, s); break;
-    case 3: launch_g<D, 3>(a, bf, s); break;
-    case 4: launch_g<D, 4>(a, bf, s); break;
+    case 2: launch_g<D, 2>(a, s); break;
+    case 3: launch_g<D, 3>(a, s); break;
+    case 4: launch_g<D, 4>(a, s); break;
     case 5:
-      if constexpr (D != 96) launch_g<D, 5>(a, bf, s);
+      if constexpr (D != 96) launch_g<D, 5>(a, s);
       break;
     case 7:
-      if constexpr (D != 96) launch_g<D, 7>(a, bf, s);
+      if constexpr (D != 96) launch_g<D, 7>(a, s);
       break;
     default: return -1;
   }
   const int np = a.ncw + a.nfw;
-  hipLaunchKernelGGL((mfma_merge_kernel<D>), dim3(a.hq, a.batch), dim3(MergeGeo<D>::NT), ((np + 63) & ~63) * 4, s, a,
-                     np);
+  constexpr int round = MergeGeo<D>::PG * MergeGeo<D>::MB;
+  hipLaunchKernelGGL((mfma_merge_kernel<D>), dim3(a.hq, a.batch), dim3(MergeGeo<D>::NT),
+                     (np + round - 1) / round * round * 4, s, a, np);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
