@@ -2091,7 +2091,7 @@ int tq_debug_decode_route(const tq_codec* kc, const tq_codec* vc, const tq_attn_
 // Test hook, not part of the ABI: the grid of the uniform-batch kernels for a
 // call, without launching anything: out[0..3] = workgroups per (sequence, kv
 // head), compressed 32-token blocks per workgroup, fp16 tokens per workgroup
-// and the blocks-per-wave instantiation (4 or 8) the launch selects. Returns
+// and the blocks-per-wave instantiation the launch selects. Returns
 // -1 when the uniform-batch grid does not take the call.
 int tq_debug_uniform_geometry(const tq_codec* kc, const tq_codec* vc, const tq_attn_desc* d, int32_t* out) {
   if (!kc || !vc || !d || !out || d->hkv <= 0 || d->hq % d->hkv) return -1;
@@ -2100,7 +2100,7 @@ int tq_debug_uniform_geometry(const tq_codec* kc, const tq_codec* vc, const tq_a
   out[0] = nwg;
   out[1] = bpw;
   out[2] = fpw;
-  out[3] = bpw > FAST_WAVES * 4 ? 8 : 4;  // the selection of launch_u / launch_w
+  out[3] = uniform_npw(bpw);
   return 0;
 }
 

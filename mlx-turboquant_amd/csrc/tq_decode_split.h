@@ -233,7 +233,7 @@ __global__ __launch_bounds__(FT) void split_decode_kernel(UniformArgs a) {
   *reinterpret_cast<u4*>(smem + Layout::f16s + (tid >> 5) * (2 * FROW) + ((tid >> 4) & 1) * FROW + 16 * (tid & 15)) = fst;
   __syncthreads();
 
-  load_slot(1);
+  if constexpr (NPW > 1) load_slot(1);
 
   // q rows as MFMA A operands, scaled by 2^-qe per head (as in the uniform
   // kernel)
@@ -266,22 +266,25 @@ __global__ __launch_bounds__(FT) void split_decode_kernel(UniformArgs a) {
       }
     }
     if (!q_exact) {
-      float x[4][8];
+      float x[4][8];  // (one branch on the type around each loop: inside, there is one per element)
+      if (a.q_dtype == TQ_F32) {
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
-        const int d = 32 * kb + 8 * q4;
-        if (a.q_dtype == TQ_F32) {
-          const float4 u0 = *reinterpret_cast<const float4*>(qr + 4 * d);
-          const float4 u1 = *reinterpret_cast<const float4*>(qr + 4 * d + 16);
-          x[kb][0] = u0.x; x[kb][1] = u0.y; x[kb][2] = u0.z; x[kb][3] = u0.w;
-          x[kb][4] = u1.x; x[kb][5] = u1.y; x[kb][6] = u1.z; x[kb][7] = u1.w;
-        } else {
-          const u4 u = *reinterpret_cast<const u4*>(qr + 2 * d);
+        for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const uint32_t hb = (u[i >> 1] >> (16 * (i & 1))) & 0xFFFFu;
-            x[kb][i] = a.q_dtype == TQ_BF16 ? __uint_as_float(hb << 16) : (float)__builtin_bit_cast(_Float16, (uint16_t)hb);
-          }
+          for (int i = 0; i < 8; ++i) x[kb][i] = reinterpret_cast<const float*>(qr)[32 * kb + 8 * q4 + i];
+      } else if (a.q_dtype == TQ_BF16) {
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) {
+          const u4 u = *reinterpret_cast<const u4*>(qr + 2 * (32 * kb + 8 * q4));
+#pragma unroll
+          for (int i = 0; i < 8; ++i) x[kb][i] = __uint_as_float(i & 1 ? u[i >> 1] & 0xFFFF0000u : u[i >> 1] << 16);
+        }
+      } else {
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) {
+          const half8 u = as_h8(*reinterpret_cast<const u4*>(qr + 2 * (32 * kb + 8 * q4)));
+#pragma unroll
+          for (int i = 0; i < 8; ++i) x[kb][i] = (float)u[i];
         }
       }
       float ss = 0.f;
@@ -365,8 +368,12 @@ __global__ __launch_bounds__(FT) void split_decode_kernel(UniformArgs a) {
       const float mnew = bm > m_run ? bm + RESCALE_MARGIN : m_run;
       const float corr = fexp2(m_run - mnew);
       l_run *= corr;
+      // (until a weight was nonzero the accumulators are zero; longer slot
+      // loops keep the multiplies, a branch per slot costs them more)
+      if (NPW > 2 || (setx && vset)) {
 #pragma unroll
-      for (int nb = 0; nb < 8; ++nb) acc[nb] *= corr;
+        for (int nb = 0; nb < 8; ++nb) acc[nb] *= corr;
+      }
       m_run = mnew;
     }
     float pv[NS];
@@ -481,7 +488,6 @@ __global__ __launch_bounds__(FT) void split_decode_kernel(UniformArgs a) {
 #pragma unroll
   for (int nb = 0; nb < 8; ++nb) acc_r[nb] = f4{0.f, 0.f, 0.f, 0.f};
 
-  static_assert(NPW >= 2, "two blocks in flight");
   uint8_t* nst = smem + Layout::nst + w * 256;
   uint8_t* vst = smem + SL::vst + w * SL::VSTW;
   const uint32_t cp = (uint32_t)(lane & 15) * 8;  // replica offset within a table row
@@ -683,12 +689,13 @@ namespace tq {
 // pair; a side is (H, L, I): hi / lo bits and whether it is integer.
 template <int G, int KH, int KL, bool KI, int VH, int VL, bool VI>
 inline void launch_split_g(const UniformArgs& a, int merge, hipStream_t s) {
-  if (a.bpw > FAST_WAVES * 4)
-    hipLaunchKernelGGL((uk::split_decode_kernel<G, 8, KH, KL, VH, VL, KI, VI>), dim3(a.nwg, a.hkv, a.batch),
-                       dim3(uk::FT), 0, s, a);
-  else
-    hipLaunchKernelGGL((uk::split_decode_kernel<G, 4, KH, KL, VH, VL, KI, VI>), dim3(a.nwg, a.hkv, a.batch),
-                       dim3(uk::FT), 0, s, a);
+  const dim3 grid(a.nwg, a.hkv, a.batch), wg(uk::FT);
+  switch (uniform_npw(a.bpw)) {
+    case 1: hipLaunchKernelGGL((uk::split_decode_kernel<G, 1, KH, KL, VH, VL, KI, VI>), grid, wg, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((uk::split_decode_kernel<G, 2, KH, KL, VH, VL, KI, VI>), grid, wg, 0, s, a); break;
+    case 4: hipLaunchKernelGGL((uk::split_decode_kernel<G, 4, KH, KL, VH, VL, KI, VI>), grid, wg, 0, s, a); break;
+    default: hipLaunchKernelGGL((uk::split_decode_kernel<G, 8, KH, KL, VH, VL, KI, VI>), grid, wg, 0, s, a); break;
+  }
   if (merge) hipLaunchKernelGGL((uk::uniform_merge_kernel<G>), dim3(a.hq, a.batch), dim3(uk::MT), 0, s, a);
 }
 

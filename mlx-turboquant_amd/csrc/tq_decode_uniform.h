@@ -5,8 +5,8 @@
 //
 // Grid (nwg, hkv, batch): workgroup c of (sequence b, kv head g) owns
 //  - the compressed 32-token blocks [c*bpw, (c+1)*bpw) of the sequence (bpw <=
-//    8 NPW, NPW = 4 or 8): wave w takes blocks c*bpw + w + 8k, k < NPW, with
-//    two blocks' loads in flight while it computes;
+//    8 NPW, NPW = 1, 2, 4 or 8): wave w takes blocks c*bpw + w + 8k, k < NPW,
+//    with two blocks' loads in flight while it computes;
 //  - the fp16 tokens [c*fpw, (c+1)*fpw) (fpw <= 16) of the sequence's [sink |
 //    residual ring] list, staged in LDS during set-up and scored by wave 0
 //    (the first to be issued on its SIMD) before its compressed blocks.
@@ -266,8 +266,13 @@ __device__ inline __amdgpu_buffer_rsrc_t rsrc(const void* p, int bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
 }
 
-// NPW: compressed blocks per wave (4, or 8 for long contexts and large
-// batches, where fewer workgroups pay the set-up and combine)
+// NPW: compressed blocks per wave. Every slot is computed, empty or not (about
+// 500 VALU instructions), so a call takes the smallest that fits: 1 up to 8
+// blocks per workgroup (8 kv heads: 8K tokens), 8 for long contexts and large
+// batches, where fewer workgroups pay the set-up and combine. Whole call per layer
+// (32 heads on 8, against 4 slots always): K4/V2 T 1,000 14.5 -> 11.4 us, T 4,000
+// 14.8 -> 11.4, T 12,000 14.9 -> 13.2; K4/V4 T 1,000 15.9 -> 11.7; 4 x 8,000
+// tokens 25.9 -> 21.2.
 template <int G, bool QB, int NPW, int KB = 4, int VB = 2, bool BF = false>
 __global__ __launch_bounds__(FT) void uniform_decode_kernel(UniformArgs a) {
   static_assert(KB >= 2 && KB <= 4 && VB >= 2 && VB <= 4, "integer widths 2-4");
@@ -553,7 +558,7 @@ __global__ __launch_bounds__(FT) void uniform_decode_kernel(UniformArgs a) {
   __syncthreads();
 
   // block 1 once the tables are built; block k + 2 as slot k starts
-  load_slot(1);
+  if constexpr (NPW > 1) load_slot(1);
 
 
   // q rows as MFMA A operands (row r = query head min(r, G-1), k-slots = dims
@@ -594,22 +599,25 @@ __global__ __launch_bounds__(FT) void uniform_decode_kernel(UniformArgs a) {
     }
     if (!q_exact) {
       // the fp16 high part / remainder of q 2^-qe
-      float x[4][8];
+      float x[4][8];  // (one branch on the type around each loop: inside, there is one per element)
+      if (a.q_dtype == TQ_F32) {
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
-        const int d = 32 * kb + 8 * q4;
-        if (a.q_dtype == TQ_F32) {
-          const float4 u0 = *reinterpret_cast<const float4*>(qr + 4 * d);
-          const float4 u1 = *reinterpret_cast<const float4*>(qr + 4 * d + 16);
-          x[kb][0] = u0.x; x[kb][1] = u0.y; x[kb][2] = u0.z; x[kb][3] = u0.w;
-          x[kb][4] = u1.x; x[kb][5] = u1.y; x[kb][6] = u1.z; x[kb][7] = u1.w;
-        } else {
-          const u4 u = *reinterpret_cast<const u4*>(qr + 2 * d);
+        for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const uint32_t hb = (u[i >> 1] >> (16 * (i & 1))) & 0xFFFFu;
-            x[kb][i] = a.q_dtype == TQ_BF16 ? __uint_as_float(hb << 16) : (float)__builtin_bit_cast(_Float16, (uint16_t)hb);
-          }
+          for (int i = 0; i < 8; ++i) x[kb][i] = reinterpret_cast<const float*>(qr)[32 * kb + 8 * q4 + i];
+      } else if (a.q_dtype == TQ_BF16) {
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) {
+          const u4 u = *reinterpret_cast<const u4*>(qr + 2 * (32 * kb + 8 * q4));
+#pragma unroll
+          for (int i = 0; i < 8; ++i) x[kb][i] = __uint_as_float(i & 1 ? u[i >> 1] & 0xFFFF0000u : u[i >> 1] << 16);
+        }
+      } else {
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) {
+          const half8 u = as_h8(*reinterpret_cast<const u4*>(qr + 2 * (32 * kb + 8 * q4)));
+#pragma unroll
+          for (int i = 0; i < 8; ++i) x[kb][i] = (float)u[i];
         }
       }
       float ss = 0.f;
@@ -712,8 +720,12 @@ __global__ __launch_bounds__(FT) void uniform_decode_kernel(UniformArgs a) {
       const float mnew = bm > m_run ? bm + RESCALE_MARGIN : m_run;
       const float corr = fexp2(m_run - mnew);
       l_run *= corr;
+      // (until a weight was nonzero the accumulators are zero; longer slot
+      // loops keep the multiplies, a branch per slot costs them more)
+      if (NPW > 2 || (setx && vset)) {
 #pragma unroll
-      for (int nb = 0; nb < 8; ++nb) acc[nb] *= corr;
+        for (int nb = 0; nb < 8; ++nb) acc[nb] *= corr;
+      }
       m_run = mnew;
     }
     float pv[NS];
@@ -860,7 +872,6 @@ __global__ __launch_bounds__(FT) void uniform_decode_kernel(UniformArgs a) {
 #pragma unroll
   for (int nb = 0; nb < 8; ++nb) acc_r[nb] = f4{0.f, 0.f, 0.f, 0.f};
 
-  static_assert(NPW >= 2, "two blocks in flight");
 
   // ---- the compressed blocks of this wave (rotated space)
   uint8_t* nst = smem + Layout::nst + w * 256;  // this wave's norm staging: [key norms 32][value norms 32]

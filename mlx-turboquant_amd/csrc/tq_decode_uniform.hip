@@ -7,12 +7,13 @@ namespace tq {
 
 template <int G, bool QB, bool BF>
 static void launch_u(const UniformArgs& a, int merge, hipStream_t s) {
-  if (a.bpw > FAST_WAVES * 4)
-    hipLaunchKernelGGL((uk::uniform_decode_kernel<G, QB, 8, 4, 2, BF>), dim3(a.nwg, a.hkv, a.batch), dim3(uk::FT), 0,
-                       s, a);
-  else
-    hipLaunchKernelGGL((uk::uniform_decode_kernel<G, QB, 4, 4, 2, BF>), dim3(a.nwg, a.hkv, a.batch), dim3(uk::FT), 0,
-                       s, a);
+  const dim3 grid(a.nwg, a.hkv, a.batch), wg(uk::FT);
+  switch (uniform_npw(a.bpw)) {
+    case 1: hipLaunchKernelGGL((uk::uniform_decode_kernel<G, QB, 1, 4, 2, BF>), grid, wg, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((uk::uniform_decode_kernel<G, QB, 2, 4, 2, BF>), grid, wg, 0, s, a); break;
+    case 4: hipLaunchKernelGGL((uk::uniform_decode_kernel<G, QB, 4, 4, 2, BF>), grid, wg, 0, s, a); break;
+    default: hipLaunchKernelGGL((uk::uniform_decode_kernel<G, QB, 8, 4, 2, BF>), grid, wg, 0, s, a); break;
+  }
   if (merge) hipLaunchKernelGGL((uk::uniform_merge_kernel<G>), dim3(a.hq, a.batch), dim3(uk::MT), 0, s, a);
 }
 

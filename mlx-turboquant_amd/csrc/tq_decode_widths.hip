@@ -8,12 +8,13 @@ namespace tq {
 
 template <int G, int KB, int VB>
 static void launch_w(const UniformArgs& a, int merge, hipStream_t s) {
-  if (a.bpw > FAST_WAVES * 4)
-    hipLaunchKernelGGL((uk::uniform_decode_kernel<G, false, 8, KB, VB>), dim3(a.nwg, a.hkv, a.batch), dim3(uk::FT), 0,
-                       s, a);
-  else
-    hipLaunchKernelGGL((uk::uniform_decode_kernel<G, false, 4, KB, VB>), dim3(a.nwg, a.hkv, a.batch), dim3(uk::FT), 0,
-                       s, a);
+  const dim3 grid(a.nwg, a.hkv, a.batch), wg(uk::FT);
+  switch (uniform_npw(a.bpw)) {
+    case 1: hipLaunchKernelGGL((uk::uniform_decode_kernel<G, false, 1, KB, VB>), grid, wg, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((uk::uniform_decode_kernel<G, false, 2, KB, VB>), grid, wg, 0, s, a); break;
+    case 4: hipLaunchKernelGGL((uk::uniform_decode_kernel<G, false, 4, KB, VB>), grid, wg, 0, s, a); break;
+    default: hipLaunchKernelGGL((uk::uniform_decode_kernel<G, false, 8, KB, VB>), grid, wg, 0, s, a); break;
+  }
   if (merge) hipLaunchKernelGGL((uk::uniform_merge_kernel<G>), dim3(a.hq, a.batch), dim3(uk::MT), 0, s, a);
 }
 
