@@ -1577,13 +1577,19 @@ static int mfma_kind(const tq_codec* c) {
   return 0;
 }
 
-// The kernels of tq_decode_mfma.h: one query token, no sketch, head_dim 64 /
-// 96 / 128 / 256, widths 2-4 and 2.5 / 3.5 on either side (keys at head_dim 96:
+// The kernels of tq_decode_mfma.h: one query token, no sketch or one of 32
+// projections (the cache's default; its two terms are one k-step and two more
+// accumulators, longer sketches do not fit the registers), head_dim 64 / 96 /
+// 128 / 256, widths 2-4 and 2.5 / 3.5 on either side (keys at head_dim 96:
 // integer, the 12 dims of a lane's half are not whole 8-dim k-steps), fp16 or
 // bf16 uncompressed tokens, any query-head ratio, uniform or ragged. Code
 // rows are read at byte granularity; q, sink and ring rows in 16-byte pieces.
 static bool mfma_eligible(const tq_codec* kc, const tq_codec* vc, const tq_attn_desc* d) {
-  if (d->n_q > 1 || (d->qjl && d->max_comp > 0)) return false;
+  if (d->n_q > 1) return false;
+  if (d->qjl && d->max_comp > 0 &&
+      !(kc->qjl_m == 32 && aligned16(kc->qjl_proj) && (reinterpret_cast<uintptr_t>(d->kstore.gamma) & 3) == 0 &&
+        (reinterpret_cast<uintptr_t>(d->vstore.gamma) & 3) == 0))
+    return false;
   if (!(kc->d == 64 || kc->d == 96 || kc->d == 128 || kc->d == 256) || vc->d != kc->d) return false;
   const int kk = mfma_kind(kc), vk = mfma_kind(vc);
   if (!kk || !vk || (kc->d == 96 && kk > 4)) return false;
@@ -1632,7 +1638,7 @@ static void mfma_geometry(const tq_attn_desc* d, int& gsub, int& g, int& ncw, in
 static size_t mfma_part_bytes(const tq_codec* kc, const tq_attn_desc* d) {
   int gsub, g, ncw, nfw;
   mfma_geometry(d, gsub, g, ncw, nfw);
-  return (size_t)d->batch * d->hq * (ncw + nfw) * (kc->d + 4) * 4;
+  return (size_t)d->batch * d->hq * (ncw + nfw) * (kc->d + 4 + (d->qjl ? 32 : 0)) * 4;
 }
 
 static int mfma_run(const tq_codec* kc, const tq_codec* vc, const tq_attn_desc* d, void* workspace, hipStream_t s) {
@@ -1659,12 +1665,33 @@ static int mfma_run(const tq_codec* kc, const tq_codec* vc, const tq_attn_desc* 
   a.vbh = vc->bits_hi; a.vbl = vk > 4 ? vc->bits_lo : vc->bits_hi; a.vfrac = vk > 4;
   a.part = static_cast<float*>(workspace);
   a.bf = d->kv_dtype == TQ_BF16;
+  if (d->qjl && d->max_comp > 0) {
+    a.ksg = d->kstore.signs; a.ksg_hs = d->kstore.sign_head_stride;
+    a.vsg = d->vstore.signs; a.vsg_hs = d->vstore.sign_head_stride;
+    a.kgam = d->kstore.gamma; a.kgam_hs = d->kstore.gamma_head_stride;
+    a.vgam = d->vstore.gamma; a.vgam_hs = d->vstore.gamma_head_stride;
+    a.proj = kc->qjl_proj;
+    switch (kc->d) {
+      case 64: return launch_mfma_d64_qjl(a, kk, s);
+      case 96: return launch_mfma_d96_qjl(a, kk, s);
+      case 128: return launch_mfma_d128_qjl(a, kk, s);
+      default: return launch_mfma_d256_qjl(a, kk, s);
+    }
+  }
   switch (kc->d) {
     case 64: return launch_mfma_d64(a, kk, s);
     case 96: return launch_mfma_d96(a, kk, s);
     case 128: return launch_mfma_d128(a, kk, s);
     default: return launch_mfma_d256(a, kk, s);
   }
+}
+
+// Sketched calls of uniform batches at 32 projections take the mfma kernels (one
+// pass, two launches) before the K4/V2 kernels with the terms around them (six
+// launches): K4/V2, 32 heads on 8, T 4,000 35.9 -> 17.4 us per layer, T 32,768
+// 39.9 -> 27.8. Ragged batches and longer sketches keep the latter.
+static bool qjl_mfma(const tq_codec* kc, const tq_codec* vc, const tq_attn_desc* d) {
+  return d->qjl && d->max_comp > 0 && !d->comp_len && !d->sink_len && !d->res_len && mfma_eligible(kc, vc, d);
 }
 
 // The QJL route: S q, key-term bias, K4/V2 partials with the bias
@@ -1959,6 +1986,10 @@ int tq_decode_attention(const tq_codec* kc, const tq_codec* vc, const tq_attn_de
   if (d->max_comp == 0 && !(d->flags & TQ_ATTN_GENERAL) && (d->max_sink > 0 || d->max_res > 0) &&
       dense_check(d, kc->d, false) == TQ_OK)
     return dense_run(d, workspace, workspace_bytes, s);
+  if (qjl_mfma(kc, vc, d) && !(d->flags & TQ_ATTN_GENERAL)) {
+    if (mfma_run(kc, vc, d, workspace, s) != 0) TQ_LAUNCH_CHECK("tq_decode_attention (mfma)");
+    return TQ_OK;
+  }
   if (qjl && d->max_comp > 0 && fast_eligible(kc, vc, d, true) && !(d->flags & TQ_ATTN_GENERAL))
     return qjl_fast_run(kc, vc, d, workspace, workspace_bytes, s);
   if (fast_eligible(kc, vc, d) && !(d->flags & TQ_ATTN_GENERAL)) {
@@ -2079,6 +2110,7 @@ int tq_debug_decode_route(const tq_codec* kc, const tq_codec* vc, const tq_attn_
   if (d->flags & TQ_ATTN_GENERAL) return 0;
   if (prefill_eligible(kc, vc, d)) return 6;
   if (d->max_comp == 0 && (d->max_sink > 0 || d->max_res > 0) && dense_check(d, kc->d, false) == TQ_OK) return 1;
+  if (qjl_mfma(kc, vc, d)) return 7;
   if (d->qjl && d->max_comp > 0 && fast_eligible(kc, vc, d, true)) return 3;
   if (fast_eligible(kc, vc, d)) return 2;
   int nwg, bpw, fpw;

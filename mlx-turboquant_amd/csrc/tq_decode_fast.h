@@ -196,16 +196,26 @@ struct MfmaArgs {
   const float* vcen_hi; const float* vcen_lo;
   int vbh, vbl, vfrac;   // value widths; vfrac: fractional (split at D / 2)
   int bf;                // bf16 sink / ring tokens (else fp16)
-  float* part;           // (batch, hkv gsub, ncw + nfw, g, D + 4)
+  // a 32-projection QJL sketch (launch_mfma_d*_qjl): sign rows of 4 bytes, residual norms, S (32, D) float32
+  const uint8_t* ksg; int64_t ksg_hs;
+  const uint8_t* vsg; int64_t vsg_hs;
+  const float* kgam;  int64_t kgam_hs;
+  const float* vgam;  int64_t vgam_hs;
+  const float* proj;
+  float* part;           // (batch, hkv gsub, ncw + nfw, g, D + 4; + 32 with a sketch)
   int ncw, nfw;
   int tail;              // LDS offset past the tables / combine buffers (set by the launch)
 };
 // Partials and merge for head_dim 64 / 96 / 128 / 256; kk: the key width kind
 // (2-4, 5 = 2.5 bits, 7 = 3.5 bits).
 int launch_mfma_d64(const MfmaArgs& a, int kk, hipStream_t s);
+int launch_mfma_d64_qjl(const MfmaArgs& a, int kk, hipStream_t s);
 int launch_mfma_d96(const MfmaArgs& a, int kk, hipStream_t s);
+int launch_mfma_d96_qjl(const MfmaArgs& a, int kk, hipStream_t s);
 int launch_mfma_d128(const MfmaArgs& a, int kk, hipStream_t s);
+int launch_mfma_d128_qjl(const MfmaArgs& a, int kk, hipStream_t s);
 int launch_mfma_d256(const MfmaArgs& a, int kk, hipStream_t s);
+int launch_mfma_d256_qjl(const MfmaArgs& a, int kk, hipStream_t s);
 
 // Arguments of the dense (fp16 / bf16 K/V) decode-attention kernel: the
 // fp16 segments of tq_attn_desc, head_dim 128.

@@ -106,6 +106,11 @@ __device__ inline void split_b(const float (&v)[8], u4 (&p)[3]) {
   }
 }
 
+constexpr int QM = 32;         // projections of the sketch
+constexpr int SQS = 2 * QM + 16;
+constexpr float SQD = 32.f;    // S q is held over this (fp16 range: |S q| <= ||S_p|| ||q||)
+constexpr float SQRT_HALF_PI_M = 1.2533141373155003f;
+
 // N bytes at any address into dwords (the compiler picks the load widths)
 template <int N>
 __device__ inline void load_bytes(uint32_t (&w)[(N + 3) / 4], const uint8_t* p) {
@@ -147,37 +152,49 @@ struct KGeo {
 
 // LDS: [key tables | value tables], reused by the combine buffers, then (from
 // MfmaArgs::tail) the query operands, the combine headers and the norm staging.
-template <int D, int GC>
+template <int D, int GC, bool QJ>
 struct Lds {
   static constexpr int QS = 2 * D + 16;               // bytes per (head, part) of the query operands
-  static constexpr int CMS = D + 4;                   // floats per (wave, head) of the combine buffers
+  static constexpr int W = D + (QJ ? QM : 0);         // sums per head
+  static constexpr int CMS = W + 4;                   // floats per (wave, head) of the combine buffers
   static constexpr int cmb = MW * GC * CMS * 4;
   static constexpr int qsrc = 0;                      // offsets past tail: the query, 2 or 3 parts per head
   static constexpr int qop = qsrc + GC * 3 * QS;      // the rotated query
   static constexpr int qex = qop + GC * 2 * QS;       // 2^qe per head
-  static constexpr int cml = qex + GC * 4;
+  static constexpr int sqo = qex + GC * 4;            // S q, high part / remainder rows of 32 (+ 8)
+  static constexpr int cml = sqo + (QJ ? GC * 2 * SQS : 0);
   static constexpr int nst = cml + MW * GC * 8;
-  static constexpr int end = nst + MW * 256;
+  static constexpr int end = nst + MW * (QJ ? 512 : 256);
 };
 
-template <int D, int KK>
+template <int D, int KK, bool QJ>
 struct Blk {
   uint32_t k[2][KGeo<D, KK>::NDW];
   uint32_t v[8][D == 256 ? 2 : 1];
   float nk, nv;  // of token t0 + (lane & 31)
+  uint32_t zk[QJ ? 2 : 1], zv[QJ ? 8 : 1];  // sign bytes: projections 8 q4 .. of token r; 8 (r >> 2) .. of the value tokens
+  float gk, gv;
 };
 
-// VF: the values' width is fractional (two tables, rows of two widths)
-template <int D, int GC, int KK, bool VF>
+// VF: the values' width is fractional (two tables, rows of two widths); QJ: the
+// terms of a 32-projection QJL sketch (qjl.py:70-94). Key term: S (scale q) is
+// computed at the query rotation (S's rows as two more tiles), its fp16 high
+// part / remainder columns meet one operand of 16 tokens x 32 signs (+-1, exact)
+// per tile: one MFMA. Value term: u = sum_t p_t gamma_t z_t accumulates in two
+// more MFMAs (rows = projections) and travels with the partial; the merge
+// applies S^T. Per layer: head_dim 64 59.4 -> 16.8 us (13.0 without the sketch),
+// head_dim 256 106.7 -> 32.5, bf16 K4/V4 28 heads on 4 104 -> 20.9 (the cases
+// above, against the general kernel).
+template <int D, int GC, int KK, bool VF, bool QJ>
 __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
   using G_ = KGeo<D, KK>;
-  using L_ = Lds<D, GC>;
+  using L_ = Lds<D, GC, QJ>;
   constexpr int U = D / 16;           // dims per MFMA row of the output
   constexpr int NF = U / 2;           // pair fields per row
   constexpr int VW = D == 256 ? 2 : 1;
   constexpr int TS = GC == 4 ? 2 : 1; // tiles sharing the columns
   constexpr int NS = 8 / TS;          // scores per lane per block
-  constexpr int PSD = D + 4;
+  constexpr int PSD = L_::W + 4;
   // the first uncompressed block's keys and values are requested before the
   // query is converted; at D = 256 the registers do not hold both: each is
   // requested where it is used
@@ -235,7 +252,7 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
     voff[i] = min(bit >> 3, vrow - 4);
     vsh[i] = bit - 8 * voff[i];
   }
-  auto load_blk = [&](Blk<D, KK>& B, int blk) {
+  auto load_blk = [&](Blk<D, KK, QJ>& B, int blk) {
     const int t0 = blk << 5, last = comp - 1;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -260,6 +277,17 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
     const int tn = min(t0 + (lane & 31), last);
     B.nk = knorm[tn];
     B.nv = vnorm[tn];
+    if constexpr (QJ) {
+      const uint8_t* ks = a.ksg + (int64_t)row * a.ksg_hs + q4;
+      const uint8_t* vs = a.vsg + (int64_t)row * a.vsg_hs + (r >> 2);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) B.zk[t] = ks[(uint32_t)min(t0 + 16 * t + r, last) * (QM / 8)];
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        B.zv[i] = vs[(uint32_t)min(t0 + (i < 4 ? 4 * q4 + i : 12 + 4 * q4 + i), last) * (QM / 8)];
+      B.gk = a.kgam[(int64_t)row * a.kgam_hs + tn];
+      B.gv = a.vgam[(int64_t)row * a.vgam_hs + tn];
+    }
   };
 
   // ---- set-up: the query (8 elements per thread, LPH lanes per head) and the
@@ -279,7 +307,7 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
     }
   }
   uint32_t cw = 0;
-  Blk<D, KK> B0, B1;
+  Blk<D, KK, QJ> B0, B1;
   // rows 16 jt + r of R (fp16 high part, remainder) as B operands of the query rotation
   u4 rqh[G_::KS], rql[G_::KS];
   auto load_rot = [&](int jt) {
@@ -410,6 +438,40 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
         }
       }
     }
+    if constexpr (QJ) {
+      // S (q 2^-qe) qscale / SQD, tiles U and U + 1 of the same waves' sequence
+      for (int jt = w; jt < U + QM / 16; jt += MW) {
+        if (jt < U) continue;
+        const int p = 16 * (jt - U) + r;
+        const float* sp = a.proj + p * D + 8 * q4;
+        f4 dq = {0.f, 0.f, 0.f, 0.f}, dl = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kb = 0; kb < G_::KS; ++kb) {
+          half8 sh, sl;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float v = sp[32 * kb + e];
+            sh[e] = (_Float16)v;
+            sl[e] = (_Float16)(v - (float)sh[e]);
+          }
+          const half8 qhi = *reinterpret_cast<const half8*>(qs + 64 * kb);
+          dq = mfma(qhi, sh, dq);
+          dl = mfma(qhi, sl, dl);
+          dl = mfma(*reinterpret_cast<const half8*>(qs + L_::QS + 64 * kb), sh, dl);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int h = 4 * q4 + i;
+          if (h < a.g && h < GC) {
+            const float v = (dq[i] + dl[i]) * (a.qscale / SQD);
+            const _Float16 hi = (_Float16)v, lo = (_Float16)(v - (float)hi);
+            uint8_t* d = tail + L_::sqo + h * 2 * SQS + 2 * p;
+            *reinterpret_cast<_Float16*>(d) = hi;
+            *reinterpret_cast<_Float16*>(d + SQS) = lo;
+          }
+        }
+      }
+    }
     __syncthreads();
   }
 
@@ -435,6 +497,8 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
   f4 acc[U];
 #pragma unroll
   for (int nb = 0; nb < U; ++nb) acc[nb] = f4{0.f, 0.f, 0.f, 0.f};
+  f4 accu[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};  // value term, projections 2 row + n2
+  float gv[NS], pu[NS];  // the block's value residual norms, weights times them
 
   bool any = false;   // the wave has accumulated a block
   // running max and sum over the block's scores s, weights times nv to pv; the
@@ -451,6 +515,7 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
         l_run *= corr;
 #pragma unroll
         for (int nb = 0; nb < U; ++nb) acc[nb] *= corr;
+        if constexpr (QJ) accu[0] *= corr, accu[1] *= corr;
       }
       m_run = mnew;
     }
@@ -460,6 +525,7 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
       const float p = fexp2(s[i] - m_run);
       l_run += p;
       pv[i] = p * nv[i];
+      if constexpr (QJ) pu[i] = p * gv[i];
     }
   };
   // the two tiles' k-slots of the P^T operand from the lane's packed pairs
@@ -476,12 +542,12 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
     }
     return pb;
   };
-  // P^T in fp16: high part or remainder by column, times 2^-vx; vx is set by
-  // the wave's first nonzero weight (the accumulators are zero until then)
-  auto weights_h = [&](const float (&pv)[NS]) {
+  // P^T in fp16 (operand_h): high part or remainder by column, times 2^-vx; vx is
+  // set by the wave's first nonzero weight (the accumulators are zero until then)
+  auto exponent_h = [&](const float (&pv)[NS]) {
     float pm = 0.f;
 #pragma unroll
-    for (int i = 0; i < NS; ++i) pm = fmaxf(pm, fabsf(pv[i]));
+    for (int i = 0; i < NS; ++i) pm = fmaxf(pm, QJ ? fmaxf(fabsf(pv[i]), fabsf(pu[i])) : fabsf(pv[i]));
     const float pmx = pm * __builtin_amdgcn_ldexpf(1.f, -vx);
     if (__builtin_amdgcn_ballot_w64(pmx > uk::PV_LIMIT || (!vset && pmx > 0.f)) != 0) {
       const float cm = rows_max(pmx);  // max of the column
@@ -493,9 +559,12 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
         const float f = __builtin_amdgcn_ldexpf(1.f, -dx);
 #pragma unroll
         for (int nb = 0; nb < U; ++nb) acc[nb] *= f;
+        if constexpr (QJ) accu[0] *= f, accu[1] *= f;
         vx += dx;
       }
     }
+  };
+  auto operand_h = [&](const float (&pv)[NS]) {
     const float down = __builtin_amdgcn_ldexpf(1.f, -vx);
     uint32_t d[NS / 2];
 #pragma unroll
@@ -531,18 +600,27 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
     const uint32_t cpv = cp + G_::TABS + (vlo ? (1u << (2 * a.vbh)) * TROW : 0u);
     const uint32_t vbw = 2 * vb;  // bits per field
     const float ks = qe_scale * (1.f / CSC);
-    float* nst = reinterpret_cast<float*>(tail + L_::nst) + w * 64;  // [key norms 32][value norms 32]
+    float* nst = reinterpret_cast<float*>(tail + L_::nst) + w * (QJ ? 128 : 64);  // [key norms 32][value norms 32][gammas]
+    half8 qz;  // S q, k-slot (q4, e) = projection 8 q4 + e
+    if constexpr (QJ) qz = *reinterpret_cast<const half8*>(tail + L_::sqo + (hd * 2 + (lo_part ? 1 : 0)) * SQS + 16 * q4);
     auto lut = [&](uint32_t addr) { return *reinterpret_cast<const u2*>(smem + addr); };
-    auto compute = [&](const Blk<D, KK>& B, int blk) {
+    auto compute = [&](const Blk<D, KK, QJ>& B, int blk) {
       const int t0 = blk << 5;
       nst[lane] = lane < 32 ? B.nk : B.nv;
-      float nk[NS], nv[NS];
+      if constexpr (QJ) nst[64 + lane] = lane < 32 ? B.gk : B.gv;
+      float nk[NS], nv[NS], gk[NS];
 #pragma unroll
       for (int t = 0; t < 2 / TS; ++t) {
         const float4 k4 = *reinterpret_cast<const float4*>(nst + 16 * (t + tile) + 4 * q4);
         const float4 v4 = *reinterpret_cast<const float4*>(nst + 32 + 16 * (t + tile) + 4 * q4);
         nk[4 * t] = k4.x * ks; nk[4 * t + 1] = k4.y * ks; nk[4 * t + 2] = k4.z * ks; nk[4 * t + 3] = k4.w * ks;
         nv[4 * t] = v4.x; nv[4 * t + 1] = v4.y; nv[4 * t + 2] = v4.z; nv[4 * t + 3] = v4.w;
+        if constexpr (QJ) {
+          const float4 a4 = *reinterpret_cast<const float4*>(nst + 64 + 16 * (t + tile) + 4 * q4);
+          const float4 b4 = *reinterpret_cast<const float4*>(nst + 96 + 16 * (t + tile) + 4 * q4);
+          gk[4 * t] = a4.x; gk[4 * t + 1] = a4.y; gk[4 * t + 2] = a4.z; gk[4 * t + 3] = a4.w;
+          gv[4 * t] = b4.x; gv[4 * t + 1] = b4.y; gv[4 * t + 2] = b4.z; gv[4 * t + 3] = b4.w;
+        }
       }
       f4 sc2[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
@@ -566,10 +644,47 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
         }
       }
       float sc[NS];
-      lane_scores(sc, sc2[0], sc2[1], nk, t0, comp);
+      if constexpr (QJ) {
+        // key term: + gamma_k sqrt(pi / 2) / D (S q) . z, before the mask
+        f4 sz[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const uint32_t nz = ~B.zk[t];
+          u4 z;
+#pragma unroll
+          for (int f = 0; f < 4; ++f)
+            z[f] = 0x3C003C00u | ((nz << (15 - 2 * f)) & 0x8000u) | ((nz << (30 - 2 * f)) & 0x80000000u);
+          sz[t] = mfma(as_h8(z), qz, f4{0.f, 0.f, 0.f, 0.f});
+        }
+        const float zs = qe_scale * (SQD * SQRT_HALF_PI_M / D);
+        float fz[NS], sq[NS];
+#pragma unroll
+        for (int i = 0; i < NS; ++i) fz[i] = gk[i] * zs;
+        lane_scores(sq, sz[0], sz[1], fz, t0, comp);
+        lane_scores(sc, sc2[0], sc2[1], nk, t0, comp);
+#pragma unroll
+        for (int i = 0; i < NS; ++i) sc[i] += sq[i];
+      } else {
+        lane_scores(sc, sc2[0], sc2[1], nk, t0, comp);
+      }
       float pv[NS];
       softmax(sc, nv, pv);
-      const half8 pb = as_h8(weights_h(pv));
+      exponent_h(pv);
+      const half8 pb = as_h8(operand_h(pv));
+      if constexpr (QJ) {
+        const half8 ub = as_h8(operand_h(pu));
+        u4 z[2];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          // bits 2 (r & 3) + n2 of the pair's sign bytes: clear = -1
+          const uint32_t x = ~B.zv[2 * j] >> (2 * (r & 3)), y = ~B.zv[2 * j + 1] >> (2 * (r & 3));
+#pragma unroll
+          for (int n2 = 0; n2 < 2; ++n2)
+            z[n2][j] = 0x3C003C00u | ((x << (15 - n2)) & 0x8000u) | ((y << (31 - n2)) & 0x80000000u);
+        }
+        accu[0] = mfma(as_h8(z[0]), ub, accu[0]);
+        accu[1] = mfma(as_h8(z[1]), ub, accu[1]);
+      }
 #pragma unroll
       for (int f = 0; f < NF; ++f) {
         // dims U r + 2 f, + 1 of the block's 4 token pairs
@@ -614,7 +729,7 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
       f4 sc2[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
       float sc[NS], kf[NS], nv[NS], pv[NS];
 #pragma unroll
-      for (int i = 0; i < NS; ++i) kf[i] = a.qscale * qe_scale, nv[i] = 1.f;
+      for (int i = 0; i < NS; ++i) kf[i] = a.qscale * qe_scale, nv[i] = 1.f, gv[i] = 0.f;
       if (a.bf) {
         // bf16 tokens on bf16 MFMAs: the third part of the query (and of the
         // weights) in an operand of its own, in the first part's columns
@@ -657,7 +772,8 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
         pb = slots(d);
         p3 = slots(d3);
       } else {
-        pb = weights_h(pv);
+        exponent_h(pv);
+        pb = operand_h(pv);
       }
 #pragma unroll
       for (int nb = 0; nb < U; ++nb) {
@@ -678,7 +794,7 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
   // ---- combine the waves through LDS (the table region); the two fp16 parts
   // of a head meet through `partner`, for GC = 4 the two tiles at their common max
   l_run = rows_sum(l_run);
-  float tsc = __builtin_amdgcn_ldexpf(packed ? 1.f / CSC : 1.f, vx);
+  float tsc = __builtin_amdgcn_ldexpf(1.f, vx);
   if constexpr (TS == 2) {
     const float m2 = fmaxf(m_run, row_ror<8>(m_run));
     const float t = fexp2(m_run - m2);
@@ -688,6 +804,7 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
     m_run = m2;
   }
   __syncthreads();
+  const float tscr = packed ? tsc * (1.f / CSC) : tsc;  // (the tables hold CSC c)
   float* cm = reinterpret_cast<float*>(smem) + (w * GC) * L_::CMS;
   float* cl = reinterpret_cast<float*>(tail + L_::cml);  // [wave][head][M, L]
 #pragma unroll
@@ -695,7 +812,7 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
     float vr[U];
 #pragma unroll
     for (int nb = 0; nb < U; ++nb) {
-      float x = (acc[nb][i] + uk::partner<GC>(acc[nb][i])) * tsc;
+      float x = (acc[nb][i] + uk::partner<GC>(acc[nb][i])) * tscr;
       if constexpr (TS == 2) x += row_ror<8>(x);
       vr[nb] = x;
     }
@@ -704,12 +821,21 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
 #pragma unroll
       for (int nb = 0; nb < U; nb += 2) *reinterpret_cast<float2*>(d + nb) = make_float2(vr[nb], vr[nb + 1]);
     }
+    if constexpr (QJ) {
+      float u[2];
+#pragma unroll
+      for (int n2 = 0; n2 < 2; ++n2) {
+        u[n2] = (accu[n2][i] + uk::partner<GC>(accu[n2][i])) * tsc;
+        if constexpr (TS == 2) u[n2] += row_ror<8>(u[n2]);
+      }
+      if (writer) *reinterpret_cast<float2*>(cm + hd * L_::CMS + D + 2 * (4 * q4 + i)) = make_float2(u[0], u[1]);
+    }
   }
   if (q4 == 0 && writer) *reinterpret_cast<float2*>(cl + (w * GC + hd) * 2) = make_float2(m_run, l_run);
   __syncthreads();
   const float* cms = reinterpret_cast<const float*>(smem);
-  for (int e = tid; e < a.g * D; e += MTH) {
-    const int h = e / D, j = e % D;
+  for (int e = tid; e < a.g * L_::W; e += MTH) {
+    const int h = e / L_::W, j = e % L_::W;
     float M = M_INIT;
 #pragma unroll
     for (int ww = 0; ww < MW; ++ww) M = fmaxf(M, cl[(ww * GC + h) * 2]);
@@ -742,13 +868,14 @@ struct MergeGeo {
   static constexpr int RR = D / RB;             // rows per block
 };
 
-template <int D>
+template <int D, bool QJ>
 __global__ __launch_bounds__(MergeGeo<D>::NT) void mfma_merge_kernel(MfmaArgs a, int np) {
   using M_ = MergeGeo<D>;
-  constexpr int PSD = D + 4, MB = M_::MB, PG = M_::PG;
+  constexpr int PSD = D + 4 + (QJ ? QM : 0), MB = M_::MB, PG = M_::PG;
+  constexpr int UG = QJ ? M_::NT / QM : 1, SR = QJ ? QM / M_::RB : 1;  // groups of the value term, rows of S per block
   extern __shared__ __align__(16) uint8_t smem[];
   float* wsh = reinterpret_cast<float*>(smem);  // [np rounded up to whole rounds] weights
-  __shared__ float ys[PG][D], xs[PG][D], yt[D];
+  __shared__ float ys[PG][D], xs[PG][D], yt[D + (QJ ? QM : 0)], us[UG][QM];
   __shared__ __align__(16) float red[M_::RB][D];
   const int hq = blockIdx.x, b = blockIdx.y;
   const int gy = hq / a.g, h = hq % a.g;
@@ -769,6 +896,12 @@ __global__ __launch_bounds__(MergeGeo<D>::NT) void mfma_merge_kernel(MfmaArgs a,
   float4 rr[M_::RR];
 #pragma unroll
   for (int k = 0; k < M_::RR; ++k) rr[k] = *reinterpret_cast<const float4*>(a.vrot + (M_::RR * ib + k) * D + j4);
+
+  float4 sr[SR];
+  if constexpr (QJ) {
+#pragma unroll
+    for (int k = 0; k < SR; ++k) sr[k] = *reinterpret_cast<const float4*>(a.proj + (SR * ib + k) * D + j4);
+  }
 
   float M = M_INIT;
 #pragma unroll
@@ -806,7 +939,23 @@ __global__ __launch_bounds__(MergeGeo<D>::NT) void mfma_merge_kernel(MfmaArgs a,
   }
   ys[grp][d] = acc;
   xs[grp][d] = acco;
+  if constexpr (QJ) {
+    const int i = tid % QM, q = tid / QM;
+    float u = 0.f;
+    for (int p = q; p < a.ncw; p += UG) {
+      const float wp = wsh[p], x = pp[p * pst + 4 + D + i];
+      u = fmaf(wp, wp != 0.f ? x : 0.f, u);
+    }
+    us[q][i] = u;
+  }
   __syncthreads();
+  if constexpr (QJ)
+    if (tid >= D && tid < D + QM) {
+      float u = 0.f;
+#pragma unroll
+      for (int q = 0; q < UG; ++q) u += us[q][tid - D];
+      yt[tid] = u * (SQRT_HALF_PI_M / D);
+    }
   if (tid < D) {
     float y = 0.f;
 #pragma unroll
@@ -824,6 +973,16 @@ __global__ __launch_bounds__(MergeGeo<D>::NT) void mfma_merge_kernel(MfmaArgs a,
       o.z = fmaf(y, rr[k].z, o.z);
       o.w = fmaf(y, rr[k].w, o.w);
     }
+    if constexpr (QJ) {
+#pragma unroll
+      for (int k = 0; k < SR; ++k) {
+        const float u = yt[D + SR * ib + k];
+        o.x = fmaf(u, sr[k].x, o.x);
+        o.y = fmaf(u, sr[k].y, o.y);
+        o.z = fmaf(u, sr[k].z, o.z);
+        o.w = fmaf(u, sr[k].w, o.w);
+      }
+    }
     *reinterpret_cast<float4*>(&red[ib][j4]) = o;
   }
   __syncthreads();
@@ -837,46 +996,47 @@ __global__ __launch_bounds__(MergeGeo<D>::NT) void mfma_merge_kernel(MfmaArgs a,
   }
 }
 
-template <int D, int GC, int KK>
+template <int D, int GC, int KK, bool QJ>
 static void launch_k(const MfmaArgs& a, hipStream_t s) {
   using G_ = KGeo<D, KK>;
+  using L_ = Lds<D, GC, QJ>;
   MfmaArgs x = a;
   const int vt = (1 << (2 * a.vbh)) * TROW + (a.vfrac ? (1 << (2 * a.vbl)) * TROW : 0);
-  x.tail = G_::TABS + vt > Lds<D, GC>::cmb ? G_::TABS + vt : Lds<D, GC>::cmb;
-  const int lds = x.tail + Lds<D, GC>::end;
+  x.tail = G_::TABS + vt > L_::cmb ? G_::TABS + vt : L_::cmb;
+  const int lds = x.tail + L_::end;
   const dim3 grid(a.ncw + a.nfw, a.hkv * a.gsub, a.batch);
   if (a.vfrac)
-    hipLaunchKernelGGL((mfma_decode_kernel<D, GC, KK, true>), grid, dim3(MTH), lds, s, x);
+    hipLaunchKernelGGL((mfma_decode_kernel<D, GC, KK, true, QJ>), grid, dim3(MTH), lds, s, x);
   else
-    hipLaunchKernelGGL((mfma_decode_kernel<D, GC, KK, false>), grid, dim3(MTH), lds, s, x);
+    hipLaunchKernelGGL((mfma_decode_kernel<D, GC, KK, false, QJ>), grid, dim3(MTH), lds, s, x);
 }
 
-template <int D, int KK>
+template <int D, int KK, bool QJ>
 static void launch_g(const MfmaArgs& a, hipStream_t s) {
   if (a.g <= 4)
-    launch_k<D, 4, KK>(a, s);
+    launch_k<D, 4, KK, QJ>(a, s);
   else
-    launch_k<D, 8, KK>(a, s);
+    launch_k<D, 8, KK, QJ>(a, s);
 }
 
 // kk: key width kind (KGeo)
-template <int D>
+template <int D, bool QJ>
 int launch_mfma(const MfmaArgs& a, int kk, hipStream_t s) {
   switch (kk) {
-    case 2: launch_g<D, 2>(a, s); break;
-    case 3: launch_g<D, 3>(a, s); break;
-    case 4: launch_g<D, 4>(a, s); break;
+    case 2: launch_g<D, 2, QJ>(a, s); break;
+    case 3: launch_g<D, 3, QJ>(a, s); break;
+    case 4: launch_g<D, 4, QJ>(a, s); break;
     case 5:
-      if constexpr (D != 96) launch_g<D, 5>(a, s);
+      if constexpr (D != 96) launch_g<D, 5, QJ>(a, s);
       break;
     case 7:
-      if constexpr (D != 96) launch_g<D, 7>(a, s);
+      if constexpr (D != 96) launch_g<D, 7, QJ>(a, s);
       break;
     default: return -1;
   }
   const int np = a.ncw + a.nfw;
   constexpr int round = MergeGeo<D>::PG * MergeGeo<D>::MB;
-  hipLaunchKernelGGL((mfma_merge_kernel<D>), dim3(a.hq, a.batch), dim3(MergeGeo<D>::NT),
+  hipLaunchKernelGGL((mfma_merge_kernel<D, QJ>), dim3(a.hq, a.batch), dim3(MergeGeo<D>::NT),
                      (np + round - 1) / round * round * 4, s, a, np);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }

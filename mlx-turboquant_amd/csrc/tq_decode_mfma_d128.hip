@@ -4,6 +4,6 @@
 
 namespace tq {
 
-int launch_mfma_d128(const MfmaArgs& a, int kk, hipStream_t s) { return mk::launch_mfma<128>(a, kk, s); }
+int launch_mfma_d128(const MfmaArgs& a, int kk, hipStream_t s) { return mk::launch_mfma<128, false>(a, kk, s); }
 
 }  // namespace tq

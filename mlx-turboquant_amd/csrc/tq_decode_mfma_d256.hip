@@ -4,6 +4,6 @@
 
 namespace tq {
 
-int launch_mfma_d256(const MfmaArgs& a, int kk, hipStream_t s) { return mk::launch_mfma<256>(a, kk, s); }
+int launch_mfma_d256(const MfmaArgs& a, int kk, hipStream_t s) { return mk::launch_mfma<256, false>(a, kk, s); }
 
 }  // namespace tq

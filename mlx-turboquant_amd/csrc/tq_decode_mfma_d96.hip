@@ -4,6 +4,6 @@
 
 namespace tq {
 
-int launch_mfma_d96(const MfmaArgs& a, int kk, hipStream_t s) { return mk::launch_mfma<96>(a, kk, s); }
+int launch_mfma_d96(const MfmaArgs& a, int kk, hipStream_t s) { return mk::launch_mfma<96, false>(a, kk, s); }
 
 }  // namespace tq

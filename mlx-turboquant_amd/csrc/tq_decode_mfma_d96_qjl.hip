@@ -1,0 +1,10 @@
+// head_dim 96 instantiations of the decode kernels of tq_decode_mfma.h with a
+// 32-projection QJL sketch.
+
+#include "tq_decode_mfma.h"
+
+namespace tq {
+
+int launch_mfma_d96_qjl(const MfmaArgs& a, int kk, hipStream_t s) { return mk::launch_mfma<96, true>(a, kk, s); }
+
+}  // namespace tq

@@ -151,3 +151,28 @@ def test_mfma_graph_replays():
         torch.cuda.synchronize()
         assert torch.equal(out, ref)
         assert torch.equal(c.attend(q), ref)
+
+
+@pytest.mark.parametrize("D,kb,vb,m,G,T,dt", [
+    (64, 4, 2, 32, 4, 1500, torch.bfloat16), (64, 3.5, 2.5, 7, 7, 300, torch.float16), (96, 3, 3, 32, 1, 5000, torch.float16),
+    (128, 3, 3, 32, 4, 700, torch.bfloat16), (128, 4, 3.5, 20, 8, 9000, torch.float16), (128, 4, 2, 32, 5, 1000, torch.float16),
+    (256, 4, 3, 32, 2, 1500, torch.bfloat16), (256, 2, 2, 32, 10, 400, torch.float16)])
+def test_mfma_sketch(D, kb, vb, m, G, T, dt):
+    """The two terms of a sketch of at most 32 projections."""
+    k, v = _kv(1, 2, T, D, seed=T + D)
+    c, o = _caches(dict(head_dim=D, num_kv_heads=2, key_bits=kb, value_bits=vb, residual_window=64, fp16_sink_size=16,
+                        qjl_correction=True, qjl_n_proj=m), k, v, dt)
+    q = np.random.RandomState(G).randn(1, 2 * G, 1, D).astype(np.float16)
+    _check(c, o, q, f"QJL d{D} K{kb}/V{vb} m={m} G={G} T={T}")
+
+
+def test_mfma_sketch_gammas_past_the_norms():
+    """Residual norms far above (and below) the value norms, as a loaded state
+    may hold: the weights' exponent follows the larger of the two."""
+    k, v = _kv(1, 2, 900, 64, seed=5)
+    c, o = _caches(dict(head_dim=64, num_kv_heads=2, residual_window=64, qjl_correction=True, qjl_n_proj=32), k, v,
+                   torch.float16)
+    q = np.random.RandomState(3).randn(1, 8, 1, 64).astype(np.float16)
+    for f in (3e4, 1e-4):
+        c._vstore.gamma.mul_(f)
+        _check(c, o, q, f"gamma x{f}")
