@@ -172,6 +172,14 @@ int tq_pack_codes(const uint8_t* idx, int64_t n_rows, int32_t d, int32_t bits,
 int tq_unpack_codes(const uint8_t* packed, int64_t n_rows, int32_t d, int32_t bits,
                     uint8_t* idx, void* stream);
 
+/* Sketch sign rows (m projections in [1, 256], LSB first, row_bytes a multiple
+ * of 4 in [m / 8, 32], 4-byte aligned) to n_rows x m bytes of 0 / 1, and back
+ * (any non-zero byte is a set sign; bits past m are 0). */
+int tq_unpack_signs(const uint8_t* rows, int64_t n_rows, int32_t m, int32_t row_bytes,
+                    uint8_t* signs, void* stream);
+int tq_pack_signs(const uint8_t* signs, int64_t n_rows, int32_t m, int32_t row_bytes,
+                  uint8_t* rows, void* stream);
+
 /* idx = #{k : y > boundaries[k]} for float32 y (codebook.py:203-225). */
 int tq_quantize_scalar(const float* y, int64_t n, const float* boundaries,
                        int32_t n_boundaries, uint8_t* idx, void* stream);

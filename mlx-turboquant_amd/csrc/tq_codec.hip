@@ -714,6 +714,79 @@ __global__ void unpack_kernel(const uint8_t* __restrict__ in, int64_t n_rows, in
   idx[e] = (uint8_t)(v & ((1u << bits) - 1u));
 }
 
+// Sign rows (m projections, LSB first, rb bytes a row, rb a multiple of 4) to
+// one bool byte per projection and back. Torch operators did both through int32
+// intermediates of 32 times the packed size (65,536 vectors, 128 projections,
+// quantize and dequantize: 226 -> 92 us a pass). Bound by HBM: each bool byte and packed
+// dword moves once, a thread takes 16 projections of one row (unpack) or one
+// packed dword (pack); VEC (m and the bool rows multiples of 16 bytes) moves
+// them 16 bytes at a time. Grids are capped and walked with a stride.
+template <bool VEC>
+__global__ __launch_bounds__(256) void unpack_signs_kernel(const uint8_t* __restrict__ in, int64_t n, int m, int rb,
+                                                           uint8_t* __restrict__ out) {
+  const int cpr = (m + 15) / 16;  // 16-projection pieces per row
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n * cpr; i += (int64_t)gridDim.x * 256) {
+    const int64_t row = i / cpr;
+    const int c = (int)(i - row * cpr);
+    const uint32_t w = *reinterpret_cast<const uint16_t*>(in + row * rb + 2 * c);
+    uint8_t* o = out + row * m + 16 * c;
+    if constexpr (VEC) {
+      // nibble b3..b0 to four bytes: the multiplier's terms never carry
+      uint4 v;
+      v.x = ((w & 15u) * 0x00204081u) & 0x01010101u;
+      v.y = ((w >> 4 & 15u) * 0x00204081u) & 0x01010101u;
+      v.z = ((w >> 8 & 15u) * 0x00204081u) & 0x01010101u;
+      v.w = ((w >> 12) * 0x00204081u) & 0x01010101u;
+      *reinterpret_cast<uint4*>(o) = v;
+    } else {
+      for (int j = 0; j < min(16, m - 16 * c); ++j) o[j] = (uint8_t)(w >> j & 1u);
+    }
+  }
+}
+
+// any non-zero byte is a set sign; projections past m are 0
+template <bool VEC>
+__global__ __launch_bounds__(256) void pack_signs_kernel(const uint8_t* __restrict__ in, int64_t n, int m, int rb,
+                                                         uint8_t* __restrict__ out) {
+  const int wpr = rb / 4;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n * wpr; i += (int64_t)gridDim.x * 256) {
+    const int64_t row = i / wpr;
+    const int c = (int)(i - row * wpr);
+    const uint8_t* p = in + row * m + 32 * c;
+    uint32_t r = 0;
+    if constexpr (VEC) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (32 * c + 16 * h >= m) break;
+        const uint4 v = *reinterpret_cast<const uint4*>(p + 16 * h);
+        const uint32_t x[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t nz = (((x[j] & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | x[j]) >> 7 & 0x01010101u;
+          r |= (nz * 0x01020408u >> 24 & 15u) << (16 * h + 4 * j);  // (bytes to a nibble, no carries)
+        }
+      }
+    } else {
+      for (int j = 0; j < min(32, m - 32 * c); ++j) r |= (p[j] ? 1u : 0u) << j;
+    }
+    reinterpret_cast<uint32_t*>(out + row * rb)[c] = r;
+  }
+}
+
+static int check_signs(const char* what, const void* in, int64_t n, int32_t m, int32_t rb, const void* out) {
+  if (n < 0) return set_error(TQ_ERR_INVALID, "%s: n_rows < 0", what);
+  if (m < 1 || m > 256 || rb % 4 != 0 || rb < (m + 7) / 8 || rb > 32)
+    return set_error(TQ_ERR_INVALID, "%s: %d projections in rows of %d bytes", what, m, rb);
+  if (n > ((int64_t)1 << 40)) return set_error(TQ_ERR_UNSUPPORTED, "%s: too many rows", what);
+  if (n && (!in || !out)) return set_error(TQ_ERR_INVALID, "%s: NULL pointer", what);
+  return TQ_OK;
+}
+
+static dim3 signs_grid(int64_t threads) {
+  const int64_t g = (threads + 255) / 256;
+  return dim3((unsigned)(g < 16384 ? g : 16384));
+}
+
 __global__ void quantize_scalar_kernel(const float* __restrict__ y, int64_t n,
                                        const float* __restrict__ b, int nb, uint8_t* __restrict__ idx) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1163,6 +1236,28 @@ int tq_unpack_codes(const uint8_t* packed, int64_t n_rows, int32_t d, int32_t bi
   hipLaunchKernelGGL(unpack_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
                      static_cast<hipStream_t>(stream), packed, n_rows, d, bits, idx);
   TQ_LAUNCH_CHECK("tq_unpack_codes");
+  return TQ_OK;
+}
+
+int tq_unpack_signs(const uint8_t* rows, int64_t n_rows, int32_t m, int32_t row_bytes, uint8_t* signs, void* stream) {
+  const int rc = check_signs("unpack_signs", rows, n_rows, m, row_bytes, signs);
+  if (rc != TQ_OK || n_rows == 0) return rc;
+  if (!aligned4(rows)) return set_error(TQ_ERR_INVALID, "unpack_signs: rows must be 4-byte aligned");
+  const bool vec = m % 16 == 0 && (reinterpret_cast<uintptr_t>(signs) & 15) == 0;
+  hipLaunchKernelGGL(vec ? unpack_signs_kernel<true> : unpack_signs_kernel<false>, signs_grid(n_rows * ((m + 15) / 16)),
+                     dim3(256), 0, static_cast<hipStream_t>(stream), rows, n_rows, m, row_bytes, signs);
+  TQ_LAUNCH_CHECK("tq_unpack_signs");
+  return TQ_OK;
+}
+
+int tq_pack_signs(const uint8_t* signs, int64_t n_rows, int32_t m, int32_t row_bytes, uint8_t* rows, void* stream) {
+  const int rc = check_signs("pack_signs", signs, n_rows, m, row_bytes, rows);
+  if (rc != TQ_OK || n_rows == 0) return rc;
+  if (!aligned4(rows)) return set_error(TQ_ERR_INVALID, "pack_signs: rows must be 4-byte aligned");
+  const bool vec = m % 16 == 0 && (reinterpret_cast<uintptr_t>(signs) & 15) == 0;
+  hipLaunchKernelGGL(vec ? pack_signs_kernel<true> : pack_signs_kernel<false>, signs_grid(n_rows * (row_bytes / 4)),
+                     dim3(256), 0, static_cast<hipStream_t>(stream), signs, n_rows, m, row_bytes, rows);
+  TQ_LAUNCH_CHECK("tq_pack_signs");
   return TQ_OK;
 }
 

@@ -128,26 +128,28 @@ class PackedStore:
         self.cap = 0
         self.codes_hi = self.codes_lo = self.norms = self.signs = self.gamma = None
 
-    def _alloc(self, cap: int):
+    def _alloc(self, cap: int, zero: bool = True):
         c, dev, B, H = self.codec, self.codec.device, self.batch, self.heads
         u8 = dict(dtype=torch.uint8, device=dev)
         f32 = dict(dtype=torch.float32, device=dev)
+        make = torch.zeros if zero else torch.empty
         new = {
-            "codes_hi": torch.zeros(B, H, cap, c.row_hi, **u8),
-            "codes_lo": torch.zeros(B, H, cap, c.row_lo, **u8) if c.fractional else None,
-            "norms": torch.zeros(B, H, cap, **f32),
-            "signs": torch.zeros(B, H, cap, c.row_sign, **u8) if self.qjl else None,
-            "gamma": torch.zeros(B, H, cap, **f32) if self.qjl else None,
+            "codes_hi": make(B, H, cap, c.row_hi, **u8),
+            "codes_lo": make(B, H, cap, c.row_lo, **u8) if c.fractional else None,
+            "norms": make(B, H, cap, **f32),
+            "signs": make(B, H, cap, c.row_sign, **u8) if self.qjl else None,
+            "gamma": make(B, H, cap, **f32) if self.qjl else None,
         }
         return new
 
-    def reserve(self, n_tokens: int, keep: int) -> None:
-        """Ensure capacity for ``n_tokens``; copies the first ``keep`` tokens."""
+    def reserve(self, n_tokens: int, keep: int, zero: bool = True) -> None:
+        """Ensure capacity for ``n_tokens``; copies the first ``keep`` tokens
+        (``zero``: the other ones are cleared)."""
         if n_tokens <= self.cap:
             return
         cap = max(n_tokens, self.cap + self.cap // 2, self.GROW)
         cap = (cap + self.GROW - 1) // self.GROW * self.GROW
-        new = self._alloc(cap)
+        new = self._alloc(cap, zero)
         for name, t in new.items():
             old = getattr(self, name)
             if t is not None and old is not None and keep > 0:

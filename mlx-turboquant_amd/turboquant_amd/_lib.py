@@ -90,6 +90,8 @@ SIGNATURES = {
     "tq_dequantize": (_i32, [_PC, _PS, _PSp, _p, _i64, _i32, _p]),
     "tq_pack_codes": (_i32, [_p, _i64, _i32, _i32, _p, _p]),
     "tq_unpack_codes": (_i32, [_p, _i64, _i32, _i32, _p, _p]),
+    "tq_unpack_signs": (_i32, [_p, _i64, _i32, _i32, _p, _p]),
+    "tq_pack_signs": (_i32, [_p, _i64, _i32, _i32, _p, _p]),
     "tq_quantize_scalar": (_i32, [_p, _i64, _p, _i32, _p, _p]),
     "tq_decode_workspace_bytes": (ctypes.c_size_t, [_PC, _PA]),
     "tq_attention_workspace_bytes": (ctypes.c_size_t, [_PC, _PC, _PA]),

@@ -10,7 +10,7 @@ from dataclasses import dataclass
 
 import torch
 
-from . import _codec
+from . import _codec, _lib
 from .qjl import check_count as check_qjl_count
 from .rotation import DEFAULT_SEED
 
@@ -35,17 +35,25 @@ def _flat(x: torch.Tensor, d: int) -> tuple[torch.Tensor, tuple]:
     return x.reshape(1, 1, -1, d).contiguous(), lead
 
 
-def _unpack_signs(bits_u8: torch.Tensor, m: int) -> torch.Tensor:
-    """The first m sign bits of LSB-first rows (the rows may hold padding)."""
-    shifts = torch.arange(8, device=bits_u8.device, dtype=torch.uint8)
-    bits = ((bits_u8[..., :, None] >> shifts) & 1).reshape(*bits_u8.shape[:-1], bits_u8.shape[-1] * 8)
-    return bits[..., :m].bool()
+def _unpack_signs(rows: torch.Tensor, m: int) -> torch.Tensor:
+    """(n, m) bool: the first m sign bits of LSB-first rows (n, row bytes),
+    contiguous (the rows may hold padding)."""
+    out = torch.empty(rows.shape[0], m, dtype=torch.bool, device=rows.device)
+    _lib.check(_lib.load().tq_unpack_signs(rows.data_ptr(), rows.shape[0], m, rows.shape[1], out.data_ptr(),
+                                           _lib.stream_ptr(rows.device)), "unpack_signs")
+    return out
 
 
 def _pack_signs(signs: torch.Tensor, mp: int) -> torch.Tensor:
     """LSB-first rows of mp bits from (..., m) signs, m <= mp (the projections
     past m are zero rows of S: their bits are never used)."""
     m = signs.shape[-1]
+    if signs.dtype == torch.bool and signs.is_cuda:
+        s = signs.contiguous()
+        out = torch.empty(*s.shape[:-1], mp // 8, dtype=torch.uint8, device=s.device)
+        _lib.check(_lib.load().tq_pack_signs(s.data_ptr(), s.numel() // m, m, mp // 8, out.data_ptr(),
+                                             _lib.stream_ptr(s.device)), "pack_signs")
+        return out
     if mp > m:
         signs = torch.cat([signs, torch.zeros(*signs.shape[:-1], mp - m, dtype=signs.dtype, device=signs.device)], -1)
     w = (1 << torch.arange(8, device=signs.device, dtype=torch.int32))
@@ -85,7 +93,7 @@ class TurboQuantMSE:
         flat, lead = _flat(x, self.d)
         n = flat.shape[2]
         store = _codec.PackedStore(codec, 1, 1, qjl=qjl_m > 0)
-        store.reserve(max(n, 1), 0)
+        store.reserve(max(n, 1), 0, zero=False)  # every row up to n is written, none past it is read
         _codec.compress_into(codec, flat, 0, n, store, 0)
         return codec, store, lead, n
 
