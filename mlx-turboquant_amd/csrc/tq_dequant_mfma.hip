@@ -24,6 +24,7 @@
 // against float64 2.0e-7 -> 1.1e-7.
 
 #include <algorithm>
+#include <atomic>
 
 #include "tq_codec.h"
 
@@ -232,11 +233,15 @@ __global__ __launch_bounds__(2 * D) void dequant_mfma_kernel(DequantArgs a, int 
 
 template <int D, int MK>
 int launch_dm(const DequantArgs& a, hipStream_t s) {
-  static int occ = 0;  // workgroups per CU at the largest table (same for every gfx950 device)
+  // workgroups per CU at the largest table (the same on every gfx950 device)
+  static std::atomic<int> known{0};
   const int lds = (1 << (2 * a.bits_hi)) * TROW + (a.split < D ? (1 << (2 * a.bits_lo)) * TROW : 0);
-  if (occ == 0 && hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, dequant_mfma_kernel<D, MK>, 2 * D, 256 * TROW) !=
-                      hipSuccess)
-    occ = 1;
+  int occ = known.load(std::memory_order_relaxed);
+  if (occ == 0) {
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, dequant_mfma_kernel<D, MK>, 2 * D, 256 * TROW) != hipSuccess)
+      occ = 1;
+    known.store(occ, std::memory_order_relaxed);
+  }
   int dev = 0, cus = 256;
   if (hipGetDevice(&dev) == hipSuccess &&
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
