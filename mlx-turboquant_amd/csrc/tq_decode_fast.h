@@ -238,16 +238,18 @@ struct DenseArgs {
 
 constexpr int DENSE_WAVES = 4;  // waves per workgroup of the dense kernel
 
-// Power of two 2^qe of one query head for the fp16 query operands of the
-// K4/V2 and uniform-batch kernels (s = qscale, the scores' scale): a head
-// with s ||q|| above `hi` is scaled down to at most `hi`; a head with
-// s ||q|| below `lo` (the fp16 remainders of its rotated coordinates s (R q)_j
-// would go subnormal) is scaled up with both 2^-qe ||q|| and 2^-qe s ||q||
-// at most `hi`; otherwise 0. The scores of the head are multiplied by 2^qe.
+// Power of two 2^qe of one query head for the fp16 query operands of the decode
+// kernels (s = qscale, the scores' scale; the operands are q itself and s (R
+// q)): a head with s ||q|| above `hi` (16384) or ||q||, which bounds the
+// elements, above fp16's range is scaled down to those; a head with s ||q|| below
+// `lo` (the fp16 remainders of its rotated coordinates s (R q)_j would go
+// subnormal) is scaled up with both 2^-qe ||q|| and 2^-qe s ||q|| at most `hi`;
+// otherwise 0. The scores of the head are multiplied by 2^qe.
 __device__ inline int query_exponent(float qnorm, float qscale, float hi, float lo) {
-  const float qn = qnorm * qscale;
-  if (qn > hi) return (int)ceilf(log2f(qn / hi));
-  if (qn < lo && qnorm > 0.f) return max(min((int)ceilf(log2f(qnorm * fmaxf(qscale, 1.f) / hi)), 0), -100);
+  const float top = qnorm * fmaxf(fabsf(qscale), 0.2502f);  // hi / 0.2502 = 65,484
+  if (top > hi) return (int)ceilf(log2f(top / hi));
+  if (qnorm * qscale < lo && qnorm > 0.f)
+    return max(min((int)ceilf(log2f(qnorm * fmaxf(fabsf(qscale), 1.f) / hi)), 0), -100);
   return 0;
 }
 

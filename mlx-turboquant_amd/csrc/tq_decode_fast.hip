@@ -78,7 +78,8 @@ constexpr float PV_LIMIT = 32768.f;
 // block's, the rescale margin) stay below PV_LIMIT unless their norms grow
 constexpr float PV_SET = 2048.f;
 // |scale * (R q)_j| <= scale * ||q|| must stay below this for the fp16 query
-// operands; larger queries are scaled by a power of two per head.
+// operands (and |q_i| <= ||q|| in fp16's range: query_exponent); larger queries
+// are scaled by a power of two per head.
 constexpr float Q_LIMIT = 16384.f;
 // scale * ||q|| below this: the head is scaled up by a power of two (keeps
 // the fp16 remainders of the rotated query normal)
@@ -807,8 +808,8 @@ __global__ __launch_bounds__(FT) void decode_partials_kernel(FastArgs a) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) ss = fmaf(x[kb][i], x[kb][i], ss);
       // the query norm of head r (4 lanes hold its 128 dims) bounds every
-      // rotated coordinate: the power of two that keeps the operands in fp16
-      // range
+      // coordinate, rotated or not: the power of two that keeps the operands
+      // in fp16 range
       ss = rows_sum(ss);
       const int qe = query_exponent(sqrtf(ss), a.qscale, Q_LIMIT, Q_LOW);  // lanes r: head r
       const float qdown = __builtin_amdgcn_ldexpf(1.f, -qe);

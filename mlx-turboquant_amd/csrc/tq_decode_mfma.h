@@ -79,9 +79,9 @@ constexpr int MW = MFMA_WAVES;
 constexpr int MTH = MW * 64;   // threads
 constexpr float M_INIT = uk::M_INIT;
 constexpr int TROW = 128;      // bytes per table entry: 16 replicas
-// The tables hold CSC times the centroids, and queries are scaled up to QLOW <=
-// scale ||q||: the fp16 remainders of both stay normal (unscaled, a remainder of
-// 0.1 is a multiple of 6e-8).
+// The tables hold CSC times the centroids, and queries are scaled to QLOW <=
+// ||q|| <= Q_LIMIT: the fp16 remainders of both stay normal (unscaled, a remainder
+// of 0.1 is a multiple of 6e-8) and no element leaves the fp16 range.
 constexpr float CSC = 256.f;
 constexpr float QLOW = 4096.f;
 
@@ -177,7 +177,7 @@ struct Blk {
 };
 
 // VF: the values' width is fractional (two tables, rows of two widths); QJ: the
-// terms of a 32-projection QJL sketch (qjl.py:70-94). Key term: S (scale q) is
+// terms of a 32-projection QJL sketch (qjl.py:70-94). Key term: S q is
 // computed at the query rotation (S's rows as two more tiles), its fp16 high
 // part / remainder columns meet one operand of 16 tokens x 32 signs (+-1, exact)
 // per tile: one MFMA. Value term: u = sum_t p_t gamma_t z_t accumulates in two
@@ -379,7 +379,25 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
     for (int i = 0; i < 8; ++i) ss = fmaf(x[i], x[i], ss);
 #pragma unroll
     for (int k = 1; k < LPH; k *= 2) ss += __shfl_xor(ss, k);
-    const int qe = query_exponent(sqrtf(ss), a.qscale, uk::Q_LIMIT, QLOW);
+    float qn = sqrtf(ss);
+    if (__builtin_amdgcn_ballot_w64(qact && !(ss > 1e-30f && ss < 1e30f)) != 0) {
+      // (a zero query, or one whose squares leave float32: the norm of q 2^-e)
+      float mx = 0.f, s2 = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) mx = fmaxf(mx, fabsf(x[i]));
+#pragma unroll
+      for (int k = 1; k < LPH; k *= 2) mx = fmaxf(mx, __shfl_xor(mx, k));
+      const int e = __builtin_amdgcn_frexp_expf(mx);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float y = __builtin_amdgcn_ldexpf(x[i], -e);
+        s2 = fmaf(y, y, s2);
+      }
+#pragma unroll
+      for (int k = 1; k < LPH; k *= 2) s2 += __shfl_xor(s2, k);
+      qn = fminf(__builtin_amdgcn_ldexpf(sqrtf(s2), e), 3.4e38f);
+    }
+    const int qe = query_exponent(qn, 1.f, uk::Q_LIMIT, QLOW);
     const float qdown = __builtin_amdgcn_ldexpf(1.f, -qe);
     if (qact) {
       uint8_t* d = tail + L_::qsrc + qh * 3 * L_::QS + 16 * qi;
@@ -413,8 +431,9 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
   const float qe_scale = *reinterpret_cast<const float*>(tail + L_::qex + 4 * hd);
   uint8_t* qop = tail + L_::qop;
   if (packed) {
-    // rotated query, D[h][n] = sum_i q[h][i] R[j0 + n][i], written (times
-    // qscale) as fp16 high part / remainder rows [head][part][D]
+    // rotated query, D[h][n] = sum_i q[h][i] R[j0 + n][i], written as fp16 high
+    // part / remainder rows [head][part][D] (the scores take qscale: a small
+    // one here would push the remainders below fp16's normal range)
     const uint8_t* qs = tail + L_::qsrc + min(r, a.g - 1) * 3 * L_::QS + 16 * q4;
     for (int jt = w; jt < U; jt += MW) {
       if (jt != w) load_rot(jt);
@@ -430,7 +449,7 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
       for (int i = 0; i < 4; ++i) {
         const int h = 4 * q4 + i;
         if (h < a.g && h < GC) {
-          const float v = (dq[i] + dl[i]) * a.qscale;
+          const float v = dq[i] + dl[i];
           const _Float16 hi = (_Float16)v, lo = (_Float16)(v - (float)hi);
           uint8_t* d = qop + (h * 2) * L_::QS + 2 * (16 * jt + r);
           *reinterpret_cast<_Float16*>(d) = hi;
@@ -439,7 +458,7 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
       }
     }
     if constexpr (QJ) {
-      // S (q 2^-qe) qscale / SQD, tiles U and U + 1 of the same waves' sequence
+      // S (q 2^-qe) / SQD, tiles U and U + 1 of the same waves' sequence
       for (int jt = w; jt < U + QM / 16; jt += MW) {
         if (jt < U) continue;
         const int p = 16 * (jt - U) + r;
@@ -463,7 +482,7 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
         for (int i = 0; i < 4; ++i) {
           const int h = 4 * q4 + i;
           if (h < a.g && h < GC) {
-            const float v = (dq[i] + dl[i]) * (a.qscale / SQD);
+            const float v = (dq[i] + dl[i]) * (1.f / SQD);
             const _Float16 hi = (_Float16)v, lo = (_Float16)(v - (float)hi);
             uint8_t* d = tail + L_::sqo + h * 2 * SQS + 2 * p;
             *reinterpret_cast<_Float16*>(d) = hi;
@@ -599,7 +618,7 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
     const uint32_t cp = (uint32_t)r * 8;  // replica of this lane
     const uint32_t cpv = cp + G_::TABS + (vlo ? (1u << (2 * a.vbh)) * TROW : 0u);
     const uint32_t vbw = 2 * vb;  // bits per field
-    const float ks = qe_scale * (1.f / CSC);
+    const float ks = qe_scale * a.qscale * (1.f / CSC);
     float* nst = reinterpret_cast<float*>(tail + L_::nst) + w * (QJ ? 128 : 64);  // [key norms 32][value norms 32][gammas]
     half8 qz;  // S q, k-slot (q4, e) = projection 8 q4 + e
     if constexpr (QJ) qz = *reinterpret_cast<const half8*>(tail + L_::sqo + (hd * 2 + (lo_part ? 1 : 0)) * SQS + 16 * q4);
@@ -656,7 +675,7 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
             z[f] = 0x3C003C00u | ((nz << (15 - 2 * f)) & 0x8000u) | ((nz << (30 - 2 * f)) & 0x80000000u);
           sz[t] = mfma(as_h8(z), qz, f4{0.f, 0.f, 0.f, 0.f});
         }
-        const float zs = qe_scale * (SQD * SQRT_HALF_PI_M / D);
+        const float zs = qe_scale * a.qscale * (SQD * SQRT_HALF_PI_M / D);
         float fz[NS], sq[NS];
 #pragma unroll
         for (int i = 0; i < NS; ++i) fz[i] = gk[i] * zs;

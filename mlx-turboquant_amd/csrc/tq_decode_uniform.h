@@ -104,7 +104,8 @@ constexpr float PV_LIMIT = 32768.f;
 // block's, the rescale margin) stay below PV_LIMIT unless their norms grow
 constexpr float PV_SET = 2048.f;
 // |scale * (R q)_j| <= scale * ||q|| must stay below this for the fp16 query
-// operands; larger queries are scaled by a power of two per head.
+// operands (and |q_i| <= ||q|| in fp16's range: query_exponent); larger queries
+// are scaled by a power of two per head.
 constexpr float Q_LIMIT = 16384.f;
 // scale * ||q|| below this: the head is scaled up by a power of two (keeps
 // the fp16 remainders of the rotated query normal)
@@ -563,7 +564,7 @@ __global__ __launch_bounds__(FT) void uniform_decode_kernel(UniformArgs a) {
 
   // q rows as MFMA A operands (row r = query head min(r, G-1), k-slots = dims
   // 32*kb + 8*q4 ..): fp16 high part and remainder of q 2^-qe, the power of
-  // two 2^qe of the head keeping scale * |R q| <= scale * ||q|| below Q_LIMIT
+  // two 2^qe of the head keeping q in fp16's range, scale * R q below Q_LIMIT
   // and, for small queries, the rotated remainders normal
   half8 qo_hi[4], qo_lo[4];
   float qe_scale = 1.f;  // 2^qe of this lane's column head: multiplies its scores
@@ -585,8 +586,8 @@ __global__ __launch_bounds__(FT) void uniform_decode_kernel(UniformArgs a) {
         }
       }
       ss = rows_sum(ss);
-      // scale * ||q|| in [Q_LOW, Q_LIMIT] (query_exponent 0) for every head:
-      // one unsigned range test of the float bits
+      // scale * ||q|| in [Q_LOW, Q_LIMIT] for every head (the elements are fp16
+      // already): one unsigned range test of the float bits
       q_exact = __builtin_amdgcn_ballot_w64(__float_as_uint(sqrtf(ss) * a.qscale) - __float_as_uint(Q_LOW) >
                                             __float_as_uint(Q_LIMIT) - __float_as_uint(Q_LOW)) == 0;
       if (q_exact) {
