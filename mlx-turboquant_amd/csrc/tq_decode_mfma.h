@@ -866,7 +866,7 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
       sr = fmaf(sc, cms[(ww * GC + h) * L_::CMS + j], sr);
       Ls = fmaf(sc, st.y, Ls);
     }
-    part[h * PSD + 4 + j] = Ls > 0.f ? sr / Ls : 0.f;
+    part[h * PSD + 4 + j] = Ls == 0.f ? 0.f : sr / Ls;
     if (j == 0) *reinterpret_cast<float4*>(part + h * PSD) = make_float4(M, Ls, 0.f, 0.f);
   }
 }
@@ -876,7 +876,10 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
 // R the value codec's float32 rotation). Grid (hq, batch): a chain of dependent
 // round trips, so everything is requested at once: PG groups of D threads hold
 // MB partials each (64 of them in one round at D <= 128), every wave reads all
-// headers, and thread (4 columns, row block) its D / RB rows of R.
+// headers, and thread (4 columns, row block) its D / RB rows of R. A partial
+// without a weight (L_p = 0) is skipped; one whose sum is NaN (a NaN or +infinite
+// score) is not: the head is then zero, as combine_kernel leaves it, and never
+// the attention over the other tokens.
 template <int D>
 struct MergeGeo {
   static constexpr int PG = D == 256 ? 4 : 8;   // partial groups
@@ -924,10 +927,10 @@ __global__ __launch_bounds__(MergeGeo<D>::NT) void mfma_merge_kernel(MfmaArgs a,
 
   float M = M_INIT;
 #pragma unroll
-  for (int k = 0; k < 4; ++k) M = hd[k].y > 0.f ? fmaxf(M, hd[k].x) : M;  // (repeats of the last header change nothing)
+  for (int k = 0; k < 4; ++k) M = hd[k].y != 0.f ? fmaxf(M, hd[k].x) : M;  // (repeats of the last header change nothing)
   for (int p = 256 + lane; p < np; p += 64) {
     const float2 e = *reinterpret_cast<const float2*>(pp + p * pst);
-    M = e.y > 0.f ? fmaxf(M, e.x) : M;
+    M = e.y != 0.f ? fmaxf(M, e.x) : M;
   }
   M = uk::wave_max(M);
   float ls = 0.f;
@@ -935,7 +938,7 @@ __global__ __launch_bounds__(MergeGeo<D>::NT) void mfma_merge_kernel(MfmaArgs a,
   for (int p = lane, k = 0; p < npr; p += 64, ++k) {
     float2 e = k == 0 ? hd[0] : k == 1 ? hd[1] : k == 2 ? hd[2] : hd[3];
     if (k >= 4 && p < np) e = *reinterpret_cast<const float2*>(pp + p * pst);
-    const float wp = p < np && e.y > 0.f ? fexp2(e.x - M) * e.y : 0.f;
+    const float wp = p < np && e.y != 0.f ? fexp2(e.x - M) * e.y : 0.f;
     if (tid < 64) wsh[p] = wp;
     ls += wp;
   }
@@ -1011,7 +1014,7 @@ __global__ __launch_bounds__(MergeGeo<D>::NT) void mfma_merge_kernel(MfmaArgs a,
     for (int k = 0; k < M_::RB; ++k) s += red[k][tid];
 #pragma unroll
     for (int q = 0; q < PG; ++q) s += xs[q][tid];
-    a.out[((int64_t)b * a.hq + hq) * D + tid] = s * inv;
+    a.out[((int64_t)b * a.hq + hq) * D + tid] = Ls > 0.f ? s * inv : 0.f;
   }
 }
 

@@ -176,3 +176,35 @@ def test_mfma_sketch_gammas_past_the_norms():
     for f in (3e4, 1e-4):
         c._vstore.gamma.mul_(f)
         _check(c, o, q, f"gamma x{f}")
+
+
+@pytest.mark.parametrize("D,kb,vb,G,dt,m", [(64, 4, 2, 4, torch.bfloat16, 0), (128, 3.5, 3, 7, torch.float16, 0),
+                                            (256, 4, 3, 4, torch.bfloat16, 0), (96, 3, 3, 2, torch.float16, 32)])
+@pytest.mark.parametrize("what", ["query NaN", "query inf", "norm NaN", "norm inf", "ring key NaN", "value norm NaN"])
+def test_mfma_non_finite(D, kb, vb, G, dt, m, what):
+    """A NaN in a query, a stored norm or a ring key takes the whole head, not one workgroup's tokens: the general
+    kernel's output (zeros where the weights' sum is NaN), the other heads as without it."""
+    k, v = _kv(1, 2, 3000, D, seed=D)
+    c, _ = _caches(dict(head_dim=D, num_kv_heads=2, key_bits=kb, value_bits=vb, residual_window=64, fp16_sink_size=16,
+                        **(dict(qjl_correction=True, qjl_n_proj=m) if m else {})), k, v, dt)
+    q = to_dev(np.random.RandomState(G).randn(1, 2 * G, 1, D).astype(np.float16))
+    clean = c.attend(q).cpu().numpy()
+    bad = float("inf") if "inf" in what else float("nan")
+    hit = slice(0, G)
+    if "query" in what:
+        q[0, 1, 0, 3] = bad
+        hit = slice(1, 2)
+    elif what.startswith("norm"):
+        c._kstore.norms[0, 0, 1500] = bad
+    elif what.startswith("value"):
+        c._vstore.norms[0, 0, 1500] = bad
+    else:
+        c._res_k[0, 0, (c._res_start + 5) % c._res_cap, 3] = bad
+    assert decode_route(c, q) == 7
+    got, gen = c.attend(q).cpu().numpy(), c.attend(q, general_kernel=True).cpu().numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(gen)) and np.isnan(gen).any() == (what == "value norm NaN")
+    if "NaN" in what:
+        assert not np.nan_to_num(got[:, hit]).any()
+    assert rel_err(np.nan_to_num(got), np.nan_to_num(gen)) < 1e-4
+    rest = np.delete(got, hit, axis=1)
+    assert np.isfinite(rest).all() and np.array_equal(rest, np.delete(clean, hit, axis=1))
