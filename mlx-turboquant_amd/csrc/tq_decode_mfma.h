@@ -520,6 +520,7 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
   float gv[NS], pu[NS];  // the block's value residual norms, weights times them
 
   bool any = false;   // the wave has accumulated a block
+  uint32_t redo = 0;  // columns whose uncompressed tokens are taken again (wave-uniform)
   // running max and sum over the block's scores s, weights times nv to pv; the
   // accumulators follow a raised max (nothing to follow in the first block)
   auto softmax = [&](const float (&s)[NS], const float (&nv)[NS], float (&pv)[NS]) {
@@ -808,6 +809,16 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
         }
       }
     }
+    // Operands in parts and zero k-slots turn an infinite key or value into NaN
+    // where its own products are not (0 times infinity): the columns with a NaN or
+    // an infinite sum
+    float nn = l_run;
+#pragma unroll
+    for (int nb = 0; nb < U; ++nb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) nn = fmaf(acc[nb][i], 0.f, nn);
+    const uint64_t nl = __builtin_amdgcn_ballot_w64(nn != nn);
+    redo = (uint32_t)(nl | nl >> 16 | nl >> 32 | nl >> 48) & 0xFFFFu;
   }
 
   // ---- combine the waves through LDS (the table region); the two fp16 parts
@@ -851,6 +862,51 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
     }
   }
   if (q4 == 0 && writer) *reinterpret_cast<float2*>(cl + (w * GC + hd) * 2) = make_float2(m_run, l_run);
+  if (redo != 0) {
+    // the heads of those columns again: the wave's tokens one at a time in
+    // float32, as in chunk_kernel (never taken with finite tokens and sums)
+    constexpr int DL = (D + 63) / 64;
+    auto elem = [&](const uint16_t* p) {
+      return a.bf ? __uint_as_float((uint32_t)*p << 16) : (float)__builtin_bit_cast(_Float16, *p);
+    };
+    for (int h = 0; h < a.g; ++h) {
+      if ((redo & (TS == 2 ? 0x0101u << h | 0x8080u >> h : 0x0101u << h)) == 0) continue;
+      const uint8_t* qs = tail + L_::qsrc + h * 3 * L_::QS;
+      const float qf = a.qscale * *reinterpret_cast<const float*>(tail + L_::qex + 4 * h);
+      float qv[DL], o[DL], mx = M_INIT, l = 0.f;
+#pragma unroll
+      for (int j = 0; j < DL; ++j) {
+        const int d = lane + 64 * j;
+        float x = 0.f;
+        for (int k = a.bf ? 2 : 1; k >= 0; --k)
+          x += d < D ? elem(reinterpret_cast<const uint16_t*>(qs + k * L_::QS) + d) : 0.f;
+        qv[j] = x * qf;
+        o[j] = 0.f;
+      }
+      for (int pass = 0; pass < 2; ++pass)
+        for (int blk = blk0 + w; blk < blk1; blk += MW)
+          for (int u = blk << 5; u < min((blk + 1) << 5, nfp); ++u) {
+            const uint16_t* kp = token(u, a.sink_k, a.res_k) + lane;
+            float s = 0.f;
+#pragma unroll
+            for (int j = 0; j < DL; ++j) s = lane + 64 * j < D ? fmaf(qv[j], elem(kp + 64 * j), s) : s;
+            s = uk::wave_sum(s);
+            if (pass == 0) {
+              mx = fmaxf(mx, s);
+              continue;
+            }
+            const float p = fexp2(s - mx);
+            l += p;
+            const uint16_t* vp = token(u, a.sink_v, a.res_v) + lane;
+#pragma unroll
+            for (int j = 0; j < DL; ++j) o[j] = lane + 64 * j < D ? fmaf(p, elem(vp + 64 * j), o[j]) : 0.f;
+          }
+#pragma unroll
+      for (int j = 0; j < DL; ++j)
+        if (lane + 64 * j < D) cm[h * L_::CMS + lane + 64 * j] = o[j];
+      if (lane == 0) *reinterpret_cast<float2*>(cl + (w * GC + h) * 2) = make_float2(mx, l);
+    }
+  }
   __syncthreads();
   const float* cms = reinterpret_cast<const float*>(smem);
   for (int e = tid; e < a.g * L_::W; e += MTH) {
@@ -952,8 +1008,8 @@ __global__ __launch_bounds__(MergeGeo<D>::NT) void mfma_merge_kernel(MfmaArgs a,
       const int p = p0 + PG * i + grp;
       const float wp = wsh[p];
       const float v = wp != 0.f ? x[i] : 0.f;  // (empty partials may hold anything)
-      acc = fmaf(p < a.ncw ? wp : 0.f, v, acc);
-      acco = fmaf(p < a.ncw ? 0.f : wp, v, acco);
+      acc = fmaf(wp, p < a.ncw ? v : 0.f, acc);  // (the other space's sum may be infinite)
+      acco = fmaf(wp, p < a.ncw ? 0.f : v, acco);
     }
     p0 += PG * MB;
     if (p0 >= np) break;

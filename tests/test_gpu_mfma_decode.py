@@ -208,3 +208,32 @@ def test_mfma_non_finite(D, kb, vb, G, dt, m, what):
     assert rel_err(np.nan_to_num(got), np.nan_to_num(gen)) < 1e-4
     rest = np.delete(got, hit, axis=1)
     assert np.isfinite(rest).all() and np.array_equal(rest, np.delete(clean, hit, axis=1))
+
+
+@pytest.mark.parametrize("D,G,dt,T", [(64, 4, torch.bfloat16, 2000), (128, 7, torch.float16, 300), (256, 2, torch.float16, 900),
+                                      (96, 8, torch.bfloat16, 700), (64, 12, torch.float16, 200)])
+@pytest.mark.parametrize("what", ["value inf", "value -inf", "key", "both"])
+def test_mfma_infinite_tokens(D, G, dt, T, what):
+    """Infinite elements of uncompressed tokens, in the sink, at the start and at the end of the ring: a value's dim is
+    that infinity and the others stay; a key whose score is -inf has no weight, one of +inf makes the head zero."""
+    k, v = _kv(1, 2, T, D, seed=D)
+    c, _ = _caches(dict(head_dim=D, num_kv_heads=2, residual_window=150, fp16_sink_size=16), k, v, dt)
+    q = to_dev(np.abs(np.random.RandomState(G).randn(1, 2 * G, 1, D)).astype(np.float16))
+    q[0, 2, 0] *= -1  # the other sign of an infinite score
+    inf = float("inf")
+    end = (c._res_start + c._fp16_len - 1) % c._res_cap
+    if what != "key":
+        x = -inf if "-" in what else inf
+        c.sink_values[0, 0, 3, 7] = x
+        c._res_v[0, 1, c._res_start, 0] = x
+        c._res_v[0, 1, end, D - 1] = -x
+    if what in ("key", "both"):
+        c.sink_keys[0, 0, 15, 2] = -inf
+        c._res_k[0, 1, end, D // 2] = -inf
+    assert decode_route(c, q) == 7
+    got, gen = c.attend(q).cpu().numpy(), c.attend(q, general_kernel=True).cpu().numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(gen))
+    assert np.array_equal(got[np.isinf(gen)], gen[np.isinf(gen)]) and np.isinf(gen).any() == (what != "key")
+    f = np.isfinite(gen)
+    assert np.isfinite(got[f]).all() and rel_err(got[f], gen[f]) < 1e-4
+    assert f.mean() > 0.9 or what == "both"
