@@ -197,9 +197,10 @@ __global__ __launch_bounds__(2 * D) void dequant_mfma_kernel(DequantArgs a, int 
         }
       }
       float o[8];
-      const float sc = C.n[h] * (1.f / (SC * SC));
+      // the scale leaves the sum before the norm comes in (2^-16 times a small
+      // norm would be subnormal)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) o[i] = (hh[i >> 2][i & 3] + xl[i >> 2][i & 3]) * sc;
+      for (int i = 0; i < 8; ++i) o[i] = (hh[i >> 2][i & 3] + xl[i >> 2][i & 3]) * (1.f / (SC * SC)) * C.n[h];
       if constexpr (MK > 0) {
         f4 zh[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}}, zl[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll

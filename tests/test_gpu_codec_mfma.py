@@ -135,3 +135,20 @@ def test_compress_mfma_special_vectors(d, dt):
         ca, cb = unpack_codes(a[0], a[1], bits, d), unpack_codes(b[0], b[1], bits, d)
         bad = (ca != cb).any(-1)[0, 0]
         assert not bad.any(), (np.nonzero(bad)[0] // 16, bits)
+
+
+@pytest.mark.parametrize("d,bits,m", [(64, 3.5, 32), (96, 3, 0), (128, 4, 128), (256, 2, 0)])
+def test_dequant_mfma_small_norms(d, bits, m):
+    """Norms from 1 down to 1e-36 (and as far up): each vector to float32 rounding. 5e-7 of its own norm, as above:
+    the coordinates are normal float32 numbers down to 1e-38, a few of them below that are exact to 1e-45."""
+    from turboquant_amd import _codec
+    codec = _codec.get_codec(d, bits, 42, m, DEV)
+    st = _random_store(codec, 1, 2, 80, seed=d)
+    st.norms[:, 0, :80] = 10.0 ** torch.linspace(0, -36, 80, device=DEV)
+    st.norms[:, 1, :80] = 10.0 ** torch.linspace(0, 36, 80, device=DEV)
+    if m:
+        st.gamma.copy_(st.norms * 0.3)
+    out = torch.empty(1, 2, 80, d, device=DEV)
+    _codec.dequantize_into(codec, st, 0, 80, out, 0, m > 0)
+    got, ref = out.double().cpu().numpy(), _exact(codec, st, bits, d, m)[:, :, :80]
+    assert (np.linalg.norm(got - ref, axis=-1) < 5e-7 * np.linalg.norm(ref, axis=-1)).all()
