@@ -570,17 +570,17 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
     for (int i = 0; i < NS; ++i) pm = fmaxf(pm, QJ ? fmaxf(fabsf(pv[i]), fabsf(pu[i])) : fabsf(pv[i]));
     const float pmx = pm * __builtin_amdgcn_ldexpf(1.f, -vx);
     if (__builtin_amdgcn_ballot_w64(pmx > uk::PV_LIMIT || (!vset && pmx > 0.f)) != 0) {
-      const float cm = rows_max(pmx);  // max of the column
+      const float cm = rows_max(pm);  // max of the column (unscaled: 2^-vx times it may pass float32)
       if (!vset) {
-        vx = cm > 0.f ? max((int)ceilf(log2f(cm / uk::PV_SET)), -110) : 0;
+        vx = cm > 0.f ? max((int)ceilf(log2f(cm) - log2f(uk::PV_SET)), -126) : 0;
         vset = true;
       } else {
-        const int dx = cm > uk::PV_LIMIT ? (int)ceilf(log2f(cm / uk::PV_LIMIT)) : 0;
-        const float f = __builtin_amdgcn_ldexpf(1.f, -dx);
+        const int up = min(max((int)ceilf(log2f(cm) - log2f(uk::PV_LIMIT)), vx), 256);
+        const float f = __builtin_amdgcn_ldexpf(1.f, vx - up);
 #pragma unroll
         for (int nb = 0; nb < U; ++nb) acc[nb] *= f;
         if constexpr (QJ) accu[0] *= f, accu[1] *= f;
-        vx += dx;
+        vx = up;
       }
     }
   };
@@ -824,6 +824,14 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
   // ---- combine the waves through LDS (the table region); the two fp16 parts
   // of a head meet through `partner`, for GC = 4 the two tiles at their common max
   l_run = rows_sum(l_run);
+  if (__builtin_amdgcn_ballot_w64(vx < -64) != 0) {
+    // small value norms: part of 2^vx now, so that the factor below stays normal
+    const float f = __builtin_amdgcn_ldexpf(1.f, min(vx + 64, 0));
+#pragma unroll
+    for (int nb = 0; nb < U; ++nb) acc[nb] *= f;
+    if constexpr (QJ) accu[0] *= f, accu[1] *= f;
+    vx = max(vx, -64);
+  }
   float tsc = __builtin_amdgcn_ldexpf(1.f, vx);
   if constexpr (TS == 2) {
     const float m2 = fmaxf(m_run, row_ror<8>(m_run));

@@ -237,3 +237,19 @@ def test_mfma_infinite_tokens(D, G, dt, T, what):
     f = np.isfinite(gen)
     assert np.isfinite(got[f]).all() and rel_err(got[f], gen[f]) < 1e-4
     assert f.mean() > 0.9 or what == "both"
+
+
+@pytest.mark.parametrize("D,m", [(64, 0), (256, 32)])
+@pytest.mark.parametrize("vmul", [1e-36, 1e33])
+def test_mfma_value_norms(D, m, vmul):
+    """Value norms near float32's ends, alone and in every other block of each wave beside ordinary ones (15 workgroups a
+    row, 14 or more blocks each): the weights' exponent covers them (1e-36 times a weight is normal down to 1e-2 of the
+    largest, below that exact to 1e-45: 2e-7 of an output; 1e33 leaves room for the general kernel's unscaled sums)."""
+    T = 6800
+    odd = np.arange(T)[:, None] // 256 % 2 == 1
+    for H, n, mul in ((2, 900, vmul), (16, T, np.where(odd, vmul, 1.0)), (16, T, np.where(odd, 1.0, vmul))):
+        k, v = _kv(1, H, n, D, seed=3)
+        q = np.random.RandomState(1).randn(1, H, 1, D).astype(np.float32)
+        c, o = _caches(dict(head_dim=D, num_kv_heads=H, residual_window=64, fp16_sink_size=16, key_bits=4, value_bits=3,
+                            **(dict(qjl_correction=True, qjl_n_proj=m) if m else {})), k, v * mul, torch.bfloat16)
+        _check(c, o, q, f"d{D} v x{vmul}")
