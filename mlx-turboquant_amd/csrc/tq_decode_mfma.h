@@ -66,9 +66,7 @@ using uk::as_h8;
 using uk::f4;
 using uk::fexp2;
 using uk::half8;
-using uk::hx2;
 using uk::mfma;
-using uk::pk_rtz;
 using uk::row_ror;
 using uk::rows_max;
 using uk::rows_sum;
@@ -86,9 +84,16 @@ constexpr float CSC = 256.f;
 constexpr float QLOW = 4096.f;
 
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef float f2 __attribute__((ext_vector_type(2)));
 __device__ inline f4 mfma_b(u4 a, u4 b, f4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, a), __builtin_bit_cast(bf8, b), c, 0, 0, 0);
 }
+
+// rounded to nearest (one v_cvt_pk_f16_f32): a high part and a remainder hold 24
+// bits of a weight without bias; truncated, 22 of them and the sum of weights
+// they are divided by too large by 1e-7
+__device__ inline h2 to_h2(float a, float b) { return __builtin_convertvector((f2{a, b}), h2); }
 
 // v = p[0] + p[1] + p[2], three bf16 parts of 8 values each (truncated: exact)
 __device__ inline void split_b(const float (&v)[8], u4 (&p)[3]) {
@@ -590,8 +595,8 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
 #pragma unroll
     for (int j = 0; j < NS / 2; ++j) {
       const float p0 = pv[2 * j] * down, p1 = pv[2 * j + 1] * down;
-      const hx2 h = __builtin_amdgcn_cvt_pkrtz(p0, p1);
-      d[j] = pk_rtz(fmaf(-partf, (float)h[0], p0), fmaf(-partf, (float)h[1], p1));
+      const h2 h = to_h2(p0, p1);
+      d[j] = __builtin_bit_cast(uint32_t, to_h2(fmaf(-partf, (float)h[0], p0), fmaf(-partf, (float)h[1], p1)));
     }
     return slots(d);
   };
