@@ -1688,10 +1688,28 @@ static int mfma_run(const tq_codec* kc, const tq_codec* vc, const tq_attn_desc* 
 
 // Sketched calls of uniform batches at 32 projections take the mfma kernels (one
 // pass, two launches) before the K4/V2 kernels with the terms around them (six
-// launches): K4/V2, 32 heads on 8, T 4,000 35.9 -> 17.4 us per layer, T 32,768
-// 39.9 -> 27.8. Ragged batches and longer sketches keep the latter.
+// launches), except where their grid leaves CUs idle for long. K4/V2, us per
+// layer, mfma kernels and the K4/V2 kernels (batch x tokens, query heads on kv
+// heads): 1 x 4,000, 32 on 8 18.4 / 33.7, 1 x 131,072 62 / 75, 4 x 32,768 66 / 73.
+// Past 64 rows (sequences x kv heads) a row has two workgroups, from 86 on one, on
+// the compressed blocks, and the launch is rounds of at most CUs of them (with
+// the uncompressed tokens' ones between): 32 on 8, 16 x 4,096 59 / 72 but 16 x 8,192 102 / 85, 12 x 10,923
+// 127 / 90, 24 x 8,192 191 / 116, 32 x 4,096 115 / 124, 32 x 8,192 197 / 148; the
+// line is at 1.25 blocks per row and round of workgroups. From 24 rows on, one or
+// two query heads per kv head (the K4/V2 kernels' terms cost per query head):
+// 8 on 8, 4 x 65,536 112 / 107, 8 x 16,384 73 / 65; 8 x 8,192 43 / 46; with four,
+// past 32 rows, long contexts: 32 on 8, 8 x 32,768 126 / 119 (8 x 16,384 74 / 75).
+// Ragged batches and longer sketches keep the K4/V2 kernels.
 static bool qjl_mfma(const tq_codec* kc, const tq_codec* vc, const tq_attn_desc* d) {
-  return d->qjl && d->max_comp > 0 && !d->comp_len && !d->sink_len && !d->res_len && mfma_eligible(kc, vc, d);
+  if (!(d->qjl && d->max_comp > 0 && !d->comp_len && !d->sink_len && !d->res_len && mfma_eligible(kc, vc, d)))
+    return false;
+  int gsub, g, ncw, nfw;
+  mfma_geometry(d, gsub, g, ncw, nfw);
+  const int64_t rows = (int64_t)d->batch * d->hkv * gsub;
+  const int64_t blocks = ((d->max_comp + 31) / 32 + ncw - 1) / ncw;  // per workgroup
+  if (rows > 64) return 4 * ((rows * (ncw + nfw) + device_cus() - 1) / device_cus()) * blocks <= 5 * rows;
+  if (g <= 2) return rows < 24 || blocks <= 128;
+  return g > 4 || rows <= 32 || blocks <= 256;
 }
 
 // The QJL route: S q, key-term bias, K4/V2 partials with the bias

@@ -253,3 +253,32 @@ def test_mfma_value_norms(D, m, vmul):
         c, o = _caches(dict(head_dim=D, num_kv_heads=H, residual_window=64, fp16_sink_size=16, key_bits=4, value_bits=3,
                             **(dict(qjl_correction=True, qjl_n_proj=m) if m else {})), k, v * mul, torch.bfloat16)
         _check(c, o, q, f"d{D} v x{vmul}")
+
+
+@pytest.mark.parametrize("hkv,G,batch,tokens,route", [
+    (8, 4, 1, 131072, 7), (8, 4, 8, 16384, 7), (8, 4, 8, 32768, 3), (8, 8, 8, 32768, 7), (8, 1, 3, 8192, 7), (8, 1, 2, 131072, 7), (8, 2, 4, 65536, 3),
+    (8, 4, 16, 4096, 7), (8, 4, 16, 8192, 3), (8, 4, 12, 10923, 3), (8, 4, 32, 4096, 7), (4, 4, 64, 8192, 3),
+    (8, 3, 16, 16384, 7), (16, 16, 16, 16384, 7)])
+def test_sketch_route_by_size(hkv, G, batch, tokens, route):
+    """K4/V2 with 32 projections: the K4/V2 kernels where the mfma grid would leave CUs idle for long, if they take the
+    ratio (a descriptor of that size over a small cache; nothing is launched)."""
+    from turboquant_amd import _lib
+    k, v = _kv(1, hkv, 100, 128, seed=0)
+    c, _ = _caches(dict(head_dim=128, num_kv_heads=hkv, residual_window=16, qjl_correction=True, qjl_n_proj=32), k, v,
+                   torch.float16)
+    q = torch.zeros(1, hkv * G, 128, device="cuda", dtype=torch.float16)
+    d = c.attention_descriptor(q, torch.empty(q.shape, device="cuda"), 0.1)
+    d.batch, d.max_comp, d.max_res = batch, tokens - 128, 128
+    fn = _lib.load().tq_debug_decode_route
+    fn.restype, fn.argtypes = ctypes.c_int32, [ctypes.c_void_p] * 3
+    assert fn(ctypes.addressof(c._kc.struct), ctypes.addressof(c._vc.struct), ctypes.addressof(d)) == route
+
+
+@pytest.mark.parametrize("G,T,route", [(4, 3520, 7), (4, 3521, 3), (1, 3521, 3)])
+def test_sketch_both_routes(G, T, route):
+    """Either side of that line (88 rows: 110 blocks)."""
+    k, v = _kv(11, 8, T + 40, 128, seed=T)
+    c, o = _caches(dict(head_dim=128, num_kv_heads=8, residual_window=40, chunk_size=1, qjl_correction=True, qjl_n_proj=32),
+                   k, v, torch.float16)
+    assert c._compressed_len == T
+    _check(c, o, np.random.RandomState(G).randn(11, 8 * G, 1, 128).astype(np.float16), f"QJL G={G} T={T}", route)
