@@ -362,9 +362,12 @@ __global__ __launch_bounds__(2 * D) void compress_mfma_kernel(CompressArgs a, in
       const float y = tq_fmul_legacy(z[k >> 2][k & 3] + zl[k >> 2][k & 3], sc);  // 0 where sc = 0
       uint32_t c;
       if constexpr (TABLE) {
-        const uint32_t i = __float_as_uint(fmaf(y, (float)L::CW, L::CW / 2 + MAGIC));
-        // (non-finite inputs: any cell of the table, the codes are dropped below)
-        const float2 q = *reinterpret_cast<const float2*>(smem + (sc < 0.f ? (uint32_t)L::qt : qadj + 8u * i));
+        // |y| <= 1 up to rounding; z may overflow beside a norm at float32's end
+        // and is anything for non-finite inputs (their codes are dropped below):
+        // the cells end at 1 + 7 / CW
+        const float yc = __builtin_amdgcn_fmed3f(y, -1.05f, 1.05f);
+        const uint32_t i = __float_as_uint(fmaf(yc, (float)L::CW, L::CW / 2 + MAGIC));
+        const float2 q = *reinterpret_cast<const float2*>(smem + (qadj + 8u * i));
         c = __float_as_uint(q.y) + (y > q.x ? 1u : 0u);
       } else {
         c = 0;

@@ -152,3 +152,21 @@ def test_dequant_mfma_small_norms(d, bits, m):
     _codec.dequantize_into(codec, st, 0, 80, out, 0, m > 0)
     got, ref = out.double().cpu().numpy(), _exact(codec, st, bits, d, m)[:, :, :80]
     assert (np.linalg.norm(got - ref, axis=-1) < 5e-7 * np.linalg.norm(ref, axis=-1)).all()
+
+
+@pytest.mark.parametrize("d", [64, 96, 128, 256])
+def test_compress_mfma_norm_at_the_end_of_float32(d):
+    """Vectors along a row of R whose norm is float32's largest value or a few units below: the rotated coordinate may
+    pass it (the quantizer's cells are looked up inside the table). Codes of the general kernel, which divides first."""
+    R = O.rotation_matrix(d).astype(np.float64)
+    top = float(np.finfo(np.float32).max)
+    f = np.array([1 - k * 2.0 ** -24 for k in (0, 1, 2, 3, 4, 8, 1 << 20)])
+    x = (np.concatenate([R, -R])[:, None] * (f[:, None] * top)).astype(np.float32).reshape(1, 1, -1, d)
+    x = torch.from_numpy(x).cuda()
+    for bits in (4, 2):
+        a, b = _compress(x, bits), _compress(x, bits, general=True)
+        assert np.array_equal(a[2], b[2]) and np.isfinite(b[2]).mean() > 0.5
+        ca, cb = unpack_codes(a[0], a[1], bits, d), unpack_codes(b[0], b[1], bits, d)
+        big = np.abs(x.cpu().double().numpy() @ R.T) > 1e38  # (the others are 0 up to rounding: a cell boundary)
+        fin = np.isfinite(b[2])[..., None] & big
+        assert (ca == cb)[fin].all()
