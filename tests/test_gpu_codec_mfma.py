@@ -170,3 +170,114 @@ def test_compress_mfma_norm_at_the_end_of_float32(d):
         big = np.abs(x.cpu().double().numpy() @ R.T) > 1e38  # (the others are 0 up to rounding: a cell boundary)
         fin = np.isfinite(b[2])[..., None] & big
         assert (ca == cb)[fin].all()
+
+
+# ---- persistent workgroups over several tiles: at most 8 / 5 / 4 / 2 workgroups per CU fit at these head_dims (LDS of the
+# x tiles), so these counts give each at least three 64-vector tiles (six of the dequantize kernel's 32)
+_TILES = {64: 3 * 256 * 8, 96: 3 * 256 * 5, 128: 3 * 256 * 4, 256: 3 * 256 * 2}
+
+
+def _long_span(d, rows_per_seq):
+    """Per-sequence lengths of 8 sequences (empty and one-token ones between, odd tails) with that many tiles, and their
+    source and destination offsets."""
+    from turboquant_amd import _lib
+    T = _TILES[d] // (5 * rows_per_seq) * 64 + 64 * 3 + 1
+    n_b = [T, 0, T - 1, 1, T - 63, T - 100, 0, T]
+    src, dst = [0, 3, 5, 0, 7, 1, 2, 0], [2, 0, 0, 9, 4, 0, 0, 7]
+    assert rows_per_seq * sum((n + 63) // 64 for n in n_b) >= _TILES[d]
+    arrays = [torch.tensor(a, dtype=torch.int32, device=DEV) for a in (n_b, src, dst)]
+    span = _lib.Span(rows=8 * rows_per_seq, heads=rows_per_seq, n_tok=T, reserved=0, n_tok_b=arrays[0].data_ptr(),
+                     src_tok0_b=arrays[1].data_ptr(), dst_tok0_b=arrays[2].data_ptr())
+    return T, n_b, src, dst, span, arrays
+
+
+def _bits(t, width, n):
+    """(..., n) codes of `width` bits from LSB-first byte rows, on the device."""
+    b = ((t[..., None] >> torch.arange(8, device=DEV, dtype=torch.uint8)) & 1).flatten(-2)[..., :n * width]
+    return (b.unflatten(-1, (n, width)).int() << torch.arange(width, device=DEV)).sum(-1)
+
+
+def _codes(codec, st, b, sl):
+    idx = _bits(st.codes_hi[b, :, sl], codec.bits_hi, codec.split)
+    if codec.fractional:
+        idx = torch.cat([idx, _bits(st.codes_lo[b, :, sl], codec.bits_lo, codec.d - codec.split)], -1)
+    return idx
+
+
+def _exact64(codec, st, b, sl):
+    idx = _codes(codec, st, b, sl)
+    c = codec.c_hi.double()[idx[..., :codec.split]]
+    if codec.fractional:
+        c = torch.cat([c, codec.c_lo.double()[idx[..., codec.split:]]], -1)
+    return st.norms[b, :, sl, None].double() * (c @ codec.rotation.double())
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("d,bits,m", [(64, 3.5, 0), (96, 3, 0), (128, 2.5, 0), (128, 1, 0), (256, 4, 0), (64, 2, 32),
+                                      (96, 4, 64), (128, 3.5, 128)])
+def test_compress_mfma_several_tiles(d, bits, m, dt):
+    """Norms and codes of the general kernel (other codes only within 2e-6 of a boundary, the float32 rotations'
+    rounding), signs and residual norms of float64 over the codes, nothing written outside the spans."""
+    from turboquant_amd import _codec, _lib
+    H = 3
+    T, n_b, src, dst, span, keep = _long_span(d, H)
+    codec = _codec.get_codec(d, bits, 42, m, DEV)
+    g = torch.Generator(device=DEV).manual_seed(d + m)
+    x = (torch.randn(8, H, T + 8, d, device=DEV, generator=g) * torch.exp(torch.randn(8, H, T + 8, 1, device=DEV, generator=g))).to(dt)
+    stores = []
+    for general in (False, True):
+        st = _codec.PackedStore(codec, 8, H, qjl=m > 0)
+        st.reserve(T + 16, 0)
+        for t in (st.codes_hi, st.codes_lo, st.norms, st.signs, st.gamma):
+            if t is not None:
+                t.fill_(77)
+        s = st.struct(0)
+        _lib.check(_lib.load().tq_compress(codec.ref(general), x.data_ptr(), _lib.dtype_code(dt), x.stride(1),
+                                           ctypes.byref(span), ctypes.byref(s), _lib.stream_ptr(DEV)), "tq_compress")
+        stores.append(st)
+    a, ref = stores
+    bnd = [codec.b_hi.double(), codec.b_lo.double()]
+    for b, (n, s0, t0) in enumerate(zip(n_b, src, dst)):
+        sl = slice(t0, t0 + n)
+        for t in (a.codes_hi, a.codes_lo, a.norms, a.signs, a.gamma):
+            if t is not None:
+                assert (t[b, :, :t0] == 77).all() and (t[b, :, t0 + n:] == 77).all()
+        if n == 0:
+            continue
+        assert torch.equal(a.norms[b, :, sl], ref.norms[b, :, sl])
+        xb = x[b, :, s0:s0 + n].double()
+        h, tok, j = torch.nonzero(_codes(codec, a, b, sl) != _codes(codec, ref, b, sl), as_tuple=True)
+        y = ((xb[h, tok] / xb[h, tok].norm(dim=-1, keepdim=True)) * codec.rotation.double()[j]).sum(-1)
+        near = torch.where(j < codec.split, (y[:, None] - bnd[0]).abs().amin(-1), (y[:, None] - bnd[1]).abs().amin(-1))
+        assert h.numel() < 1e-5 * xb.numel() + 3 and (near < 2e-6).all()
+        if m:
+            res = xb - _exact64(codec, a, b, sl)
+            proj = res @ codec.proj.double().T
+            clear = proj.abs() > 1e-4 * xb.norm(dim=-1, keepdim=True)
+            assert (_bits(a.signs[b, :, sl], 1, m).bool() == (proj >= 0))[clear].all() and clear.double().mean() > 0.9
+            assert (a.gamma[b, :, sl] - res.norm(dim=-1)).norm() < 2e-6 * res.norm()
+
+
+@pytest.mark.parametrize("d,bits,m", [(64, 3.5, 0), (64, 1, 32), (96, 3, 0), (96, 2.5, 96), (128, 4, 0), (128, 2, 128),
+                                      (256, 3.5, 0), (256, 4, 32)])
+def test_dequant_mfma_several_tiles(d, bits, m):
+    """Float64 over the codes at 5e-7 as above, nothing else written."""
+    from turboquant_amd import _codec, _lib
+    H = 3
+    T, n_b, src, dst, span, keep = _long_span(d, H)
+    codec = _codec.get_codec(d, bits, 42, m, DEV)
+    st = _random_store(codec, 8, H, T + 8, seed=d + m)
+    out = torch.full((8, H, T + 16, d), 7.0, device=DEV)
+    s = st.struct(0)
+    _lib.check(_lib.load().tq_dequantize(codec.ref(), ctypes.byref(s), ctypes.byref(span), out.data_ptr(), out.stride(1),
+                                         1 if m else 0, _lib.stream_ptr(DEV)), "tq_dequantize")
+    for b, (n, s0, t0) in enumerate(zip(n_b, src, dst)):
+        assert (out[b, :, :t0] == 7.0).all() and (out[b, :, t0 + n:] == 7.0).all()
+        if n == 0:
+            continue
+        ref = _exact64(codec, st, b, slice(s0, s0 + n))
+        if m:
+            z = 2 * _bits(st.signs[b, :, s0:s0 + n], 1, m).double() - 1
+            ref = ref + 1.2533141373155003 / d * st.gamma[b, :, s0:s0 + n, None].double() * (z @ codec.proj.double()[:m])
+        err = (out[b, :, t0:t0 + n] - ref).norm(dim=-1) / ref.norm(dim=-1)
+        assert err.max() < 2e-6 and (out[b, :, t0:t0 + n] - ref).norm() < 5e-7 * ref.norm()
