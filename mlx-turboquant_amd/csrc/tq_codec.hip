@@ -1001,7 +1001,7 @@ int tq_ragged_step(const tq_codec* kcodec, const tq_codec* vcodec, const void* k
   if (dtype != TQ_F16 && dtype != TQ_BF16) return set_error(TQ_ERR_UNSUPPORTED, "ragged_step: dtype %d", dtype);
   if (!k || !v || !ring_k || !ring_v || !kstore || !vstore || !seq_ints || !seq_ints_dev)
     return set_error(TQ_ERR_INVALID, "ragged_step: NULL pointer");
-  if (batch < 0 || heads <= 0 || ring_cap <= 0 || (ring_head_stride & 7) || ring_head_stride < (int64_t)ring_cap * 128 ||
+  if (batch < 0 || heads <= 0 || ring_cap <= 0 || (ring_head_stride & 7) || ring_head_stride < (int64_t)ring_cap * kcodec->d ||
       n_ints < 4 * batch || (int64_t)batch * heads >= ((int64_t)1 << 24))
     return set_error(TQ_ERR_INVALID, "ragged_step: bad shape (batch %d heads %d cap %d stride %lld ints %d)", batch, heads,
                      ring_cap, (long long)ring_head_stride, n_ints);

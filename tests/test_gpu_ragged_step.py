@@ -203,3 +203,24 @@ def test_stream_handle_is_torch_current_stream():
     with torch.cuda.stream(s):
         assert _lib.stream_ptr(DEV) == s.cuda_stream != 0
     assert _lib.stream_ptr(DEV) == torch.cuda.current_stream(DEV).cuda_stream
+
+
+@pytest.mark.parametrize("D", [64, 96])
+def test_step_below_head_dim_128(D):
+    """tq_ragged_step has no launch for these (TQ_ERR_UNSUPPORTED, whatever the ring's stride): the batch takes the
+    append and the drains in calls of their own, and its attention follows."""
+    from turboquant_amd.ragged import RaggedKVBatch
+    rb = RaggedKVBatch(2, 2, head_dim=D, residual_window=32, fp16_sink_size=8)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    for b, t in enumerate((20, 100)):
+        rb.load(b, *(torch.randn(2, t, D, generator=g, device="cuda").half() for _ in range(2)))
+    for i in range(30):
+        k, v = (torch.randn(2, 2, D, generator=g, device="cuda").half() for _ in range(2))
+        slot = (rb.res_start + rb.res_len) % rb.cap
+        rb.step(k, v)
+        for b in range(2):
+            assert torch.equal(rb.ring_k[b, :, slot[b]], k[b]) and torch.equal(rb.ring_v[b, :, slot[b]], v[b])
+    assert rb.comp_len.tolist() == [10, 90]
+    q = torch.randn(2, 4, D, generator=g, device="cuda")
+    got, gen = rb.attend(q), rb.attend(q, general=True)
+    assert (got - gen).norm() < 1e-5 * gen.norm()
