@@ -102,31 +102,142 @@ def test_mfma_magnitudes(D, kmul, vmul, qmul):
     _check(c, o, q, f"d{D} k x{kmul} v x{vmul} q x{qmul}")
 
 
-def test_mfma_ragged_equals_single_sequences():
+def _one_sequence(d, b, H, q, out):
+    """Descriptor d with sequence b of its batch alone (same stores, sink and ring)."""
+    one = type(d).from_buffer_copy(d)
+    one.batch, one.q, one.out = 1, q.data_ptr(), out.data_ptr()
+    for st in (one.kstore, one.vstore):
+        for name, stride, size in (("codes_hi", st.hi_head_stride, 1), ("codes_lo", st.lo_head_stride, 1), ("norms", st.norm_head_stride, 4),
+                                   ("signs", st.sign_head_stride, 1), ("gamma", st.gamma_head_stride, 4)):
+            if getattr(st, name):
+                setattr(st, name, getattr(st, name) + b * H * stride * size)
+    for name, stride in (("sink_k", d.sink_head_stride), ("sink_v", d.sink_head_stride), ("res_k", d.res_head_stride),
+                         ("res_v", d.res_head_stride)):
+        setattr(one, name, getattr(one, name) + b * H * stride * 2)
+    for name in ("comp_len", "sink_len", "res_len", "res_start"):
+        setattr(one, name, getattr(one, name) + 4 * b)
+    return one
+
+
+@pytest.mark.parametrize("D,kb,vb,m,G,bf", [(128, 3.5, 3, 0, 3, False), (128, 3, 3, 32, 4, False), (64, 4, 2, 0, 4, True),
+                                            (256, 4, 3, 0, 2, True), (256, 4, 2, 32, 8, False), (64, 3.5, 2.5, 32, 7, True)])
+def test_mfma_ragged_equals_single_sequences(D, kb, vb, m, G, bf):
     """A ragged batch (per-sequence lengths, a sequence with nothing
     compressed, wrapped rings) on these kernels: each sequence equals its own
-    call over the same stores, whose partials are cut elsewhere."""
+    call over the same stores, whose partials are cut elsewhere, and float64
+    attention over what is stored."""
     from turboquant_amd import _lib
     from turboquant_amd.ragged import RaggedKVBatch
-    H, G, D = 2, 3, 128
+    H = 2
     lens = [40, 300, 1777, 5000]
-    rb = RaggedKVBatch(4, H, head_dim=D, key_bits=3.5, value_bits=3, residual_window=64, fp16_sink_size=16)
+    rb = RaggedKVBatch(4, H, head_dim=D, key_bits=kb, value_bits=vb, residual_window=64, fp16_sink_size=16, qjl_n_proj=m)
     rng = np.random.RandomState(9)
     for b, t in enumerate(lens):
         rb.load(b, *(to_dev(rng.randn(H, t, D).astype(np.float16)) for _ in range(2)))
     for _ in range(5):
         rb.step(*(to_dev(rng.randn(4, H, D).astype(np.float16)) for _ in range(2)))
+    assert rb.comp_len[0] == 0 and (rb.res_start[1:] + rb.res_len[1:] > rb.cap).all()
     q = to_dev(rng.randn(4, H * G, D).astype(np.float16))
     out = torch.empty(q.shape, dtype=torch.float32, device=q.device)
     d, keep = rb.descriptor(q, out, D ** -0.5)
-    fn = _lib.load().tq_debug_decode_route
+    d = type(d).from_buffer_copy(d)  # (the batch refreshes its own for every call)
+    sink_k, sink_v, ring_k, ring_v = rb.sink_k, rb.sink_v, rb.ring_k, rb.ring_v
+    if bf:
+        sink_k, sink_v, ring_k, ring_v = (t.bfloat16() for t in (sink_k, sink_v, ring_k, ring_v))
+        d.kv_dtype = _lib.TQ_BF16
+        d.sink_k, d.sink_v, d.res_k, d.res_v = (t.data_ptr() for t in (sink_k, sink_v, ring_k, ring_v))
+    lib = _lib.load()
+    fn = lib.tq_debug_decode_route
     fn.restype, fn.argtypes = ctypes.c_int32, [ctypes.c_void_p] * 3
-    assert fn(ctypes.addressof(rb.kc.struct), ctypes.addressof(rb.vc.struct), ctypes.addressof(d)) == 7
-    got = rb.attend(q).cpu().numpy()
-    gen = rb.attend(q, general=True).cpu().numpy()
-    assert np.isfinite(got).all()
+
+    def call(desc):
+        assert fn(ctypes.addressof(rb.kc.struct), ctypes.addressof(rb.vc.struct), ctypes.addressof(desc)) == 7
+        need = lib.tq_attention_workspace_bytes(rb.kc.ref(), rb.vc.ref(), ctypes.byref(desc))
+        ws = torch.empty(need, dtype=torch.uint8, device=q.device)
+        _lib.check(lib.tq_decode_attention(rb.kc.ref(), rb.vc.ref(), ctypes.byref(desc), ws.data_ptr(), need,
+                                           _lib.stream_ptr(q.device)), "tq_decode_attention")
+        torch.cuda.synchronize()
+
+    call(d)
+    got = out.cpu().numpy()
+    if not bf:
+        assert np.array_equal(got, rb.attend(q).cpu().numpy())
+        gen = rb.attend(q, general=True).cpu().numpy()
+    R = O.rotation_matrix(D)
+    n64 = lambda t: t.cpu().double().numpy()
     for b in range(4):
-        assert rel_err(got[b], gen[b]) < REL_TOL, b
+        qb, ob = q[b:b + 1].contiguous(), torch.empty(1, H * G, D, device=q.device)
+        call(_one_sequence(d, b, H, qb, ob))
+        assert rel_err(got[b:b + 1], ob.cpu().numpy()) < 2e-6, b
+        C, S = int(rb.comp_len[b]), int(rb.sink_len[b])
+        slots = torch.as_tensor((rb.res_start[b] + np.arange(rb.res_len[b])) % rb.cap, device=q.device)
+        dense = []
+        for st, codec, sk, ring in ((rb.kstore, rb.kc, sink_k, ring_k), (rb.vstore, rb.vc, sink_v, ring_v)):
+            seg = [n64(sk[b:b + 1, :, :S])]
+            if C:
+                part = lambda t: None if t is None else t[b:b + 1, :, :C].cpu().numpy()
+                x = O.dequantize(part(st.codes_hi), part(st.codes_lo), part(st.norms), R, codec.bits, D)
+                if m:
+                    signs = np.unpackbits(part(st.signs), axis=-1, bitorder="little").astype(bool)
+                    x = x + O.qjl_correction(signs, part(st.gamma), rb.kc.proj.cpu().numpy(), D)
+                seg.append(x)
+            dense.append(np.concatenate(seg + [n64(ring[b:b + 1][:, :, slots])], axis=2))
+        ref = O.attention(n64(qb)[:, :, None], *dense)[:, :, 0]
+        assert rel_err(got[b:b + 1], ref) < REL_TOL and min_cos(got[b:b + 1], ref) >= COS_TOL, b
+        if not bf:
+            assert rel_err(got[b], gen[b]) < REL_TOL, b
+
+
+def test_mfma_more_than_256_partials():
+    """A residual window of 70,000 tokens: 274 workgroups of uncompressed tokens beside those of the compressed ones,
+    more headers than the merge holds in registers."""
+    T, W = 73000, 70000
+    k, v = _kv(1, 1, T, 64, seed=1)
+    c, o = _caches(dict(head_dim=64, num_kv_heads=1, residual_window=W, chunk_size=1, fp16_sink_size=8), k, v, torch.bfloat16)
+    assert c._compressed_len == T - W - 8
+    _check(c, o, np.random.RandomState(4).randn(1, 4, 1, 64).astype(np.float16), "window 70000")
+
+
+@pytest.mark.parametrize("D,kb,vb,m,dt", [(64, 4, 2, 0, torch.bfloat16), (256, 4, 3, 32, torch.float16)])
+def test_mfma_no_allocation_entry(D, kb, vb, m, dt):
+    """tq_decode_attention_noalloc on these kernels: bit-equal to the workspace entry point, eager (a smaller call over
+    the scratch of a larger one) and captured, replayed with eager calls on the same scratch between."""
+    from turboquant_amd import _lib
+    lib = _lib.load()
+    calls = []
+    for T, seed in ((3000, 1), (700, 2)):
+        k, v = _kv(1, 2, T, D, seed=seed)
+        c, _ = _caches(dict(head_dim=D, num_kv_heads=2, key_bits=kb, value_bits=vb, residual_window=64, fp16_sink_size=16,
+                            **(dict(qjl_correction=True, qjl_n_proj=m) if m else {})), k, v, dt)
+        q = to_dev(np.random.RandomState(seed).randn(1, 8, 1, D).astype(np.float16))
+        assert decode_route(c, q) == 7
+        calls.append((c, q, c.attend(q)))
+
+    def noalloc(c, q, out):
+        desc = c.attention_descriptor(q, out, D ** -0.5)
+        _lib.check(lib.tq_decode_attention_noalloc(c._kc.ref(), c._vc.ref(), ctypes.byref(desc), _lib.stream_ptr(q.device)),
+                   "tq_decode_attention_noalloc")
+
+    for c, q, ref in calls:
+        out = torch.full_like(ref, float("nan"))
+        noalloc(c, q, out)
+        assert torch.equal(out, ref)
+    (c, q, ref), (c2, q2, ref2) = calls
+    out = torch.empty_like(ref)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        noalloc(c, q, out)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref)
+        out2 = torch.full_like(ref2, float("nan"))
+        noalloc(c2, q2, out2)
+        torch.cuda.synchronize()
+        assert torch.equal(out2, ref2)
 
 
 def test_mfma_graph_replays():
@@ -239,7 +350,7 @@ def test_mfma_infinite_tokens(D, G, dt, T, what):
     assert f.mean() > 0.9 or what == "both"
 
 
-@pytest.mark.parametrize("D,m", [(64, 0), (256, 32)])
+@pytest.mark.parametrize("D,m", [(64, 0), (128, 32)])
 @pytest.mark.parametrize("vmul", [1e-36, 1e33])
 def test_mfma_value_norms(D, m, vmul):
     """Value norms near float32's ends, alone and in every other block of each wave beside ordinary ones (15 workgroups a
@@ -274,7 +385,7 @@ def test_sketch_route_by_size(hkv, G, batch, tokens, route):
     assert fn(ctypes.addressof(c._kc.struct), ctypes.addressof(c._vc.struct), ctypes.addressof(d)) == route
 
 
-@pytest.mark.parametrize("G,T,route", [(4, 3520, 7), (4, 3521, 3), (1, 3521, 3)])
+@pytest.mark.parametrize("G,T,route", [(4, 3520, 7), (1, 3521, 3)])
 def test_sketch_both_routes(G, T, route):
     """Either side of that line (88 rows: 110 blocks)."""
     k, v = _kv(11, 8, T + 40, 128, seed=T)
