@@ -1616,7 +1616,8 @@ static bool mfma_eligible(const tq_codec* kc, const tq_codec* vc, const tq_attn_
 // round of loads (head_dim 256, T 12,000, 96 partials instead of 48: partials
 // 20.2 -> 18.7 us, merge 6.3 -> 8.4 us), so past that the workgroups are filled
 // first. Uncompressed tokens: likewise, 8 blocks per workgroup where 4 would
-// take a quarter of the CUs.
+// take a quarter of the CUs, and more past a million tokens, whose partials'
+// weights would not fit the merge's LDS.
 static void mfma_geometry(const tq_attn_desc* d, int& gsub, int& g, int& ncw, int& nfw) {
   const int G = d->hq / d->hkv;
   g = group_heads(G);
@@ -1624,8 +1625,10 @@ static void mfma_geometry(const tq_attn_desc* d, int& gsub, int& g, int& ncw, in
   const int64_t rows = (int64_t)d->batch * d->hkv * gsub;
   const int half = MFMA_WAVES / 2 * 32;
   const int cus = device_cus();
+  constexpr int MOST_NFW = 4096;
   nfw = (int)(((int64_t)d->max_sink + d->max_res + half - 1) / half);
   if (rows * nfw > cus / 4) nfw = (nfw + 1) / 2;
+  if (nfw > MOST_NFW) nfw = MOST_NFW;
   constexpr int ONE_ROUND = 60;
   int most = (d->max_comp + half - 1) / half;
   if (most > ONE_ROUND) most = most / 2 > ONE_ROUND ? (most + 1) / 2 : ONE_ROUND;
@@ -2005,7 +2008,8 @@ int tq_decode_attention(const tq_codec* kc, const tq_codec* vc, const tq_attn_de
       dense_check(d, kc->d, false) == TQ_OK)
     return dense_run(d, workspace, workspace_bytes, s);
   if (qjl_mfma(kc, vc, d) && !(d->flags & TQ_ATTN_GENERAL)) {
-    if (mfma_run(kc, vc, d, workspace, s) != 0) TQ_LAUNCH_CHECK("tq_decode_attention (mfma)");
+    if (mfma_run(kc, vc, d, workspace, s) != 0) return set_error(TQ_ERR_UNSUPPORTED, "key width has no mfma kernel");
+    TQ_LAUNCH_CHECK("tq_decode_attention (mfma)");
     return TQ_OK;
   }
   if (qjl && d->max_comp > 0 && fast_eligible(kc, vc, d, true) && !(d->flags & TQ_ATTN_GENERAL))
@@ -2032,7 +2036,8 @@ int tq_decode_attention(const tq_codec* kc, const tq_codec* vc, const tq_attn_de
     }
   }
   if (mfma_eligible(kc, vc, d) && !(d->flags & TQ_ATTN_GENERAL)) {
-    if (mfma_run(kc, vc, d, workspace, s) != 0) TQ_LAUNCH_CHECK("tq_decode_attention (mfma)");
+    if (mfma_run(kc, vc, d, workspace, s) != 0) return set_error(TQ_ERR_UNSUPPORTED, "key width has no mfma kernel");
+    TQ_LAUNCH_CHECK("tq_decode_attention (mfma)");
     return TQ_OK;
   }
 

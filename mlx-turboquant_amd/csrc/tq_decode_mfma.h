@@ -1110,7 +1110,8 @@ static void launch_g(const MfmaArgs& a, hipStream_t s) {
     launch_k<D, 8, KK, QJ>(a, s);
 }
 
-// kk: key width kind (KGeo)
+// kk: key width kind (KGeo); -1 for one that has no kernel, launch errors are the
+// caller's to ask for
 template <int D, bool QJ>
 int launch_mfma(const MfmaArgs& a, int kk, hipStream_t s) {
   switch (kk) {
@@ -1129,7 +1130,7 @@ int launch_mfma(const MfmaArgs& a, int kk, hipStream_t s) {
   constexpr int round = MergeGeo<D>::PG * MergeGeo<D>::MB;
   hipLaunchKernelGGL((mfma_merge_kernel<D, QJ>), dim3(a.hq, a.batch), dim3(MergeGeo<D>::NT),
                      (np + round - 1) / round * round * 4, s, a, np);
-  return hipGetLastError() == hipSuccess ? 0 : -1;
+  return 0;
 }
 
 }  // namespace mk

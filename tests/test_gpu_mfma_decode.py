@@ -198,6 +198,22 @@ def test_mfma_more_than_256_partials():
     _check(c, o, np.random.RandomState(4).randn(1, 4, 1, 64).astype(np.float16), "window 70000")
 
 
+def test_mfma_ten_million_tokens():
+    """An uncompressed list whose partials, one per 256 tokens, would pass the merge's LDS (a launch that fails is an error
+    too, not a call without output): the general kernel's result."""
+    from turboquant_amd import TurboQuantKVCache
+    T = 9_600_000
+    g = torch.Generator(device="cuda").manual_seed(1)
+    k, v = (torch.randn(1, 1, T, 64, generator=g, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    c = TurboQuantKVCache(head_dim=64, num_kv_heads=1, residual_window=T, chunk_size=1)
+    c.update(k, v)
+    q = torch.randn(1, 2, 1, 64, generator=g, device="cuda")
+    assert c._compressed_len == 0 and decode_route(c, q) == 7
+    got, gen = c.attend(q), c.attend(q, general_kernel=True)
+    # 9.6M weights of one part each: the sums carry float32 rounding of their order, 1e-5 of the small average
+    assert (got - gen).norm() < 1e-4 * gen.norm()
+
+
 @pytest.mark.parametrize("D,kb,vb,m,dt", [(64, 4, 2, 0, torch.bfloat16), (256, 4, 3, 32, torch.float16)])
 def test_mfma_no_allocation_entry(D, kb, vb, m, dt):
     """tq_decode_attention_noalloc on these kernels: bit-equal to the workspace entry point, eager (a smaller call over
