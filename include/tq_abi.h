@@ -64,8 +64,12 @@ typedef struct tq_codec {
                                      The K4/V2 decode kernels rotate the query
                                      with the key codec's planes (the output
                                      goes back with the value codec's float32
-                                     `rotation`); others ignore it. Arrays with
-                                     more planes work: only [0, 1] are read. */
+                                     `rotation`), those of the other widths,
+                                     fractional widths and head_dims 64 / 96 /
+                                     256 likewise; compress, dequantize, prefill
+                                     and the general kernel ignore it. Arrays
+                                     with more planes work: only [0, 1] are
+                                     read, and [2] with TQ_CODEC_ROTATION_LO2. */
   /* Host-side tables, filled by tq_codec_prepare() from a host copy of
    * centroids_hi (codebooks of at most 16 entries; passed to kernels by value):
    * host_centroids = centroids_hi, n_host_centroids entries; and for 2-bit
@@ -92,6 +96,13 @@ typedef struct tq_codec {
  * general compress kernel instead of the MFMA kernel (no reference
  * counterpart; lets tests compare the two kernels, per call). */
 #define TQ_CODEC_GENERAL_COMPRESS 1
+
+/* tq_codec.flags: rotation_parts holds a third plane, [2] = fp16(2048 (R -
+ * [0])), which keeps the bits of the remainder that are below fp16's normal
+ * range in [1] (R's entries are about d^-1/2, so [1] holds 8 to 10 bits). The
+ * decode kernels of head_dims 64 / 96 / 256 and of bf16 caches read it in place
+ * of [1]. */
+#define TQ_CODEC_ROTATION_LO2 2
 
 /* Fills the host-side tables of `codec` (host_centroids, value_table,
  * value_scale, value_table_err) from a host copy of centroids_hi

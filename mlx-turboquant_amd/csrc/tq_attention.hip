@@ -1662,7 +1662,10 @@ static int mfma_run(const tq_codec* kc, const tq_codec* vc, const tq_attn_desc* 
   a.q = d->q; a.q_dtype = d->q_dtype; a.out = d->out;
   a.batch = d->batch; a.hq = d->hq; a.hkv = d->hkv;
   a.qscale = d->scale * 1.4426950408889634f;
-  a.rot16 = kc->rotation_parts; a.vrot = vc->rotation;
+  const bool lo2 = (kc->flags & TQ_CODEC_ROTATION_LO2) != 0;
+  a.rot16 = kc->rotation_parts;
+  a.rot_lo = a.rot16 + (lo2 ? 2 : 1) * kc->d * kc->d; a.rls = lo2 ? 2048.f : 1.f;
+  a.vrot = vc->rotation;
   a.kcen_hi = kc->centroids_hi; a.kcen_lo = kk > 4 ? kc->centroids_lo : kc->centroids_hi;
   a.vcen_hi = vc->centroids_hi; a.vcen_lo = vk > 4 ? vc->centroids_lo : vc->centroids_hi;
   a.vbh = vc->bits_hi; a.vbl = vk > 4 ? vc->bits_lo : vc->bits_hi; a.vfrac = vk > 4;

@@ -190,7 +190,8 @@ struct MfmaArgs {
   int batch, hq, hkv;
   int gsub, g;           // head groups per kv head, query heads per group (at most 8)
   float qscale;          // scale * log2(e)
-  const uint16_t* rot16; // (2, D, D) fp16 high part / remainder of R (key codec)
+  const uint16_t* rot16; // (D, D) fp16 high part of R (key codec)
+  const uint16_t* rot_lo; float rls;  // (D, D) fp16(rls times the remainder)
   const float* vrot;     // (D, D) R float32, row-major (value codec)
   const float* kcen_hi; const float* kcen_lo;  // codebooks in device memory
   const float* vcen_hi; const float* vcen_lo;

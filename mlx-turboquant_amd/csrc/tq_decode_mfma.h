@@ -313,14 +313,15 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
   }
   uint32_t cw = 0;
   Blk<D, KK, QJ> B0, B1;
-  // rows 16 jt + r of R (fp16 high part, remainder) as B operands of the query rotation
+  // rows 16 jt + r of R (fp16 high part, rls times the remainder) as B operands
+  // of the query rotation
   u4 rqh[G_::KS], rql[G_::KS];
   auto load_rot = [&](int jt) {
-    const uint16_t* rh = a.rot16 + (16 * jt + r) * D + 8 * q4;
+    const int o = (16 * jt + r) * D + 8 * q4;
 #pragma unroll
     for (int kb = 0; kb < G_::KS; ++kb) {
-      rqh[kb] = *reinterpret_cast<const u4*>(rh + 32 * kb);
-      rql[kb] = *reinterpret_cast<const u4*>(rh + D * D + 32 * kb);
+      rqh[kb] = *reinterpret_cast<const u4*>(a.rot16 + o + 32 * kb);
+      rql[kb] = *reinterpret_cast<const u4*>(a.rot_lo + o + 32 * kb);
     }
   };
   if (packed) {
@@ -414,11 +415,13 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
 #pragma unroll
         for (int k = 0; k < 3; ++k) *reinterpret_cast<u4*>(d + k * L_::QS) = p[k];
       } else {
+        // (the remainder in the scale of R's, whose products it joins)
         half8 hi, lo;
+        const float ls = packed ? a.rls : 1.f;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           hi[i] = (_Float16)x[i];
-          lo[i] = (_Float16)(x[i] - (float)hi[i]);
+          lo[i] = (_Float16)((x[i] - (float)hi[i]) * ls);
         }
         *reinterpret_cast<half8*>(d) = hi;
         *reinterpret_cast<half8*>(d + L_::QS) = lo;
@@ -440,6 +443,7 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
     // part / remainder rows [head][part][D] (the scores take qscale: a small
     // one here would push the remainders below fp16's normal range)
     const uint8_t* qs = tail + L_::qsrc + min(r, a.g - 1) * 3 * L_::QS + 16 * q4;
+    const float lup = 1.f / a.rls;  // a power of two
     for (int jt = w; jt < U; jt += MW) {
       if (jt != w) load_rot(jt);
       f4 dq = {0.f, 0.f, 0.f, 0.f}, dl = {0.f, 0.f, 0.f, 0.f};
@@ -454,7 +458,7 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
       for (int i = 0; i < 4; ++i) {
         const int h = 4 * q4 + i;
         if (h < a.g && h < GC) {
-          const float v = dq[i] + dl[i];
+          const float v = fmaf(dl[i], lup, dq[i]);
           const _Float16 hi = (_Float16)v, lo = (_Float16)(v - (float)hi);
           uint8_t* d = qop + (h * 2) * L_::QS + 2 * (16 * jt + r);
           *reinterpret_cast<_Float16*>(d) = hi;
@@ -476,7 +480,7 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
           for (int e = 0; e < 8; ++e) {
             const float v = sp[32 * kb + e];
             sh[e] = (_Float16)v;
-            sl[e] = (_Float16)(v - (float)sh[e]);
+            sl[e] = (_Float16)((v - (float)sh[e]) * a.rls);
           }
           const half8 qhi = *reinterpret_cast<const half8*>(qs + 64 * kb);
           dq = mfma(qhi, sh, dq);
@@ -487,7 +491,7 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
         for (int i = 0; i < 4; ++i) {
           const int h = 4 * q4 + i;
           if (h < a.g && h < GC) {
-            const float v = (dq[i] + dl[i]) * (1.f / SQD);
+            const float v = fmaf(dl[i], lup, dq[i]) * (1.f / SQD);
             const _Float16 hi = (_Float16)v, lo = (_Float16)(v - (float)hi);
             uint8_t* d = tail + L_::sqo + h * 2 * SQS + 2 * p;
             *reinterpret_cast<_Float16*>(d) = hi;

@@ -37,11 +37,11 @@ class DeviceCodec:
             raise ValueError(f"Unsupported bit-width: {bits}. Use 1, 2, 3, or 4.")
         self.device = device
         self.rotation = get_rotation_matrix(d, seed, device)
-        # MFMA operands of the K4/V2 decode kernels' query rotation: fp16
-        # high part and remainder of R, as 16-bit words
+        # MFMA operands of the decode kernels' query rotation: fp16 high part
+        # and remainder of R, and 2048 times the remainder, as 16-bit words
         hi = self.rotation.half()
-        self.rotation_parts = torch.stack([
-            hi.view(torch.int16), (self.rotation - hi.float()).half().view(torch.int16)]).contiguous()
+        lo = self.rotation - hi.float()
+        self.rotation_parts = torch.stack([x.view(torch.int16) for x in (hi, lo.half(), (2048 * lo).half())]).contiguous()
         self.c_hi, self.b_hi = get_codebook(d, self.bits_hi, device)
         self.c_lo, self.b_lo = get_codebook(d, self.bits_lo, device)
         # the sketch's m projections, held as qjl_mp rows (zero rows past m)
@@ -58,7 +58,7 @@ class DeviceCodec:
             boundaries_hi=self.b_hi.data_ptr(), centroids_lo=self.c_lo.data_ptr(),
             boundaries_lo=self.b_lo.data_ptr(),
             qjl_proj=self.proj.data_ptr() if self.proj is not None else None,
-            qjl_m=self.qjl_mp, flags=0, rotation_parts=self.rotation_parts.data_ptr())
+            qjl_m=self.qjl_mp, flags=_lib.TQ_CODEC_ROTATION_LO2, rotation_parts=self.rotation_parts.data_ptr())
         # host-side tables: the codebook by value and, for 2-bit codebooks,
         # its exact fp16 copy (the K4/V2 decode kernels' value table)
         cen = self.c_hi.detach().cpu().numpy().astype("float32")

@@ -41,6 +41,7 @@ class Codec(ctypes.Structure):
                 ("value_table_err", ctypes.c_float), ("decode_table", _p)]
 
 TQ_CODEC_GENERAL_COMPRESS = 1
+TQ_CODEC_ROTATION_LO2 = 2
 
 
 class Store(ctypes.Structure):
