@@ -204,6 +204,11 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
   // query is converted; at D = 256 the registers do not hold both: each is
   // requested where it is used
   constexpr bool EARLY = D < 256;
+  // the remainders' score products in accumulators of their own: half as many
+  // roundings at the scores' magnitude (a sketch at D >= 128 has no registers
+  // for them). Error against float64, relative to the general kernel's, 0.62 ->
+  // 0.54 over 53 drawn cases; at most 0.1 us per layer
+  constexpr bool SL = !QJ || D < 128;
   extern __shared__ __align__(16) uint8_t smem[];
   uint8_t* tail = smem + a.tail;
 
@@ -651,7 +656,7 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
           gv[4 * t] = b4.x; gv[4 * t + 1] = b4.y; gv[4 * t + 2] = b4.z; gv[4 * t + 3] = b4.w;
         }
       }
-      f4 sc2[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+      f4 sc2[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}}, sl2[2] = {sc2[0], sc2[1]};
 #pragma unroll
       for (int s = 0; s < G_::KS; ++s) {
         const int seg = s / G_::SST, bits = G_::bits(seg), o = seg ? G_::ndw(0) : 0;
@@ -669,9 +674,11 @@ __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {
             lo[f] = e[1];
           }
           sc2[t] = mfma(as_h8(hi), qb[s], sc2[t]);
-          sc2[t] = mfma(as_h8(lo), qb[s], sc2[t]);
+          f4& sl = SL ? sl2[t] : sc2[t];
+          sl = mfma(as_h8(lo), qb[s], sl);
         }
       }
+      if constexpr (SL) sc2[0] += sl2[0], sc2[1] += sl2[1];
       float sc[NS];
       if constexpr (QJ) {
         // key term: + gamma_k sqrt(pi / 2) / D (S q) . z, before the mask

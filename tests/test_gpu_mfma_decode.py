@@ -409,3 +409,28 @@ def test_sketch_both_routes(G, T, route):
                    k, v, torch.float16)
     assert c._compressed_len == T
     _check(c, o, np.random.RandomState(G).randn(11, 8 * G, 1, 128).astype(np.float16), f"QJL G={G} T={T}", route)
+
+
+@pytest.mark.parametrize("D,m", [(64, 0), (256, 32)])
+def test_mfma_rotation_parts_of_two_planes(D, m):
+    """A key codec without the third plane's flag: the remainder of [1], the same bound."""
+    from turboquant_amd import _lib
+    k, v = _kv(1, 2, 1500, D, seed=D)
+    c, o = _caches(dict(head_dim=D, num_kv_heads=2, residual_window=64, fp16_sink_size=16,
+                        **(dict(qjl_correction=True, qjl_n_proj=m) if m else {})), k, v, torch.bfloat16)
+    q = np.random.RandomState(3).randn(1, 8, 1, D).astype(np.float16)
+    qd = to_dev(q)
+    three = c.attend(qd).cpu().numpy()
+    two = _lib.Codec.from_buffer_copy(c._kc.struct)
+    assert two.flags & _lib.TQ_CODEC_ROTATION_LO2
+    two.flags = 0
+    out = torch.empty(1, 8, 1, D, device="cuda")
+    d = c.attention_descriptor(qd, out, D ** -0.5)
+    lib = _lib.load()
+    need = lib.tq_attention_workspace_bytes(ctypes.byref(two), c._vc.ref(), ctypes.byref(d))
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    _lib.check(lib.tq_decode_attention(ctypes.byref(two), c._vc.ref(), ctypes.byref(d), ws.data_ptr(), need,
+                                       _lib.stream_ptr(out.device)), "tq_decode_attention")
+    got = out.cpu().numpy()
+    ref = O.attention(q, *dense_from_gpu_codes(c, o))
+    assert not np.array_equal(got, three) and rel_err(got, ref) < REL_TOL and rel_err(three, ref) < REL_TOL
