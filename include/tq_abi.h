@@ -78,7 +78,7 @@ typedef struct tq_codec {
    * value_table_err (relative). The K4/V2 route runs only when the key
    * codec has rotation_parts, 16 host_centroids and its decode_table, and the
    * value codec its decode_table with value_table_err <= 2e-7 (else the
-   * general kernels). */
+   * kernels of the other widths and head_dims, or the general kernels). */
   float host_centroids[16];
   int32_t n_host_centroids;
   uint16_t value_table[4];
@@ -93,7 +93,7 @@ typedef struct tq_codec {
 } tq_codec;
 
 /* tq_codec.flags: route tq_compress calls with this codec through the
- * general compress kernel instead of the MFMA kernel (no reference
+ * general compress kernel instead of the MFMA kernels (no reference
  * counterpart; lets tests compare the two kernels, per call). */
 #define TQ_CODEC_GENERAL_COMPRESS 1
 
@@ -236,7 +236,7 @@ typedef struct tq_attn_desc {
 } tq_attn_desc;
 
 /* tq_attn_desc.flags: force the general kernel (every width / QJL) even where
- * the K4/V2 partials + merge kernels apply. */
+ * one of the MFMA kernels applies. */
 #define TQ_ATTN_GENERAL 1
 
 /* Workspace: scratch for the per-workgroup partials of one call (no state is

@@ -19,7 +19,8 @@
 // in an LDS table whose 8-byte entry is (c_hi pair, c_lo pair) in fp16, c_lo =
 // c - fp16(c): four lookups fill the high-part and the remainder operand of a
 // k-step. The query's fp16 high part and remainder are two columns of B, so
-// two MFMAs per step give the product to 2^-22. For GC = 4 the 16 columns are
+// two MFMAs per step give the whole product but for the operands' own rounding
+// (see "Operands" below). For GC = 4 the 16 columns are
 // two groups of 8, group t serving 16-token tile t of the block (column c8
 // the high part of head c8, c8 < 4, or the remainder of head 7 - c8); for
 // GC = 8 column r is part r >> 3 of head r & 7. Columns past the group's
@@ -35,22 +36,32 @@
 // Tables have 16 replicas per entry (128-byte rows): both sides of every width
 // pair fit 80 KB, against 2-way bank conflicts on some lookups.
 //
-// Bound: latency and VALU issue, not memory (one layer's codes are 2-9 MB,
-// under 2 us of HBM time): launch, the set-up's two barriers, the first block's
-// round trip, about 1,000 VALU instructions per block and wave at four cycles
-// each (two waves per SIMD), the combine. So the set-up shares its work: a
-// thread converts 8 query elements for all waves, one branch per type around
-// each loop (a per-element branch on the query's type alone cost 1,000-2,400
-// instructions per wave: 2.6 us per layer at head_dim 128), bf16 tokens go to
-// bf16 MFMAs as they are against three bf16 parts of the query and the weights
-// (scaling them into fp16 took 500 instructions per block), and the
-// accumulators are not rescaled before the first block.
+// Operands in two fp16 parts (query, rotated query, R, S, S q, centroids,
+// weights) hold 22 to 24 bits where the general kernel's float32 holds 24, and
+// low x low products are left out where both sides are in parts. What the sums
+// round is more: sixteen MFMA steps here, D float32 steps there. Error against
+// float64 over 53 drawn cases (queries N(0, 2), keys of mixed scale) of 3 inputs
+// each: 0.54 of the general kernel's (geometric mean; root mean squares 7.0e-7
+// and 1.36e-6; 155 of the 159 below it).
+//
+// Bound: latency, not memory (one layer's codes are 2-9 MB, under 2 us of HBM
+// time) and not issue: launch, the set-up's two barriers, the first block's
+// round trip, a block's chain of lookups and MFMAs, the combine. Counted: 1,034
+// VALU, 150 LDS and 43 MFMA instructions per wave at the first shape below (one
+// block a wave), 931 / 103 / 35 at the second (two), 1,323 / 208 / 91 at the third
+// (one or none); at four cycles each and two waves per SIMD the VALU takes 3.4,
+// 3.1 and 4.4 us of the partials kernel's 12.1, 10.6 and 20.3. Both shrink
+// with the work each wave repeats, so the set-up shares it: a thread converts 8
+// query elements for all waves, one branch per type around each loop (a branch
+// per element took 2.6 us per layer at head_dim 128), bf16 tokens go to bf16
+// MFMAs as they are against three bf16 parts of the query and the weights, and
+// the accumulators are not rescaled before the first block.
 // Measured per layer in a graph of 16 layers, partials + merge against the
 // general kernel's three launches (float32 VALU dot products): bf16 K4/V4, 28
-// heads on 4, T 16,001: 15.6 us (kernels 11.2 + 4.6) from 101 us; head_dim 64,
-// bf16 K4/V2, 2 sequences, 32 heads on 8, T 8,229: 13.1 us (10.2 + 4.0) from 56
-// us; head_dim 256, bf16 K4/V3, 8 heads on 2, T 12,000: 26.4 us (20.2 + 6.3)
-// from 112 us (its rotation reads 256 KB of R per workgroup).
+// heads on 4, T 16,001: 15.6 us from 101 us (merge 4.1); head_dim 64, bf16
+// K4/V2, 2 sequences, 32 heads on 8, T 8,229: 13.0 us from 56 us (merge 3.7);
+// head_dim 256, bf16 K4/V3, 8 heads on 2, T 12,000: 26.3 us from 112 us (merge
+// 6.5; its rotation reads 256 KB of R per workgroup).
 #pragma once
 
 #include <math.h>
@@ -188,7 +199,7 @@ struct Blk {
 // per tile: one MFMA. Value term: u = sum_t p_t gamma_t z_t accumulates in two
 // more MFMAs (rows = projections) and travels with the partial; the merge
 // applies S^T. Per layer: head_dim 64 59.4 -> 16.8 us (13.0 without the sketch),
-// head_dim 256 106.7 -> 32.5, bf16 K4/V4 28 heads on 4 104 -> 20.9 (the cases
+// head_dim 256 106.7 -> 33.4, bf16 K4/V4 28 heads on 4 104 -> 20.9 (the cases
 // above, against the general kernel).
 template <int D, int GC, int KK, bool VF, bool QJ>
 __global__ __launch_bounds__(MTH) void mfma_decode_kernel(MfmaArgs a) {

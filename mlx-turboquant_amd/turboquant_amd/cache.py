@@ -103,7 +103,8 @@ class TurboQuantKVCache:
     @staticmethod
     def attend_head_dim(head_dim: int) -> bool:
         """head_dims the codecs and the attention kernels take: multiples of 16
-        in [16, 256] (the MFMA kernels at 128, the general kernels at all)."""
+        in [16, 256] (the MFMA kernels at 64, 96, 128 and 256, the general
+        kernels at all)."""
         return 16 <= head_dim <= 256 and head_dim % 16 == 0
 
     def __init__(self, head_dim: int = 128, num_kv_heads: int = 1, key_bits: float = 4,
@@ -387,7 +388,7 @@ class TurboQuantKVCache:
         "causal" prefill mask, cache.py:722-724). Returns float32
         (B, Hq, T_q, D): softmax(scale * q K^T) V over the same tokens
         update_and_fetch would return (default scale D**-0.5).
-        ``general_kernel`` forces the general kernel where the K4/V2 fast
+        ``general_kernel`` forces the general kernel where one of the MFMA
         kernels would run (used to cross-check the two)."""
         if self._B is None or self.offset == 0:
             raise ValueError("attend() on an empty cache")
